@@ -250,4 +250,62 @@ template <> struct dft<7> : dft_odd<7> {};
 template <> struct dft<11> : dft_odd<11> {};
 template <> struct dft<13> : dft_odd<13> {};
 
+// N = A B with coprime factors, without twiddles (Good's prime factor mapping): input B n1 + A n2,
+// output k with k = k1 mod A and k = k2 mod B.
+template <int A, int B> struct dft_coprime {
+    static constexpr int crt(int k1, int k2) {
+        for (int k = 0; k < A * B; k++)
+            if (k % A == k1 && k % B == k2) return k;
+        return 0;
+    }
+    template <typename C> __device__ __forceinline__ static void run(C *x) {
+        C y[B][A];
+#pragma unroll
+        for (int n2 = 0; n2 < B; n2++) {
+#pragma unroll
+            for (int n1 = 0; n1 < A; n1++) y[n2][n1] = x[(B * n1 + A * n2) % (A * B)];
+            dft<A>::run(y[n2]);
+        }
+#pragma unroll
+        for (int k1 = 0; k1 < A; k1++) {
+            C z[B];
+#pragma unroll
+            for (int n2 = 0; n2 < B; n2++) z[n2] = y[n2][k1];
+            dft<B>::run(z);
+#pragma unroll
+            for (int k2 = 0; k2 < B; k2++) x[crt(k1, k2)] = z[k2];
+        }
+    }
+};
+template <> struct dft<6> : dft_coprime<2, 3> {};
+template <> struct dft<10> : dft_coprime<2, 5> {};
+template <> struct dft<12> : dft_coprime<4, 3> {};
+template <> struct dft<14> : dft_coprime<2, 7> {};
+template <> struct dft<15> : dft_coprime<3, 5> {};
+
+// 9 = 3 x 3: DFT3 over h of x[p + 3h], twiddle by w9^{p m}, DFT3 over p.
+template <> struct dft<9> {
+    template <typename C> __device__ __forceinline__ static void run(C *x) {
+        using T = decltype(C::x);
+        C y[3][3];
+#pragma unroll
+        for (int p = 0; p < 3; p++) {
+#pragma unroll
+            for (int h = 0; h < 3; h++) y[p][h] = x[p + 3 * h];
+            dft<3>::run(y[p]);
+        }
+        y[1][1] = cmul(y[1][1], cmk<C>((T)0.76604444311897803520, (T)-0.64278760968653932632));
+        y[1][2] = cmul(y[1][2], cmk<C>((T)0.17364817766693034885, (T)-0.98480775301220805937));
+        y[2][1] = cmul(y[2][1], cmk<C>((T)0.17364817766693034885, (T)-0.98480775301220805937));
+        y[2][2] = cmul(y[2][2], cmk<C>((T)-0.93969262078590838405, (T)-0.34202014332566873304));
+#pragma unroll
+        for (int m = 0; m < 3; m++) {
+            C z[3] = {y[0][m], y[1][m], y[2][m]};
+            dft<3>::run(z);
+#pragma unroll
+            for (int q = 0; q < 3; q++) x[m + 3 * q] = z[q];
+        }
+    }
+};
+
 }  // namespace hmi

@@ -1,0 +1,236 @@
+// Radix plans, tile shapes and twiddle tables of the runtime-length pass (fft_generic).
+#include <algorithm>
+#include <cmath>
+#include <cstring>
+#include <limits>
+#include <stdexcept>
+
+#include "hmi_plan.h"
+
+namespace hmi {
+
+namespace {
+
+constexpr int kRadices[] = {16, 15, 14, 13, 12, 11, 10, 9, 8, 7, 6, 5, 4, 3, 2};
+
+// Real operations of the radix-r butterfly (additions and multiply-adds).
+double butterfly_ops(int r) {
+    switch (r) {
+        case 2: return 4;
+        case 3: return 16;
+        case 4: return 16;
+        case 5: return 40;
+        case 6: return 44;
+        case 7: return 72;
+        case 8: return 64;
+        case 9: return 120;
+        case 10: return 100;
+        case 11: return 150;
+        case 12: return 112;
+        case 13: return 210;
+        case 14: return 172;
+        case 15: return 200;
+        default: return 170;
+    }
+}
+
+// Cost per element of one stage: its butterfly and twiddles, and a fixed part for the LDS exchange
+// and the index work.
+double stage_cost(int r, bool dbl) {
+    // radices past the light build's cost resident waves
+    return 14.0 + (butterfly_ops(r) + 6.0 * (r - 1)) / r + (r > kLightRadix ? (dbl ? 4.0 : 2.0) : 0.0);
+}
+
+void search(int n, int top, bool dbl, std::vector<int> &cur, double cost, std::vector<int> &best, double &best_cost) {
+    if (cost >= best_cost) return;
+    if (n == 1) {
+        best = cur;
+        best_cost = cost;
+        return;
+    }
+    if ((int)cur.size() == kMixedStages) return;
+    for (int r : kRadices)
+        if (r <= top && n % r == 0) {
+            cur.push_back(r);
+            search(n / r, r, dbl, cur, cost + stage_cost(r, dbl), best, best_cost);
+            cur.pop_back();
+        }
+}
+
+fast_div make_div(unsigned d) {
+    unsigned s = 0;
+    while ((1ull << s) < d) s++;
+    const unsigned long long p = 1ull << (31 + s);
+    return {(unsigned)((p + d - 1) / d), s};
+}
+
+// LDS cycles of the last stage's reads when lanes walk the FFT axis: lane u reads position u's block,
+// k_0 m_0 pitch + k_0 pad + (rest); the LDS serves `group` lanes at once from
+// `group` element slots (32 of 8 bytes over its 64 banks, 16 of 16 bytes).
+int read_conflicts(const mixed_plan &g, int pad, int group) {
+    const int nb = g.n / g.last, lanes = std::min(nb, 4 * group);
+    int total = 0;
+    for (int u0 = 0; u0 < lanes; u0 += group) {
+        int used[32] = {}, worst = 0;
+        for (int u = u0; u < std::min(u0 + group, nb); u++) {
+            int t = u, pos = 0, k0 = 0, span = g.n;
+            for (int s = 0; s + 1 < g.nst; s++) {
+                span /= g.radix[s];
+                const int d = t % g.radix[s];
+                t /= g.radix[s];
+                if (s == 0) k0 = d;
+                pos += d * span;
+            }
+            worst = std::max(worst, ++used[(pos * g.pitch + k0 * pad) % group]);
+        }
+        total += worst;
+    }
+    return total;
+}
+
+}  // namespace
+
+std::vector<int> mixed_radices(int n, bool dbl) {
+    std::vector<int> cur, best;
+    double cost = std::numeric_limits<double>::infinity();
+    search(n, 16, dbl, cur, 0.0, best, cost);
+    if (best.size() > 2) {
+        // the largest radix first and the next one last: the stages on global memory keep the most
+        // accesses in flight
+        std::rotate(best.begin() + 1, best.begin() + 2, best.end());
+    }
+    return best;
+}
+
+mixed_config make_mixed(int n, bool dbl, bool copy, bool load_across, bool store_across, long long ncol,
+                        long long nlines) {
+    mixed_config c{};
+    mixed_plan &g = c.plan;
+    const std::vector<int> rad = (copy || n == 1) ? std::vector<int>{} : mixed_radices(n, dbl);
+    c.ok = copy || n == 1 || !rad.empty();
+    if (!c.ok) return c;
+    const long long elem = dbl ? 16 : 8;
+    g.n = n;
+    g.nst = (int)rad.size();
+    for (int s = 0; s < kMixedStages; s++) {
+        g.radix[s] = s < g.nst ? rad[s] : 1;
+        g.by_r[s] = make_div(g.radix[s]);
+        if (s == 0) g.m0 = n / g.radix[0];
+
+    }
+    g.last = g.nst ? rad.back() : 1;
+    g.by_m0 = make_div(g.m0);
+    g.by_last = make_div(n / g.last);
+    g.by_n = make_div(n);
+    g.postoff = mixed_post_offset(rad);
+    // Lines per tile: about kMixedTile bytes, and in any case the 128-byte column chunk where a side
+    // walks the column axis or where that keeps two blocks per CU.
+    const bool across = load_across || store_across;
+    const bool walk = !load_across || !store_across;  // a side on which lanes walk the FFT axis
+    auto bytes = [&](int t) {
+        const long long pitch = walk && t > 1 ? t + 1 : t;
+        return ((long long)n * pitch + 32LL * g.radix[0]) * elem;
+    };
+    int l2 = 0;
+    while (l2 < 6 && (n * elem << (l2 + 1)) <= kMixedTile) l2++;
+    while ((elem << l2) < 128 && bytes(2 << l2) <= (across ? kGenericMaxLds : kGenericMaxLds / 2)) l2++;
+    const long long cap = across ? ncol : nlines;
+    while (l2 > 0 && (1LL << (l2 - 1)) >= cap) l2--;
+    g.log2t = l2;
+    const int T = 1 << l2;
+    g.pitch = walk && T > 1 ? T + 1 : T;
+    g.pad = 0;
+    if (g.nst > 1 && !store_across) {
+        int best = std::numeric_limits<int>::max();
+        for (int pad = 0; pad < (dbl ? 16 : 32); pad++) {
+            const int k = read_conflicts(g, pad, dbl ? 16 : 32);
+            if (k < best && ((long long)n * g.pitch + (long long)(g.radix[0] - 1) * pad) * elem <= kGenericMaxLds) {
+                best = k;
+                g.pad = pad;
+            }
+        }
+    }
+    c.lds = (size_t)(((long long)n * g.pitch + (long long)(g.radix[0] - 1) * g.pad) * elem);
+    // Threads: the rounds a block spends in each stage (the ones on global memory weigh more) over
+    // the blocks a CU holds, and the idle lanes of the last rounds.  Blocks of more than four waves
+    // count as whole sets of four, one for each SIMD: 320 points complex<double>, 8 lines, contiguous:
+    // 256 threads 5.36 TB/s, 320 4.54, 512 5.22; 400 points: 256 4.62, 320 4.73, 512 5.25.
+    const bool light = rad.empty() || *std::max_element(rad.begin(), rad.end()) <= kLightRadix;
+    const int by_lds = (int)(kGenericMaxLds / std::max<long long>(1, (long long)c.lds));
+    const int waves = 4 * (dbl ? (light ? 4 : 3) : (light ? 8 : 5));
+    double best = std::numeric_limits<double>::infinity();
+    for (int th = 64; th <= kMixedThreads; th += 64) {
+        if (th % T) continue;
+        const int held = th <= 256 ? th : (th + 255) / 256 * 256;
+        double rounds = 0.0, lanes = 0.0, ideal = 0.0;
+        const int stages = std::max(1, g.nst);
+        for (int s = 0; s < stages; s++) {
+            const long long units = (long long)T * n / (g.nst ? rad[s] : 1);
+            const double w = (g.nst ? rad[s] : 1) * stage_cost(g.nst ? rad[s] : 1, dbl);
+            const double k = (double)((units + th - 1) / th);
+            rounds += k * (s == 0 ? 3.0 : s + 1 == stages ? 2.0 : 1.0);
+            lanes += w * k * held;
+            ideal += w * (double)units;
+        }
+        const int resident = std::max(1, std::min({by_lds, waves * 64 / held, 16}));
+        const double cost = rounds / resident * (0.5 + 0.5 * lanes / ideal);
+        if (cost < best - 1e-9) {
+            best = cost;
+            c.threads = th;
+        }
+    }
+    return c;
+}
+
+void mixed_launch_divs(mixed_plan &g, const pass_args &a) {
+    g.by_ncol = make_div((unsigned)a.ncol);
+    g.by_nb1 = make_div((unsigned)a.nb1);
+}
+
+int mixed_post_offset(const std::vector<int> &rad) {
+    int off = 0;
+    long long m = 1;
+    for (int r : rad) m *= r;
+    for (size_t s = 0; s + 1 < rad.size(); s++) {
+        m /= rad[s];
+        off += (int)m * (rad[s] - 1);
+    }
+    return off;
+}
+
+std::vector<unsigned char> mixed_table(int n, bool dbl, bool copy, int tail_count, long long tail_mod) {
+    const std::vector<int> rad = (copy || n == 1) ? std::vector<int>{} : mixed_radices(n, dbl);
+    std::vector<unsigned char> out(kMixedHead, 0);
+    auto push = [&](long long e, long long mod) {
+        const long double pi = 3.141592653589793238462643383279502884L;
+        const long double ang = 2.0L * pi * (long double)(e % mod) / (long double)mod;
+        const size_t at = out.size();
+        if (dbl) {
+            const double v[2] = {(double)cosl(ang), (double)(-sinl(ang))};
+            out.resize(at + sizeof(v));
+            std::memcpy(&out[at], v, sizeof(v));
+        } else {
+            const float v[2] = {(float)cosl(ang), (float)(-sinl(ang))};
+            out.resize(at + sizeof(v));
+            std::memcpy(&out[at], v, sizeof(v));
+        }
+    };
+    long long len = n, off = 0, blocks = 1;
+    for (size_t s = 0; s + 1 < rad.size(); s++) {
+        const int r = rad[s];
+        const long long m = len / r;
+        if (s > 0) {
+            const mixed_stage st{r, (int)m, (int)off, make_div((unsigned)m), make_div((unsigned)blocks)};
+            std::memcpy(&out[(s - 1) * sizeof(mixed_stage)], &st, sizeof(st));
+            blocks *= r;
+        }
+        for (long long j = 0; j < m; j++)
+            for (int q = 1; q < r; q++) push(j * q, len);
+        off += m * (r - 1);
+        len = m;
+    }
+    for (int k = 0; k < tail_count; k++) push(k, tail_mod);
+    return out;
+}
+
+}  // namespace hmi

@@ -33,6 +33,20 @@ const fast_kernel_info *find_fast_kernel(int n, bool dbl, bool wide);
 hipError_t launch_generic(bool dbl, const pass_args &a, const generic_plan &g, long long nblocks, size_t lds_bytes,
                           hipStream_t s);
 
+// Runtime-length pass (hmi_generic.h): at most kMixedThreads threads per block; plans whose radices
+// all stay within kLightRadix run a build of their own with fewer registers.
+constexpr int kMixedThreads = 512;
+constexpr int kLightRadix = 10;
+constexpr long long kMixedTile = 16 * 1024;  // bytes a tile aims at
+hipError_t launch_mixed_f32(const pass_args &a, const mixed_plan &g, int threads, long long nblocks, size_t lds_bytes,
+                            hipStream_t s);
+hipError_t launch_mixed_f64(const pass_args &a, const mixed_plan &g, int threads, long long nblocks, size_t lds_bytes,
+                            hipStream_t s);
+inline hipError_t launch_mixed(bool dbl, const pass_args &a, const mixed_plan &g, int threads, long long nblocks,
+                               size_t lds_bytes, hipStream_t s) {
+    return (dbl ? launch_mixed_f64 : launch_mixed_f32)(a, g, threads, nblocks, lds_bytes, s);
+}
+
 // Compile-time tile of the batched kernel for one length: lines per tile and LDS bytes
 // for each precision, and the complex-unit size of its stage twiddle table.
 struct batch_kernel_info {

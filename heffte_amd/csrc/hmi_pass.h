@@ -78,6 +78,42 @@ struct generic_plan {
     int postoff;               // offset of the real-data twiddles (modes other than kModeC2C)
 };
 
+// Division of x < 2^31 by a fixed divisor d: q = umulhi(2 x, mul) >> shift, with 2^(shift-1) < d <=
+// 2^shift and mul = ceil(2^(31 + shift) / d); exact, since x (mul d - 2^(31 + shift)) < 2^(31 + shift).
+struct fast_div {
+    unsigned mul, shift;
+};
+
+// Radix plan of the runtime-length pass (fft_generic): an in-place decimation in frequency over one
+// LDS tile.  n = r_0 r_1 ... r_{S-1}; after stage s the remaining sub-transforms have m_s =
+// n / (r_0 ... r_s) points.  Stage s runs the butterflies of the elements base + j + p m_s
+// (p < r_s, j < m_s) of each of the n / (r_s m_s) blocks, twiddles output q by w_{r_s m_s}^{j q} and
+// leaves it at base + j + q m_s; frequency k_0 + r_0 k_1 + r_0 r_1 k_2 + ... ends at position
+// k_0 m_0 + k_1 m_1 + ...  Element (line l, position i) of a tile sits at
+// i pitch + (i / m_0) pad + l.
+enum : int { kMixedStages = 6 };
+struct mixed_plan {
+    int n, nst;
+    int log2t, pitch, pad;           // lines per tile 2^log2t, LDS strides (elements)
+    int radix[kMixedStages];
+    int m0;                          // the first stage's twiddles w_n^{j q}: table[j (r_0 - 1) + q - 1]
+    int last;                        // r_{S-1}
+    int postoff;                     // real-data twiddles (modes other than kModeC2C)
+    fast_div by_r[kMixedStages];     // / r_s
+    fast_div by_m0, by_last;         // / m_0, / (n / r_{S-1})
+    fast_div by_n, by_ncol, by_nb1;  // line and element numbering
+};
+
+// Stages 1 to S - 2 of the plan, at the start of its device table (kMixedHead bytes; the twiddles
+// follow): the kernel walks them with a run-time index, which a kernel argument would not allow
+// without a copy to scratch memory.
+struct mixed_stage {
+    int radix, m, twoff;
+    fast_div by_m, by_k0;            // / m_s, / (r_1 ... r_{s-1}): block number -> k_0
+};
+enum : int { kMixedHead = 128 };
+static_assert(sizeof(mixed_stage) * (kMixedStages - 2) <= kMixedHead, "the middle stages fit the table head");
+
 // Batched mixed-size transforms (one phase = one axis of every transform).
 // Every transform is a c2c box in order (0, 1, 2) at its own element offset.
 struct batch_xform {

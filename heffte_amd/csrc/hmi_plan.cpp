@@ -128,7 +128,7 @@ fft_plan::fft_plan(kind k, const box3 &inbox, const box3 &outbox, int r2c_dir)
     long long ws = 0;
     // (a length may be split in one precision only: lines of complex<double> fill LDS sooner)
     for (bool dbl : {false, true})
-        for_each_variant([&](int dir, bool ir, bool orl, bool ip) { ws = std::max(ws, build(dir, dbl, ir, orl, ip).ws_elems); });
+        for_each_variant([&](int dir, bool ir, bool orl, bool ip) { ws = std::max(ws, build(dir, dbl, ir, orl, ip, true).ws_elems); });
     ws_elems_ = ws;
 }
 
@@ -197,7 +197,7 @@ const exec_plan &fft_plan::get_exec_plan(int dir, bool dbl, bool in_real, bool o
     return it->second;
 }
 
-exec_plan fft_plan::build(int dir, bool dbl, bool in_real, bool out_real, bool in_place) const {
+exec_plan fft_plan::build(int dir, bool dbl, bool in_real, bool out_real, bool in_place, bool sizes_only) const {
     const bool fwd = dir < 0;
     const box3 &bin = fwd ? inbox_ : outbox_;
     const box3 &bout = fwd ? outbox_ : inbox_;
@@ -325,6 +325,8 @@ exec_plan fft_plan::build(int dir, bool dbl, bool in_real, bool out_real, bool i
                     if (!cp.identity && (p.load_colfast || p.store_colfast)) cost += narrow_chunk_cost(p, dbl);
                     // a copy pass runs one LDS tile per line: not along an axis too long for one
                     if (cp.identity) cost += 0.5 + (2 * dims[cp.axis] * (dbl ? 16 : 8) > kGenericMaxLds ? 100.0 : 0.0);
+                    // costs only grow along the sequence: not cheaper than the best one so far
+                    if (cost >= best_cost) { ok = false; break; }
                     ep.passes.push_back(p);
                     cur = p.lout;
                     cur_buf = p.dst;
@@ -361,7 +363,7 @@ exec_plan fft_plan::build(int dir, bool dbl, bool in_real, bool out_real, bool i
     } while (std::next_permutation(perm.begin(), perm.end()));
     if (!std::isfinite(best_cost)) throw std::runtime_error("no valid pass schedule for these boxes");
 
-    for (pass &p : best.passes) configure(p, dbl);
+    for (pass &p : best.passes) configure(p, dbl, sizes_only);
     // the step buffer of split axes follows the intermediate arrays in the workspace
     long long split_elems = 0;
     for (pass &p : best.passes)
@@ -373,7 +375,7 @@ exec_plan fft_plan::build(int dir, bool dbl, bool in_real, bool out_real, bool i
     return best;
 }
 
-void fft_plan::configure(pass &p, bool dbl) const {
+void fft_plan::configure(pass &p, bool dbl, bool sizes_only) const {
     const size_t elem = dbl ? 16 : 8;
     const bool wide = p.load_colfast || p.store_colfast;
     if (p.mode >= kModeDCT2) {
@@ -400,8 +402,20 @@ void fft_plan::configure(pass &p, bool dbl) const {
         p.lines = p.fast->T;
         return;
     }
-    generic_plan &g = p.gen;
-    g = generic_plan{};
+    const size_t per_line = 2 * (size_t)p.n * elem;
+    if (per_line <= (size_t)kGenericMaxLds) {
+        if (sizes_only) return;  // no step buffer: nothing else the workspace depends on
+        const long long ncol = std::max(p.lin.n[p.col], p.lout.n[p.col]);
+        const mixed_config c = make_mixed(p.n, dbl, p.identity, p.load_colfast, p.store_colfast, ncol,
+                                          ncol * std::max(p.lin.n[p.b1], p.lout.n[p.b1]));
+        if (c.ok) {
+            p.mixed = std::make_shared<mixed_config>(c);
+            p.lines = 1 << c.plan.log2t;
+            return;
+        }
+    }
+    p.gen = std::make_shared<generic_plan>();
+    generic_plan &g = *p.gen;
     g.n = p.n;
     std::vector<int> rad = p.identity ? std::vector<int>{} : factorize(p.n);
     if ((int)rad.size() > kMaxStages) throw std::runtime_error("too many radix stages");
@@ -418,7 +432,6 @@ void fft_plan::configure(pass &p, bool dbl) const {
         if (!has_butterfly(rad[s])) off += rad[s];
     }
     g.postoff = off;
-    const size_t per_line = 2 * (size_t)p.n * elem;
     if (per_line > (size_t)kGenericMaxLds) {
         // beyond one LDS tile: two passes of lengths n1 * n2 = n (plain c2c lines only)
         int n1 = 0, n2 = 0;
@@ -436,6 +449,7 @@ void fft_plan::configure(pass &p, bool dbl) const {
             const long long big = 1LL << 20;  // many columns: no cap on the lines per block
             q.lin = q.lout = layout{{big, big, big}, {1, big, big * big}};
             q.col = 0;
+            q.b1 = 1;
             configure(q, dbl);
         }
         p.split_n1 = n1;
@@ -585,20 +599,24 @@ std::string pass_kernel_name(const pass &p, bool dbl, bool mfma, int precision, 
 const twiddles &fft_plan::get_twiddles(bool dbl, const pass &p, bool may_alloc) {
     const int n = p.n;
     const long long key = ((long long)n << 8) | (dbl ? 1 : 0) | (p.fast ? 2 : 0) | (p.identity ? 4 : 0) |
-                          ((long long)p.mode << 3) | (p.fast ? (long long)p.fast->T << 40 : 0);
+                          ((long long)p.mode << 3) | (p.fast ? (long long)p.fast->T << 40 : 0) | (p.mixed ? 1LL << 56 : 0);
     std::lock_guard<std::mutex> lock(mtx_);
     auto it = tw_.find(key);
     if (it != tw_.end()) return it->second;
     if (!may_alloc) throw std::runtime_error(kNotResident);
-    const int *radix = p.fast ? p.fast->radix : p.gen.radix;
-    const int ns = p.fast ? p.fast->nstages : p.gen.nstages;
+    const int *radix = p.fast ? p.fast->radix : (p.gen ? p.gen->radix : nullptr);
+    const int ns = p.fast ? p.fast->nstages : (p.gen ? p.gen->nstages : 0);
     twiddles t;
     // r2c / c2r: w_n^k for k < n/2 (n = real line length); r2r: w_{4n}^k for k < n
     int tail_count = 0;
     long long tail_mod = 1;
     if (p.mode == kModeR2C || p.mode == kModeC2R) { tail_count = n / 2; tail_mod = n; }
     if (p.mode >= kModeDCT2 && p.mode <= kModeDST3) { tail_count = n; tail_mod = 4LL * n; }
-    if (dbl) {
+    if (p.mixed) {
+        const std::vector<unsigned char> v = mixed_table(n, dbl, p.identity, tail_count, tail_mod);
+        t.bytes = v.size();
+        t.dev = upload_bytes(v.data(), t.bytes);
+    } else if (dbl) {
         std::vector<double> v = make_table<double>(radix, ns, !p.fast, tail_count, tail_mod);
         t.bytes = v.size() * sizeof(double);
         t.dev = upload_bytes(v.data(), t.bytes);
@@ -773,6 +791,14 @@ void split_steps(const pass &p, const pass_args &base, bool dbl, int bt, void *t
     }
 }
 
+namespace {
+void launch_mixed_pass(const pass &p, const pass_args &a, bool dbl, long long nblocks, hipStream_t s) {
+    mixed_plan g = p.mixed->plan;
+    mixed_launch_divs(g, a);
+    check_hip(launch_mixed(dbl, a, g, p.mixed->threads, nblocks, p.mixed->lds, s), "runtime-length FFT pass");
+}
+}  // namespace
+
 void fft_plan::launch_split(const pass &p, const pass_args &base, bool dbl, int batch, void *tmp) {
     const size_t elem = dbl ? 16 : 8;
     for (int bt = 0; bt < batch; bt++) {
@@ -784,7 +810,8 @@ void fft_plan::launch_split(const pass &p, const pass_args &base, bool dbl, int 
             st[i].tw = get_twiddles(dbl, q, false).dev;
             const long long nblocks = ((long long)st[i].nlines + q.lines - 1) / q.lines;
             if (q.fast) check_hip(q.fast->launch(st[i], nblocks, stream_), "split FFT pass");
-            else check_hip(launch_generic(dbl, st[i], q.gen, nblocks, 2 * (size_t)q.gen.lines * q.n * elem, stream_),
+            else if (q.mixed) launch_mixed_pass(q, st[i], dbl, nblocks, stream_);
+            else check_hip(launch_generic(dbl, st[i], *q.gen, nblocks, 2 * (size_t)q.gen->lines * q.n * elem, stream_),
                            "split FFT pass");
         }
     }
@@ -885,9 +912,11 @@ void fft_plan::execute(int dir, bool dbl, bool in_real, bool out_real, int batch
             check_hip(launch_mfma512(precision_, a, ((long long)a.nlines + 15) / 16, stream_), "MFMA FFT pass");
         } else if (p.fast) {
             check_hip(p.fast->launch(a, nblocks, stream_), "fast FFT pass");
+        } else if (p.mixed) {
+            launch_mixed_pass(p, a, dbl, nblocks, stream_);
         } else {
-            const size_t lds = 2 * (size_t)p.gen.lines * p.n * (dbl ? 16 : 8);
-            check_hip(launch_generic(dbl, a, p.gen, nblocks, lds, stream_), "generic FFT pass");
+            const size_t lds = 2 * (size_t)p.gen->lines * p.n * (dbl ? 16 : 8);
+            check_hip(launch_generic(dbl, a, *p.gen, nblocks, lds, stream_), "generic FFT pass");
         }
         if (tprev) {
             const std::string name = pass_kernel_name(p, dbl, mfma, precision_, a);

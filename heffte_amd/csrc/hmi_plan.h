@@ -48,6 +48,14 @@ struct layout {
     int fastest() const;  // axis with the smallest stride among axes with n > 1 (-1 if none)
 };
 
+// Radix plan, tile and block of the runtime-length pass for one pass of length n.
+struct mixed_config {
+    bool ok = false;   // false: n has a prime factor without a butterfly
+    mixed_plan plan{};
+    int threads = 64;
+    size_t lds = 0;
+};
+
 struct pass {
     int axis = 0, n = 1;
     buf src = buf::in, dst = buf::out;
@@ -61,7 +69,8 @@ struct pass {
     int mode = 0;           // kModeC2C, or kModeR2C / kModeC2R when the half-length kernel runs it
     // launch configuration
     const fast_kernel_info *fast = nullptr;
-    generic_plan gen{};
+    std::shared_ptr<generic_plan> gen;          // set: lengths with a prime factor above 13
+    std::shared_ptr<const mixed_config> mixed;  // set: the runtime-length pass runs it
     int lines = 1;  // lines (columns) per block
     // A length whose line does not fit one LDS tile runs as two passes (four-step), n = n1 n2,
     // position j = n2 j1 + j2, bin k = k1 + n1 k2: the first step takes the n1-point lines of
@@ -141,8 +150,9 @@ class fft_plan {
     std::string timing_report();
 
   private:
-    exec_plan build(int dir, bool dbl, bool in_real, bool out_real, bool in_place) const;
-    void configure(pass &p, bool dbl) const;
+    // sizes_only: enough of the plan for its workspace (the constructor asks for every variant's)
+    exec_plan build(int dir, bool dbl, bool in_real, bool out_real, bool in_place, bool sizes_only = false) const;
+    void configure(pass &p, bool dbl, bool sizes_only = false) const;
     const twiddles &get_twiddles(bool dbl, const pass &p, bool may_alloc);
     const twiddles &get_split_table(bool dbl, int n, bool may_alloc);
     void launch_split(const pass &p, const pass_args &base, bool dbl, int batch, void *tmp);
@@ -166,6 +176,18 @@ class fft_plan {
     std::vector<hipEvent_t> timing_events_;
     void clear_timing();
 };
+
+// Radix order of the runtime-length pass (empty: n has a prime factor above 13), its tile for one
+// pass (copy: no transform, only the layout change; *_across: that side walks the column axis; ncol
+// columns, nlines lines in all), and its device table: the middle stages' entries, the stage
+// twiddles, then w_{tail_mod}^k for k < tail_count (at mixed_post_offset).
+std::vector<int> mixed_radices(int n, bool dbl);
+mixed_config make_mixed(int n, bool dbl, bool copy, bool load_across, bool store_across, long long ncol,
+                        long long nlines);
+int mixed_post_offset(const std::vector<int> &radices);
+std::vector<unsigned char> mixed_table(int n, bool dbl, bool copy, int tail_count, long long tail_mod);
+// the divisors of one launch's line numbering
+void mixed_launch_divs(mixed_plan &g, const pass_args &a);
 
 // Runtime radix plan of length n for the generic tile (stage/root/post offsets
 // filled in; lines = lines per tile) and its twiddle table in either precision.

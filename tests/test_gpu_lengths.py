@@ -1,0 +1,63 @@
+"""GPU parity of the runtime-length pass over the lengths whose plans differ: one to five stages, every
+radix, odd and even, up to the longest lines of one LDS tile, with the axis contiguous or across
+columns on either side."""
+import numpy as np
+import pytest
+
+import fftcase as fc
+
+pytestmark = pytest.mark.gpu
+
+LENGTHS = [2, 3, 7, 10, 11, 13, 14, 15, 18, 22, 25, 26, 36, 49, 50, 60, 72, 81, 90, 91, 100, 121, 125, 143, 150, 169, 180,
+           225, 240, 250, 320, 343, 384, 400, 625, 768, 1000, 1331, 2187, 2400, 3125, 5000]
+
+
+@pytest.mark.parametrize("dtype", ["complex64", "complex128"])
+@pytest.mark.parametrize("n", LENGTHS)
+def test_c2c_lengths(hmi, cuda, oracle, dtype, n):
+    import torch
+    # lines of n points walked along the axis and across columns, odd column counts (partial tiles)
+    for size, inorder, outorder in [((n, 19, 3), (0, 1, 2), (1, 2, 0)), ((7, n, 5), (0, 1, 2), (0, 1, 2)),
+                                    ((3, 37, n), (2, 0, 1), (2, 0, 1))]:
+        inbox = hmi.box3d([0, 0, 0], [s - 1 for s in size], inorder)
+        outbox = hmi.box3d([0, 0, 0], [s - 1 for s in size], outorder)
+        plan = hmi.fft3d(hmi.backend.mi355, inbox, outbox)
+        x = fc.uniform_complex(2 * int(np.prod(size)), n)
+        tx = fc.to_gpu(x, np.complex64 if dtype == "complex64" else np.complex128)
+        ty, tz = torch.empty_like(tx), torch.empty_like(tx)
+        plan.forward(tx, ty, hmi.scale.none, 2)
+        plan.backward(ty, tz, hmi.scale.full, 2)
+        bi = oracle.Box.make((0, 0, 0), [s - 1 for s in size], inorder)
+        bo = oracle.Box.make((0, 0, 0), [s - 1 for s in size], outorder)
+        ref = oracle.fft3d_c2c(bi, bo, x, -1, 1.0, 2)
+        assert fc.rel_l2(fc.to_host(ty), ref) <= fc.TOL[dtype], (size, inorder, outorder)
+        assert fc.rel_l2(fc.to_host(tz), x) <= fc.TOL[dtype], (size, inorder, outorder)
+
+
+@pytest.mark.parametrize("dtype", ["float32", "float64"])
+@pytest.mark.parametrize("n", [2, 6, 15, 25, 36, 50, 60, 99, 100, 147, 180, 225, 250, 300, 390, 720, 1000])
+def test_r2c_and_r2r_lengths(hmi, cuda, oracle, dtype, n):
+    import torch
+    rdt = np.float32 if dtype == "float32" else np.float64
+    rng = np.random.default_rng(n)
+    for size, order, axis in [((n, 18, 3), (0, 1, 2), 0), ((5, n, 7), (0, 1, 2), 1), ((9, 5, n), (1, 2, 0), 2)]:
+        inbox = hmi.box3d([0, 0, 0], [s - 1 for s in size], order)
+        plan = hmi.fft3d_r2c(hmi.backend.mi355, inbox, inbox.r2c(axis), axis)
+        x = rng.standard_normal(inbox.count())
+        tx = torch.from_numpy(x.astype(rdt)).to(cuda)
+        ty = torch.empty(plan.size_outbox(), dtype=torch.complex64 if rdt == np.float32 else torch.complex128, device=cuda)
+        tz = torch.empty_like(tx)
+        plan.forward(tx, ty)
+        plan.backward(ty, tz, hmi.scale.full)
+        b = oracle.Box.make((0, 0, 0), [s - 1 for s in size], order)
+        half = inbox.r2c(axis)
+        ref = oracle.fft3d_r2c(b, oracle.Box.make(half.low, half.high, order), axis, x)
+        assert fc.rel_l2(fc.to_host(ty), ref) <= fc.TOL[dtype], (size, order)
+        assert fc.rel_l2(fc.to_host(tz), x) <= fc.TOL[dtype], (size, order)
+        for kind, fn in [("cos", oracle.r2r_cos), ("sin", oracle.r2r_sin)]:
+            rplan = hmi.rtransform(hmi.backend.mi355, inbox, inbox, getattr(hmi.kind, kind))
+            tr = torch.empty_like(tx)
+            rplan.forward(tx, tr)
+            assert fc.rel_l2(fc.to_host(tr), fn(b, b, x, -1)) <= fc.TOL[dtype], (kind, size)
+            rplan.backward(tr, tz, hmi.scale.full)
+            assert fc.rel_l2(fc.to_host(tz), x) <= fc.TOL[dtype], (kind, size)

@@ -64,20 +64,21 @@ template <typename C> __device__ __forceinline__ const C *mixed_twiddles(const p
 
 // Forms of the pass: every mode and overload; plain complex lines (no product, real side, partial
 // store or split twiddle); the same where both arrays lie within 4 GiB (each access is a uniform
-// base plus one 32-bit offset per thread, half the address registers).
-enum : int { kFormAny = 0, kFormPlain = 1, kFormPlain32 = 2 };
+// base plus one 32-bit offset per thread, half the address registers); chirp convolutions and plans with direct
+// stages (any mode).
+enum : int { kFormAny = 0, kFormPlain = 1, kFormPlain32 = 2, kFormChirp = 3, kFormDirect = 4 };
 
-// Elements j0, j0 + step, ... (RX of them) of a line in the pass's input form.
+// Elements j0, j0 + step, ... (RX of them; j0 < step) of a line in the pass's input form.
 template <int RX, int FORM, int NTM, typename R, typename C>
 __device__ __forceinline__ void mixed_load(C (&x)[RX], const pass_args &a, const mixed_plan &g, const line_at &ln, int j0,
                                            int step) {
     constexpr bool NTL = (NTM & 2) != 0;
     const R sg = a.conj ? R(-1) : R(1);
-    const int n = g.n;
+    const int n = g.len;
     if (!ln.valid) {
 #pragma unroll
         for (int p = 0; p < RX; p++) x[p] = cmk<C>(R(0), R(0));
-    } else if (FORM == kFormAny && (a.mode == kModeDCT2 || a.mode == kModeDST2)) {
+    } else if ((FORM == kFormAny || FORM == kFormDirect) && (a.mode == kModeDCT2 || a.mode == kModeDST2)) {
         const R *__restrict__ src = static_cast<const R *>(a.in) + ln.base;
 #pragma unroll
         for (int p = 0; p < RX; p++) {
@@ -86,7 +87,7 @@ __device__ __forceinline__ void mixed_load(C (&x)[RX], const pass_args &a, const
             const R v = ldg<NTL>(&src[(long long)jj * a.in_sa]);
             x[p] = cmk<C>((a.mode == kModeDST2 && (jj & 1)) ? -v : v, R(0));
         }
-    } else if (FORM == kFormAny && (a.mode == kModeDCT3 || a.mode == kModeDST3)) {
+    } else if ((FORM == kFormAny || FORM == kFormDirect) && (a.mode == kModeDCT3 || a.mode == kModeDST3)) {
         const bool sine = (a.mode == kModeDST3);
         const R *__restrict__ src = static_cast<const R *>(a.in) + ln.base;
         const C *__restrict__ post = mixed_twiddles<C>(a) + g.postoff;
@@ -98,18 +99,18 @@ __device__ __forceinline__ void mixed_load(C (&x)[RX], const pass_args &a, const
             const C w = post[j];
             x[p] = cmk<C>(w.x * xk - w.y * xm, w.x * xm + w.y * xk);  // conj of conj(w) (xk - i xm)
         }
-    } else if (FORM == kFormAny && (a.mode == kModeDCT1 || a.mode == kModeDCT1B)) {
+    } else if ((FORM == kFormAny || FORM == kFormDirect) && (a.mode == kModeDCT1 || a.mode == kModeDCT1B)) {
         const R *__restrict__ src = static_cast<const R *>(a.in) + ln.base;
 #pragma unroll
         for (int p = 0; p < RX; p++) {
             const int j = j0 + p * step;
             x[p] = cmk<C>(ldg<NTL>(&src[(long long)(j <= n / 2 ? j : n - j) * a.in_sa]), R(0));
         }
-    } else if (FORM == kFormAny && a.in_real) {
+    } else if ((FORM == kFormAny || FORM == kFormDirect) && a.in_real) {
         const R *__restrict__ src = static_cast<const R *>(a.in) + ln.base;
 #pragma unroll
         for (int p = 0; p < RX; p++) x[p] = cmk<C>(ldg<NTL>(&src[(long long)(j0 + p * step) * a.in_sa]), R(0));
-    } else if (FORM == kFormAny && a.herm_load) {
+    } else if ((FORM == kFormAny || FORM == kFormDirect) && a.herm_load) {
         const C *__restrict__ src = static_cast<const C *>(a.in) + ln.base;
 #pragma unroll
         for (int p = 0; p < RX; p++) {
@@ -118,7 +119,7 @@ __device__ __forceinline__ void mixed_load(C (&x)[RX], const pass_args &a, const
             const C v = ldg<NTL>(&src[(long long)(mirror ? n - j : j) * a.in_sa]);
             x[p] = cmk<C>(v.x, (mirror ? -sg : sg) * v.y);
         }
-    } else if (FORM == kFormAny && a.mul) {
+    } else if ((FORM == kFormAny || FORM == kFormDirect) && a.mul) {
         const C *src = static_cast<const C *>(a.in) + ln.base;
         const C *mul = static_cast<const C *>(a.mul) + ln.base;
         C y[RX];
@@ -156,8 +157,8 @@ __device__ __forceinline__ void mixed_store(const C (&x)[RX], const pass_args &a
     constexpr bool NTS = (NTM & 1) != 0;
     const R sg = a.conj ? R(-1) : R(1);
     const R sc = (R)a.scale;
-    const int n = g.n;
-    if (FORM == kFormAny && (a.mode == kModeDCT2 || a.mode == kModeDST2)) {
+    const int n = g.len;
+    if ((FORM == kFormAny || FORM == kFormDirect) && (a.mode == kModeDCT2 || a.mode == kModeDST2)) {
         R *__restrict__ dst = static_cast<R *>(a.out) + ln.base;
         const C *__restrict__ post = mixed_twiddles<C>(a) + g.postoff;
 #pragma unroll
@@ -167,7 +168,7 @@ __device__ __forceinline__ void mixed_store(const C (&x)[RX], const pass_args &a
             stg<NTS>(&dst[(long long)(a.mode == kModeDST2 ? n - 1 - k : k) * a.out_sa],
                      R(2) * (w.x * x[p].x - w.y * x[p].y) * sc);
         }
-    } else if (FORM == kFormAny && (a.mode == kModeDCT3 || a.mode == kModeDST3)) {
+    } else if ((FORM == kFormAny || FORM == kFormDirect) && (a.mode == kModeDCT3 || a.mode == kModeDST3)) {
         R *__restrict__ dst = static_cast<R *>(a.out) + ln.base;
 #pragma unroll
         for (int p = 0; p < RX; p++) {
@@ -176,13 +177,13 @@ __device__ __forceinline__ void mixed_store(const C (&x)[RX], const pass_args &a
             const R y = R(2) * x[p].x;
             stg<NTS>(&dst[(long long)j * a.out_sa], ((a.mode == kModeDST3 && (j & 1)) ? -y : y) * sc);
         }
-    } else if (FORM == kFormAny && a.out_real) {
+    } else if ((FORM == kFormAny || FORM == kFormDirect) && a.out_real) {
         R *__restrict__ dst = static_cast<R *>(a.out) + ln.base;
         const R f = (a.mode == kModeDCT1B) ? R(2) * sc : sc;
 #pragma unroll
         for (int p = 0; p < RX; p++)
             if (k0 + p * step < a.store_len) stg<NTS>(&dst[(long long)(k0 + p * step) * a.out_sa], x[p].x * f);
-    } else if (FORM == kFormAny && (a.store_len < n || a.tw4)) {
+    } else if ((FORM == kFormAny || FORM == kFormDirect) && (a.store_len < n || a.tw4)) {
         C *__restrict__ dst = static_cast<C *>(a.out) + ln.base;
         const C *__restrict__ w4 = static_cast<const C *>(a.tw4);
         const unsigned jl = w4 ? mixed_line_index(ln.line, a, g, a.tw4_dim) : 0;
@@ -205,6 +206,14 @@ __device__ __forceinline__ void mixed_store(const C (&x)[RX], const pass_args &a
     }
 }
 
+// Element j of a line in the pass's input form (the chirp passes; any mode).
+template <int NTM, typename R, typename C>
+__device__ __forceinline__ C mixed_element(const pass_args &a, const mixed_plan &g, const line_at &ln, int j) {
+    C x[1];
+    mixed_load<1, kFormAny, NTM, R>(x, a, g, ln, j, 0);
+    return x[0];
+}
+
 // Stage 0: global memory -> LDS.
 template <int RX, int FORM, int NTM, typename R, typename C>
 __device__ __forceinline__ void mixed_first(const pass_args &a, const mixed_plan &g, unsigned tile, C *lds) {
@@ -225,7 +234,22 @@ __device__ __forceinline__ void mixed_first(const pass_args &a, const mixed_plan
             ln.locate(tile * T + l, a, g, false);
         }
         C x[RX];
-        mixed_load<RX, FORM, NTM, R>(x, a, g, ln, j, m);
+        if constexpr (FORM == kFormChirp) {
+            // x_j c_j for j < len, zeros behind it
+            const C *__restrict__ chirp = tw + g.chirpoff;
+#pragma unroll
+            for (int p = 0; p < RX; p++) {
+                x[p] = cmk<C>(R(0), R(0));
+                if (p * m < g.len) {
+                    const int at = j + p * m;
+                    const int jc = at < g.len ? at : g.len - 1;
+                    const C v = cmul(mixed_element<NTM, R, C>(a, g, ln, jc), chirp[jc]);
+                    if (at < g.len) x[p] = v;
+                }
+            }
+        } else {
+            mixed_load<RX, FORM, NTM, R>(x, a, g, ln, j, m);
+        }
         dft<RX>::run(x);
         if (m > 1) {
             const C *w = tw + j * (RX - 1);
@@ -238,8 +262,8 @@ __device__ __forceinline__ void mixed_first(const pass_args &a, const mixed_plan
     }
 }
 
-// A stage between two others, in place in LDS.
-template <int RX, typename R, typename C>
+// A stage between two others, in place in LDS; BACK: its transpose (twiddles before the butterfly).
+template <int RX, bool BACK, typename R, typename C>
 __device__ __forceinline__ void mixed_middle(const pass_args &a, const mixed_plan &g, const mixed_stage &st, C *lds) {
     const int T = 1 << g.log2t, m = st.m, nth = blockDim.x;
     const int stride = m * g.pitch;
@@ -254,12 +278,84 @@ __device__ __forceinline__ void mixed_middle(const pass_args &a, const mixed_pla
         C x[RX];
 #pragma unroll
         for (int p = 0; p < RX; p++) x[p] = dp[p * stride];
-        dft<RX>::run(x);
         const C *w = tw + j * (RX - 1);
+        if (BACK) {
 #pragma unroll
-        for (int q = 1; q < RX; q++) x[q] = cmul(x[q], w[q - 1]);
+            for (int q = 1; q < RX; q++) x[q] = cmul(x[q], w[q - 1]);
+        }
+        dft<RX>::run(x);
+        if (!BACK) {
+#pragma unroll
+            for (int q = 1; q < RX; q++) x[q] = cmul(x[q], w[q - 1]);
+        }
 #pragma unroll
         for (int q = 0; q < RX; q++) dp[q * stride] = x[q];
+    }
+}
+
+// Chirp passes: the last stage, the product with the transformed chirp and the first transposed
+// stage, which works on the same elements.
+template <int RX, typename R, typename C>
+__device__ __forceinline__ void mixed_center(const pass_args &a, const mixed_plan &g, const mixed_stage &st, C *lds) {
+    const int T = 1 << g.log2t, nth = blockDim.x;
+    const unsigned nb = (unsigned)g.n / RX;
+    const C *__restrict__ hat = mixed_twiddles<C>(a) + g.chirpoff + g.len;
+    for (unsigned idx = threadIdx.x; idx < nb << g.log2t; idx += nth) {
+        const int l = idx & (T - 1);
+        const unsigned c = idx >> g.log2t;
+        C *dp = lds + (int)c * RX * g.pitch + (int)fdiv(c, st.by_k0) * g.pad + l;
+        C x[RX];
+#pragma unroll
+        for (int p = 0; p < RX; p++) x[p] = dp[p * g.pitch];
+        dft<RX>::run(x);
+#pragma unroll
+        for (int q = 0; q < RX; q++) {
+            const C v = cmul(x[q], hat[c * RX + q]);
+            x[q] = cmk<C>(v.x, -v.y);
+        }
+        dft<RX>::run(x);
+#pragma unroll
+        for (int q = 0; q < RX; q++) dp[q * g.pitch] = x[q];
+    }
+}
+
+// Chirp passes: the transpose of stage 0, LDS -> global memory.
+template <int RX, int NTM, typename R, typename C>
+__device__ __forceinline__ void mixed_chirp_last(const pass_args &a, const mixed_plan &g, unsigned tile, const C *lds) {
+    const int T = 1 << g.log2t, m = g.m0, nth = blockDim.x;
+    const int stride = m * g.pitch + g.pad;
+    const C *__restrict__ tw = mixed_twiddles<C>(a);
+    const C *__restrict__ chirp = tw + g.chirpoff;
+    const bool across = a.store_colfast != 0;
+    line_at ln;
+    if (across) ln.locate(tile * T + (threadIdx.x & (T - 1)), a, g, true);
+    for (int idx = threadIdx.x; idx < m << g.log2t; idx += nth) {
+        int l, j;
+        if (across) {
+            l = idx & (T - 1);
+            j = idx >> g.log2t;
+        } else {
+            l = fdiv(idx, g.by_m0);
+            j = idx - l * m;
+            ln.locate(tile * T + l, a, g, true);
+        }
+        if (!ln.valid) continue;
+        const C *sp = lds + j * g.pitch + l;
+        const C *w = tw + j * (RX - 1);
+        C x[RX];
+#pragma unroll
+        for (int q = 0; q < RX; q++) x[q] = sp[q * stride];
+#pragma unroll
+        for (int q = 1; q < RX; q++) x[q] = cmul(x[q], w[q - 1]);
+        dft<RX>::run(x);
+#pragma unroll
+        for (int p = 0; p < RX; p++) {
+            const int k = j + p * m;
+            if (p * m < g.len && k < g.len) {
+                const C y[1] = {cmul(cmk<C>(x[p].x, -x[p].y), chirp[k])};
+                mixed_store<1, kFormAny, NTM, R>(y, a, g, ln, k, 0);
+            }
+        }
     }
 }
 
@@ -332,6 +428,105 @@ __device__ __forceinline__ void mixed_drain(const pass_args &a, const mixed_plan
     }
 }
 
+// Sums of one direct p-point butterfly at sp (elements pitch apart): outputs q and p - q for q = q0 and
+// q0 + 1.  root = w_p^t, t < p.
+template <typename R, typename C>
+__device__ __forceinline__ void mixed_direct_sums(const C *sp, int pitch, int p, int q0, const C *__restrict__ root, C (&lo)[2],
+                                                  C (&hi)[2]) {
+    const C x0 = sp[0];
+    C re[2] = {x0, x0}, im[2] = {cmk<C>(R(0), R(0)), cmk<C>(R(0), R(0))};
+    int t[2] = {0, 0};
+    const C *a = sp, *b = sp + p * pitch;
+#pragma unroll 2
+    for (int k = 1; k <= (p - 1) / 2; k++) {
+        a += pitch;
+        b -= pitch;
+        const C xa = *a, xb = *b;
+        const C s = cadd(xa, xb), d = csub(xa, xb);
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            t[i] += q0 + i;
+            t[i] -= t[i] >= p ? p : 0;
+            const C w = root[t[i]];  // (cos, -sin) of 2 pi k q / p
+            re[i].x += s.x * w.x;
+            re[i].y += s.y * w.x;
+            im[i].x += d.x * w.y;
+            im[i].y += d.y * w.y;
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+        lo[i] = cmk<C>(re[i].x - im[i].y, re[i].y + im[i].x);
+        hi[i] = cmk<C>(re[i].x + im[i].y, re[i].y - im[i].x);
+    }
+}
+
+// A direct stage before the last one: from one LDS buffer to the other.
+template <typename R, typename C>
+__device__ __forceinline__ void mixed_direct(const pass_args &a, const mixed_plan &g, const mixed_stage &st, const C *from, C *to) {
+    const int T = 1 << g.log2t, p = st.radix, m = st.m, groups = (p + 3) / 4;
+    const unsigned nb = (unsigned)(g.n / p);
+    const C *__restrict__ tw = mixed_twiddles<C>(a) + st.twoff, *__restrict__ root = mixed_twiddles<C>(a) + st.root;
+    for (unsigned idx = threadIdx.x; idx < (nb * groups) << g.log2t; idx += blockDim.x) {
+        const int l = idx & (T - 1);
+        const unsigned v = idx >> g.log2t;
+        const unsigned grp = v / nb, b = v - grp * nb;
+        const unsigned c = fdiv(b, st.by_m);
+        const int j = (int)(b - c * (unsigned)m), at = ((int)c * p * m + j) * g.pitch + l;
+        C lo[2], hi[2];
+        mixed_direct_sums<R>(from + at, m * g.pitch, p, 2 * (int)grp, root, lo, hi);
+        C *dp = to + at;
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            const int q = 2 * (int)grp + i;
+            if (q > (p - 1) / 2) continue;
+            dp[q * m * g.pitch] = q == 0 ? lo[i] : cmul(lo[i], tw[j * (p - 1) + q - 1]);
+            if (q > 0) dp[(p - q) * m * g.pitch] = cmul(hi[i], tw[j * (p - 1) + p - q - 1]);
+        }
+    }
+}
+
+// A direct last stage: LDS -> global memory.
+template <int NTM, typename R, typename C>
+__device__ __forceinline__ void mixed_direct_last(const pass_args &a, const mixed_plan &g, unsigned tile, const C *lds) {
+    const int T = 1 << g.log2t, p = g.last, groups = (p + 3) / 4;
+    const unsigned nb = (unsigned)(g.n / p), per_line = nb * groups;
+    const C *__restrict__ root = mixed_twiddles<C>(a) + g.root_last;
+    for (unsigned idx = threadIdx.x; idx < per_line << g.log2t; idx += blockDim.x) {
+        unsigned l, v;
+        if (a.store_colfast) {
+            l = idx & (T - 1);
+            v = idx >> g.log2t;
+        } else {
+            l = idx / per_line;
+            v = idx - l * per_line;
+        }
+        const unsigned grp = fdiv(v, g.by_last), u = v - grp * nb;
+        line_at ln;
+        ln.locate(tile * T + l, a, g, true);
+        if (!ln.valid) continue;
+        unsigned c = 0, t = u;
+#pragma unroll
+        for (int s = 0; s + 2 < kMixedStages; s++) {
+            if (s + 2 >= g.nst) break;
+            const unsigned q = fdiv(t, g.by_r[s]);
+            c = (c + t - q * (unsigned)g.radix[s]) * (unsigned)g.radix[s + 1];
+            t = q;
+        }
+        c += t;
+        C lo[2], hi[2];
+        mixed_direct_sums<R>(lds + (int)c * p * g.pitch + (int)l, g.pitch, p, 2 * (int)grp, root, lo, hi);
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            const int q = 2 * (int)grp + i;
+            if (q > (p - 1) / 2) continue;
+            const C x[1] = {lo[i]}, y[1] = {hi[i]};
+            mixed_store<1, kFormAny, NTM, R>(x, a, g, ln, (int)(u + nb * q), 0);
+            if (q > 0) mixed_store<1, kFormAny, NTM, R>(y, a, g, ln, (int)(u + nb * (p - q)), 0);
+        }
+    }
+}
+
 // Radices of the light build (every thread holds at most kLightRadix values) and of the full one.
 #define HMI_MIXED_LIGHT(X) X(2) X(3) X(4) X(5) X(6) X(7) X(8) X(9) X(10)
 #define HMI_MIXED_HEAVY(X) X(11) X(12) X(13) X(14) X(15) X(16)
@@ -354,37 +549,64 @@ __global__ void __launch_bounds__(kMixedThreads) fft_generic(pass_args a, mixed_
         }
     }
 #define HMI_MIXED_FIRST(RX) case RX: mixed_first<RX, FORM, NTM, R>(a, g, tile, lds); break;
-#define HMI_MIXED_MID(RX) case RX: mixed_middle<RX, R>(a, g, st, lds); break;
+#define HMI_MIXED_MID(RX) case RX: mixed_middle<RX, false, R>(a, g, st, lds); break;
+#define HMI_MIXED_BACK(RX) case RX: mixed_middle<RX, true, R>(a, g, st, lds); break;
+#define HMI_MIXED_CENTER(RX) case RX: mixed_center<RX, R>(a, g, st, lds); break;
 #define HMI_MIXED_LAST(RX) case RX: mixed_last<RX, FORM, NTM, R>(a, g, tile, lds); break;
-    if (g.nst == 0) {
-        mixed_fill<FORM, NTM, R>(a, g, tile, lds);
-    } else if constexpr (HEAVY) {
-        switch (g.radix[0]) { HMI_MIXED_LIGHT(HMI_MIXED_FIRST) HMI_MIXED_HEAVY(HMI_MIXED_FIRST) }
+#define HMI_MIXED_CHIRP_LAST(RX) case RX: mixed_chirp_last<RX, NTM, R>(a, g, tile, lds); break;
+#define HMI_MIXED_SWITCH(R, CASE)                                                     \
+    if constexpr (HEAVY) {                                                            \
+        switch (R) { HMI_MIXED_LIGHT(CASE) HMI_MIXED_HEAVY(CASE) }                    \
+    } else {                                                                          \
+        switch (R) { HMI_MIXED_LIGHT(CASE) }                                          \
+    }
+    const mixed_stage *stages = static_cast<const mixed_stage *>(a.tw);
+    [[maybe_unused]] C *other = lds + g.n * g.pitch;  // plans with two direct stages or more
+    if (FORM != kFormChirp && (g.nst == 0 || g.radix[0] > 16)) {
+        if constexpr (FORM != kFormChirp) mixed_fill<FORM, NTM, R>(a, g, tile, lds);
+        if (FORM == kFormDirect && g.nst > 1) {
+            __syncthreads();
+            const mixed_stage st{g.radix[0], g.m0, 0, g.by_m0, fast_div{}, g.root0};
+            mixed_direct<R>(a, g, st, lds, other);
+            C *t = lds; lds = other; other = t;
+        }
     } else {
-        switch (g.radix[0]) { HMI_MIXED_LIGHT(HMI_MIXED_FIRST) }
+        HMI_MIXED_SWITCH(g.radix[0], HMI_MIXED_FIRST)
     }
     __syncthreads();
     for (int s = 1; s + 1 < g.nst; s++) {
-        const mixed_stage st = static_cast<const mixed_stage *>(a.tw)[s - 1];
-        if constexpr (HEAVY) {
-            switch (st.radix) { HMI_MIXED_LIGHT(HMI_MIXED_MID) HMI_MIXED_HEAVY(HMI_MIXED_MID) }
+        const mixed_stage st = stages[s - 1];
+        if (FORM == kFormDirect && st.radix > 16) {
+            mixed_direct<R>(a, g, st, lds, other);
+            C *t = lds; lds = other; other = t;
         } else {
-            switch (st.radix) { HMI_MIXED_LIGHT(HMI_MIXED_MID) }
+            HMI_MIXED_SWITCH(st.radix, HMI_MIXED_MID)
         }
         __syncthreads();
     }
-    if (g.nst < 2) {
+    if constexpr (FORM == kFormChirp) {
+        for (int s = g.nst - 1; s > 0; s--) {
+            const mixed_stage st = stages[s - 1];
+            if (s == g.nst - 1) {
+                HMI_MIXED_SWITCH(st.radix, HMI_MIXED_CENTER)
+            } else {
+                HMI_MIXED_SWITCH(st.radix, HMI_MIXED_BACK)
+            }
+            __syncthreads();
+        }
+        HMI_MIXED_SWITCH(g.radix[0], HMI_MIXED_CHIRP_LAST)
+    } else if (FORM == kFormDirect) {
+        mixed_direct_last<NTM, R>(a, g, tile, lds);
+    } else if (g.nst < 2) {
         mixed_drain<FORM, NTM, R>(a, g, tile, lds);
-    } else if constexpr (HEAVY) {
-        switch (g.last) { HMI_MIXED_LIGHT(HMI_MIXED_LAST) HMI_MIXED_HEAVY(HMI_MIXED_LAST) }
     } else {
-        switch (g.last) { HMI_MIXED_LIGHT(HMI_MIXED_LAST) }
+        HMI_MIXED_SWITCH(g.last, HMI_MIXED_LAST)
     }
 }
 
 template <typename R> struct generic_builds {
     using fn = void (*)(pass_args, mixed_plan);
-    // [full radix set][kFormAny, kFormPlain, kFormPlain32][non-temporal: none, stores, loads and stores]
+    // [full radix set][kFormAny, kFormPlain, kFormPlain32, kFormChirp, kFormDirect][non-temporal: none, stores, both]
     static fn pick(bool heavy, int form, int stream) {
 #ifdef HMI_EMULATE  // the CPU tests run the kernels without the non-temporal hints
 #define HMI_MIXED_BUILDS(H, F) {&fft_generic<R, H, F, 0>, nullptr, nullptr}
@@ -392,16 +614,16 @@ template <typename R> struct generic_builds {
 #define HMI_MIXED_BUILDS(H, F) \
     {&fft_generic<R, H, F, 0>, &fft_generic<R, H, F, kStreamStores>, &fft_generic<R, H, F, kStreamLoadsStores>}
 #endif
-        static const fn f[2][3][3] = {
-            {HMI_MIXED_BUILDS(false, 0), HMI_MIXED_BUILDS(false, 1), HMI_MIXED_BUILDS(false, 2)},
-            {HMI_MIXED_BUILDS(true, 0), HMI_MIXED_BUILDS(true, 1), HMI_MIXED_BUILDS(true, 2)}};
+        static const fn f[2][5][3] = {
+            {HMI_MIXED_BUILDS(false, 0), HMI_MIXED_BUILDS(false, 1), HMI_MIXED_BUILDS(false, 2), HMI_MIXED_BUILDS(false, 3), HMI_MIXED_BUILDS(false, 4)},
+            {HMI_MIXED_BUILDS(true, 0), HMI_MIXED_BUILDS(true, 1), HMI_MIXED_BUILDS(true, 2), HMI_MIXED_BUILDS(true, 3), HMI_MIXED_BUILDS(true, 4)}};
         return f[heavy ? 1 : 0][form][stream == 0 ? 0 : (stream == kStreamStores ? 1 : 2)];
     }
     static fn choose(const pass_args &a, const mixed_plan &g) {
         int top = 0;
-        for (int i = 0; i < g.nst; i++) top = std::max(top, g.radix[i]);
+        for (int i = 0; i < g.nst; i++) top = g.radix[i] <= 16 ? std::max(top, g.radix[i]) : top;
         const bool plain = a.mode == kModeC2C && !a.in_real && !a.out_real && !a.herm_load && !a.mul && !a.tw4 &&
-                           a.store_len == g.n;
+                           a.store_len == g.len;
         // elements up to the furthest one of either side (no stride is negative)
         auto span = [&](long long sa, long long sc, long long sb1, long long sb2) {
             return (g.n - 1) * sa + (a.ncol - 1) * sc + (a.nb1 - 1) * sb1 + (a.nbatch - 1) * sb2 + 1;
@@ -409,7 +631,7 @@ template <typename R> struct generic_builds {
         const long long most = std::max(span(a.in_sa, a.in_sc, a.in_sb1, a.in_sb2),
                                         span(a.out_sa, a.out_sc, a.out_sb1, a.out_sb2));
         const bool near = most * (long long)sizeof(typename cvec<R>::type) <= (1LL << 32);
-        return pick(top > kLightRadix, !plain ? kFormAny : (near ? kFormPlain32 : kFormPlain), a.stream);
+        return pick(top > kLightRadix, g.chirp ? kFormChirp : g.direct ? kFormDirect : !plain ? kFormAny : (near ? kFormPlain32 : kFormPlain), a.stream);
     }
 #ifndef HMI_EMULATE
     static hipError_t launch(const pass_args &a, const mixed_plan &g, int threads, long long nblocks, size_t lds,
@@ -417,7 +639,7 @@ template <typename R> struct generic_builds {
         // once per process, thread-safe (static initialisation)
         static const bool configured = [] {
             for (bool heavy : {false, true})
-                for (int form = 0; form < 3; form++)
+                for (int form = 0; form < 5; form++)
                     for (int st : {0, (int)kStreamStores, (int)kStreamLoadsStores})
                         (void)hipFuncSetAttribute(reinterpret_cast<const void *>(pick(heavy, form, st)),
                                                   hipFuncAttributeMaxDynamicSharedMemorySize, kGenericMaxLds);

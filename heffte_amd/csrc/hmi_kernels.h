@@ -30,9 +30,6 @@ struct fast_kernel_info {
 // chunks); otherwise the variant with the fewest lines per block is returned.
 const fast_kernel_info *find_fast_kernel(int n, bool dbl, bool wide);
 
-hipError_t launch_generic(bool dbl, const pass_args &a, const generic_plan &g, long long nblocks, size_t lds_bytes,
-                          hipStream_t s);
-
 // Runtime-length pass (hmi_generic.h): at most kMixedThreads threads per block; plans whose radices
 // all stay within kLightRadix run a build of their own with fewer registers.
 constexpr int kMixedThreads = 512;

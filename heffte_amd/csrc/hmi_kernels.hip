@@ -640,12 +640,6 @@ __device__ __forceinline__ void staged_tile(const pass_args &a, unsigned tile, t
     }
 }
 
-template <typename R>
-__global__ void __launch_bounds__(256) fft_generic(pass_args a, generic_plan g) {
-    extern __shared__ __align__(16) unsigned char smem_raw[];
-    generic_tile<R>(a, g, blockIdx.x, reinterpret_cast<typename cvec<R>::type *>(smem_raw));
-}
-
 // --------------------------------------------------------------- batched
 
 // One phase (one axis) of a batch of independent c2c transforms of different
@@ -1342,22 +1336,6 @@ const fast_kernel_info *find_fast_kernel(int n, bool dbl, bool wide) {
         if (!best || (wide ? k.T > best->T : k.T < best->T)) best = &k;
     }
     return best;
-}
-
-hipError_t launch_generic(bool dbl, const pass_args &a, const generic_plan &g, long long nblocks, size_t lds_bytes,
-                          hipStream_t s) {
-    // once per process, thread-safe (static initialisation)
-    static const bool configured = [] {
-        (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&fft_generic<float>),
-                                  hipFuncAttributeMaxDynamicSharedMemorySize, kGenericMaxLds);
-        (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&fft_generic<double>),
-                                  hipFuncAttributeMaxDynamicSharedMemorySize, kGenericMaxLds);
-        return true;
-    }();
-    (void)configured;
-    if (dbl) fft_generic<double><<<dim3((unsigned)nblocks), dim3(256), lds_bytes, s>>>(a, g);
-    else fft_generic<float><<<dim3((unsigned)nblocks), dim3(256), lds_bytes, s>>>(a, g);
-    return hipGetLastError();
 }
 
 hipError_t launch_permute(int elem_bytes, const void *src, void *dst, const permute_args &p, hipStream_t s) {

@@ -91,28 +91,44 @@ struct fast_div {
 // leaves it at base + j + q m_s; frequency k_0 + r_0 k_1 + r_0 r_1 k_2 + ... ends at position
 // k_0 m_0 + k_1 m_1 + ...  Element (line l, position i) of a tile sits at
 // i pitch + (i / m_0) pad + l.
+//
+// Prime factors from 17 to 61 are direct stages, behind the others: an output pair (q, p - q) sums the
+// (p - 1) / 2 input pairs (k, p - k) against the table w_p^t.  The last stage takes them from LDS to
+// global memory; a length with two or three such factors runs the earlier ones from one LDS buffer
+// to a second one.
+//
+// Lines of len points whose length has a larger prime factor run as a chirp convolution (Bluestein,
+// 1970): j k = (j^2 + k^2 - (k - j)^2) / 2, so X_k = c_k sum_j (x_j c_j) conj(c_{k-j}) with c_j =
+// exp(-i pi j^2 / len), a cyclic convolution of n >= 2 len - 1 points, n with radices up to 16.  The
+// stages above transform x_j c_j, the last one multiplies by the transform of conj(c) (in position
+// order, times 1 / n) and conjugates, and the transposed stages S-1 ... 0 lead back to natural order.
 enum : int { kMixedStages = 6 };
 struct mixed_plan {
     int n, nst;
+    int len;                         // points of a line (n, unless chirp)
+    int chirp, direct;               // direct: number of direct stages
     int log2t, pitch, pad;           // lines per tile 2^log2t, LDS strides (elements)
     int radix[kMixedStages];
     int m0;                          // the first stage's twiddles w_n^{j q}: table[j (r_0 - 1) + q - 1]
     int last;                        // r_{S-1}
     int postoff;                     // real-data twiddles (modes other than kModeC2C)
+    int root0, root_last;            // w_p^t, t < p, of a direct first and last stage
+    int chirpoff;                    // c_j, j < len, then the transform of conj(c) in position order
     fast_div by_r[kMixedStages];     // / r_s
     fast_div by_m0, by_last;         // / m_0, / (n / r_{S-1})
     fast_div by_n, by_ncol, by_nb1;  // line and element numbering
 };
 
-// Stages 1 to S - 2 of the plan, at the start of its device table (kMixedHead bytes; the twiddles
+// Stages 1 to S - 1 of the plan, at the start of its device table (kMixedHead bytes; the twiddles
 // follow): the kernel walks them with a run-time index, which a kernel argument would not allow
 // without a copy to scratch memory.
 struct mixed_stage {
     int radix, m, twoff;
     fast_div by_m, by_k0;            // / m_s, / (r_1 ... r_{s-1}): block number -> k_0
+    int root;                        // w_r^t, t < r, of a direct stage
 };
-enum : int { kMixedHead = 128 };
-static_assert(sizeof(mixed_stage) * (kMixedStages - 2) <= kMixedHead, "the middle stages fit the table head");
+enum : int { kMixedHead = 192 };
+static_assert(sizeof(mixed_stage) * (kMixedStages - 1) <= kMixedHead, "the stages fit the table head");
 
 // Batched mixed-size transforms (one phase = one axis of every transform).
 // Every transform is a c2c box in order (0, 1, 2) at its own element offset.

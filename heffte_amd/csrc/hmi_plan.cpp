@@ -403,35 +403,6 @@ void fft_plan::configure(pass &p, bool dbl, bool sizes_only) const {
         return;
     }
     const size_t per_line = 2 * (size_t)p.n * elem;
-    if (per_line <= (size_t)kGenericMaxLds) {
-        if (sizes_only) return;  // no step buffer: nothing else the workspace depends on
-        const long long ncol = std::max(p.lin.n[p.col], p.lout.n[p.col]);
-        const mixed_config c = make_mixed(p.n, dbl, p.identity, p.load_colfast, p.store_colfast, ncol,
-                                          ncol * std::max(p.lin.n[p.b1], p.lout.n[p.b1]));
-        if (c.ok) {
-            p.mixed = std::make_shared<mixed_config>(c);
-            p.lines = 1 << c.plan.log2t;
-            return;
-        }
-    }
-    p.gen = std::make_shared<generic_plan>();
-    generic_plan &g = *p.gen;
-    g.n = p.n;
-    std::vector<int> rad = p.identity ? std::vector<int>{} : factorize(p.n);
-    if ((int)rad.size() > kMaxStages) throw std::runtime_error("too many radix stages");
-    g.nstages = (int)rad.size();
-    int off = 0, ls = 1;
-    for (int s = 0; s < g.nstages; s++) {
-        g.radix[s] = rad[s];
-        g.twoff[s] = off;
-        off += ls * (rad[s] - 1);
-        ls *= rad[s];
-    }
-    for (int s = 0; s < g.nstages; s++) {
-        g.rootoff[s] = off;
-        if (!has_butterfly(rad[s])) off += rad[s];
-    }
-    g.postoff = off;
     if (per_line > (size_t)kGenericMaxLds) {
         // beyond one LDS tile: two passes of lengths n1 * n2 = n (plain c2c lines only)
         int n1 = 0, n2 = 0;
@@ -459,12 +430,14 @@ void fft_plan::configure(pass &p, bool dbl, bool sizes_only) const {
         p.lines = 1;
         return;
     }
-    int lines = (int)std::min<size_t>(64, std::max<size_t>(1, (64 * 1024) / per_line));
-    // no more lines per block than columns
-    const long long ncol = p.lin.n[p.col] > 0 ? std::max(p.lin.n[p.col], p.lout.n[p.col]) : 1;
-    while (lines > 1 && lines / 2 >= ncol) lines /= 2;
-    g.lines = lines;
-    p.lines = lines;
+    if (sizes_only) return;  // no step buffer: nothing else the workspace depends on
+    const long long ncol = std::max(p.lin.n[p.col], p.lout.n[p.col]);
+    const int tail = (p.mode >= kModeDCT2 && p.mode <= kModeDST3) ? p.n : 0;
+    auto c = std::make_shared<mixed_config>(make_mixed(p.n, dbl, p.identity, p.load_colfast, p.store_colfast, ncol,
+                                                       ncol * std::max(p.lin.n[p.b1], p.lout.n[p.b1]), tail));
+    if (!c->ok) throw std::runtime_error("transform length " + std::to_string(p.n) + " has no single-pass plan");
+    p.lines = 1 << c->plan.log2t;
+    p.mixed = c;
 }
 
 namespace {
@@ -599,13 +572,11 @@ std::string pass_kernel_name(const pass &p, bool dbl, bool mfma, int precision, 
 const twiddles &fft_plan::get_twiddles(bool dbl, const pass &p, bool may_alloc) {
     const int n = p.n;
     const long long key = ((long long)n << 8) | (dbl ? 1 : 0) | (p.fast ? 2 : 0) | (p.identity ? 4 : 0) |
-                          ((long long)p.mode << 3) | (p.fast ? (long long)p.fast->T << 40 : 0) | (p.mixed ? 1LL << 56 : 0);
+                          ((long long)p.mode << 3) | (p.fast ? (long long)p.fast->T << 40 : 0);
     std::lock_guard<std::mutex> lock(mtx_);
     auto it = tw_.find(key);
     if (it != tw_.end()) return it->second;
     if (!may_alloc) throw std::runtime_error(kNotResident);
-    const int *radix = p.fast ? p.fast->radix : (p.gen ? p.gen->radix : nullptr);
-    const int ns = p.fast ? p.fast->nstages : (p.gen ? p.gen->nstages : 0);
     twiddles t;
     // r2c / c2r: w_n^k for k < n/2 (n = real line length); r2r: w_{4n}^k for k < n
     int tail_count = 0;
@@ -613,15 +584,15 @@ const twiddles &fft_plan::get_twiddles(bool dbl, const pass &p, bool may_alloc) 
     if (p.mode == kModeR2C || p.mode == kModeC2R) { tail_count = n / 2; tail_mod = n; }
     if (p.mode >= kModeDCT2 && p.mode <= kModeDST3) { tail_count = n; tail_mod = 4LL * n; }
     if (p.mixed) {
-        const std::vector<unsigned char> v = mixed_table(n, dbl, p.identity, tail_count, tail_mod);
+        const std::vector<unsigned char> v = mixed_table(p.mixed->plan, dbl, tail_mod);
         t.bytes = v.size();
         t.dev = upload_bytes(v.data(), t.bytes);
     } else if (dbl) {
-        std::vector<double> v = make_table<double>(radix, ns, !p.fast, tail_count, tail_mod);
+        std::vector<double> v = make_table<double>(p.fast->radix, p.fast->nstages, false, tail_count, tail_mod);
         t.bytes = v.size() * sizeof(double);
         t.dev = upload_bytes(v.data(), t.bytes);
     } else {
-        std::vector<float> v = make_table<float>(radix, ns, !p.fast, tail_count, tail_mod);
+        std::vector<float> v = make_table<float>(p.fast->radix, p.fast->nstages, false, tail_count, tail_mod);
         t.bytes = v.size() * sizeof(float);
         t.dev = upload_bytes(v.data(), t.bytes);
     }
@@ -800,7 +771,6 @@ void launch_mixed_pass(const pass &p, const pass_args &a, bool dbl, long long nb
 }  // namespace
 
 void fft_plan::launch_split(const pass &p, const pass_args &base, bool dbl, int batch, void *tmp) {
-    const size_t elem = dbl ? 16 : 8;
     for (int bt = 0; bt < batch; bt++) {
         pass_args st[2];
         split_steps(p, base, dbl, bt, tmp, st);
@@ -810,9 +780,7 @@ void fft_plan::launch_split(const pass &p, const pass_args &base, bool dbl, int 
             st[i].tw = get_twiddles(dbl, q, false).dev;
             const long long nblocks = ((long long)st[i].nlines + q.lines - 1) / q.lines;
             if (q.fast) check_hip(q.fast->launch(st[i], nblocks, stream_), "split FFT pass");
-            else if (q.mixed) launch_mixed_pass(q, st[i], dbl, nblocks, stream_);
-            else check_hip(launch_generic(dbl, st[i], *q.gen, nblocks, 2 * (size_t)q.gen->lines * q.n * elem, stream_),
-                           "split FFT pass");
+            else launch_mixed_pass(q, st[i], dbl, nblocks, stream_);
         }
     }
 }
@@ -912,11 +880,8 @@ void fft_plan::execute(int dir, bool dbl, bool in_real, bool out_real, int batch
             check_hip(launch_mfma512(precision_, a, ((long long)a.nlines + 15) / 16, stream_), "MFMA FFT pass");
         } else if (p.fast) {
             check_hip(p.fast->launch(a, nblocks, stream_), "fast FFT pass");
-        } else if (p.mixed) {
-            launch_mixed_pass(p, a, dbl, nblocks, stream_);
         } else {
-            const size_t lds = 2 * (size_t)p.gen->lines * p.n * (dbl ? 16 : 8);
-            check_hip(launch_generic(dbl, a, *p.gen, nblocks, lds, stream_), "generic FFT pass");
+            launch_mixed_pass(p, a, dbl, nblocks, stream_);
         }
         if (tprev) {
             const std::string name = pass_kernel_name(p, dbl, mfma, precision_, a);

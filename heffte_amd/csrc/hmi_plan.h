@@ -50,7 +50,7 @@ struct layout {
 
 // Radix plan, tile and block of the runtime-length pass for one pass of length n.
 struct mixed_config {
-    bool ok = false;   // false: n has a prime factor without a butterfly
+    bool ok = false;   // false: no plan fits one LDS tile
     mixed_plan plan{};
     int threads = 64;
     size_t lds = 0;
@@ -69,7 +69,6 @@ struct pass {
     int mode = 0;           // kModeC2C, or kModeR2C / kModeC2R when the half-length kernel runs it
     // launch configuration
     const fast_kernel_info *fast = nullptr;
-    std::shared_ptr<generic_plan> gen;          // set: lengths with a prime factor above 13
     std::shared_ptr<const mixed_config> mixed;  // set: the runtime-length pass runs it
     int lines = 1;  // lines (columns) per block
     // A length whose line does not fit one LDS tile runs as two passes (four-step), n = n1 n2,
@@ -177,15 +176,15 @@ class fft_plan {
     void clear_timing();
 };
 
-// Radix order of the runtime-length pass (empty: n has a prime factor above 13), its tile for one
+// Radix order of the runtime-length pass (empty: n has a prime factor above 13), and its tile for one
 // pass (copy: no transform, only the layout change; *_across: that side walks the column axis; ncol
-// columns, nlines lines in all), and its device table: the middle stages' entries, the stage
-// twiddles, then w_{tail_mod}^k for k < tail_count (at mixed_post_offset).
+// columns, nlines lines in all; tail: real-data twiddles).  Device table: the later stages' entries,
+// the stage twiddles, w_{tail_mod}^k for k < tail, the chirp and its transform.
 std::vector<int> mixed_radices(int n, bool dbl);
 mixed_config make_mixed(int n, bool dbl, bool copy, bool load_across, bool store_across, long long ncol,
-                        long long nlines);
+                        long long nlines, int tail);
 int mixed_post_offset(const std::vector<int> &radices);
-std::vector<unsigned char> mixed_table(int n, bool dbl, bool copy, int tail_count, long long tail_mod);
+std::vector<unsigned char> mixed_table(const mixed_plan &g, bool dbl, long long tail_mod);
 // the divisors of one launch's line numbering
 void mixed_launch_divs(mixed_plan &g, const pass_args &a);
 

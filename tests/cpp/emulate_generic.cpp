@@ -59,7 +59,8 @@ template <typename R> int run_case(int n, int mode, int flags, int oi, int oo, i
     if (herm) nin = n / 2 + 1;
     const sides si = layout_of(oi, nin, ncol, nb1), so = layout_of(oo, nout, ncol, nb1);
     const bool load_across = si.sa != 1 && nin > 1, store_across = so.sa != 1 && nout > 1;
-    const hmi::mixed_config c = hmi::make_mixed(n, dbl, copy, load_across, store_across, ncol, (long long)ncol * nb1);
+    const int tail = (mode >= hmi::kModeDCT2 && mode <= hmi::kModeDST3) ? n : 0;
+    const hmi::mixed_config c = hmi::make_mixed(n, dbl, copy, load_across, store_across, ncol, (long long)ncol * nb1, tail);
     what = "n=" + std::to_string(n) + (dbl ? " f64" : " f32") + " mode=" + std::to_string(mode) + " flags=" +
            std::to_string(flags) + " orders=" + std::to_string(oi) + std::to_string(oo) + " ncol=" + std::to_string(ncol) +
            " nb1=" + std::to_string(nb1) + " batch=" + std::to_string(batch);
@@ -72,9 +73,7 @@ template <typename R> int run_case(int n, int mode, int flags, int oi, int oo, i
     for (size_t i = 0; i < cin * (rin ? 1 : 2); i++) in[i] = (R)d(rng);
     if (mul) for (size_t i = 0; i < cin * 2; i++) mul[i] = (R)d(rng);
     for (size_t i = 0; i < cout * (rout ? 1 : 2); i++) out[i] = (R)77;
-    int tail = 0;
-    if (mode >= hmi::kModeDCT2 && mode <= hmi::kModeDST3) tail = n;
-    const std::vector<unsigned char> tab = hmi::mixed_table(n, dbl, copy, tail, 4LL * n);
+    const std::vector<unsigned char> tab = hmi::mixed_table(c.plan, dbl, 4LL * n);
     unsigned char *table = new unsigned char[tab.size()];
     std::copy(tab.begin(), tab.end(), table);
     // w_{n ncol}^m of a split axis whose interleaved index is the column
@@ -194,7 +193,13 @@ int main(int argc, char **argv) {
             for (int k = 0; k < 3; k++)
                 one(dbl, n, hmi::kModeC2C, pick(0, 1) * 64, k == 0 ? 0 : pick(0, 5), k == 0 ? 2 : pick(0, 5), pick(1, 21),
                     pick(1, 3), pick(1, 2));
-    const int few[] = {1, 2, 6, 13, 22, 45, 60, 77, 105, 180, 216};
+    // direct stages, one to three of them, and chirp convolutions of two to four stages
+    for (bool dbl : {false, true})
+        for (int n : {17, 19, 23, 34, 37, 51, 61, 67, 68, 97, 127, 158, 186, 199, 254, 257, 289, 323, 509, 578})
+            for (int k = 0; k < 3; k++)
+                one(dbl, n, hmi::kModeC2C, pick(0, 1) * 64, k == 0 ? 0 : pick(0, 5), k == 0 ? 2 : pick(0, 5), pick(1, 21),
+                    pick(1, 3), pick(1, 2));
+    const int few[] = {1, 2, 6, 13, 17, 22, 38, 134, 289, 45, 60, 77, 105, 127, 180, 216};
     for (bool dbl : {false, true})
         for (int n : few) {
             for (int flags : {1, 2, 2 | 8, 4 | 64, 4 | 16 | 64, 16 | 64, 32, 32 | 64, 128, 256, 256 | 64, 8}) {
@@ -207,7 +212,7 @@ int main(int argc, char **argv) {
         }
     // few lines per tile and the largest tile
     for (bool dbl : {false, true})
-        for (int n : {1000, 1331, 2187, 2400, 5000}) one(dbl, n, hmi::kModeC2C, 0, 0, pick(2, 5), 3, 1, 1);
+        for (int n : {1000, 1021, 1331, 2187, 2400, 4913, 4999, 5000}) one(dbl, n, hmi::kModeC2C, 0, 0, pick(2, 5), 3, 1, 1);
     std::printf("%s %d\n", fails ? "failed" : "ok", cases);
     return fails ? 1 : 0;
 }

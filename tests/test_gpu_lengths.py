@@ -1,6 +1,6 @@
 """GPU parity of the runtime-length pass over the lengths whose plans differ: one to five stages, every
-radix, odd and even, up to the longest lines of one LDS tile, with the axis contiguous or across
-columns on either side."""
+radix, direct stages (a prime factor from 17 to 61), chirp convolutions (a larger one), odd and even,
+up to the longest lines of one LDS tile, with the axis contiguous or across columns on either side."""
 import numpy as np
 import pytest
 
@@ -9,7 +9,8 @@ import fftcase as fc
 pytestmark = pytest.mark.gpu
 
 LENGTHS = [2, 3, 7, 10, 11, 13, 14, 15, 18, 22, 25, 26, 36, 49, 50, 60, 72, 81, 90, 91, 100, 121, 125, 143, 150, 169, 180,
-           225, 240, 250, 320, 343, 384, 400, 625, 768, 1000, 1331, 2187, 2400, 3125, 5000]
+           225, 240, 250, 320, 343, 384, 400, 625, 768, 1000, 1331, 2187, 2400, 3125, 5000,
+           17, 19, 34, 37, 51, 61, 186, 289, 323, 4913, 67, 127, 158, 199, 254, 509, 2003, 4999]
 
 
 @pytest.mark.parametrize("dtype", ["complex64", "complex128"])
@@ -35,7 +36,7 @@ def test_c2c_lengths(hmi, cuda, oracle, dtype, n):
 
 
 @pytest.mark.parametrize("dtype", ["float32", "float64"])
-@pytest.mark.parametrize("n", [2, 6, 15, 25, 36, 50, 60, 99, 100, 147, 180, 225, 250, 300, 390, 720, 1000])
+@pytest.mark.parametrize("n", [17, 38, 127, 254, 2, 6, 15, 25, 36, 50, 60, 99, 100, 147, 180, 225, 250, 300, 390, 720, 1000])
 def test_r2c_and_r2r_lengths(hmi, cuda, oracle, dtype, n):
     import torch
     rdt = np.float32 if dtype == "float32" else np.float64

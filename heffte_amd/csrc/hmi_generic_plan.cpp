@@ -144,8 +144,8 @@ int chirp_length(int n, bool dbl) {
     return best;
 }
 
-mixed_config make_mixed(int n, bool dbl, bool copy, bool load_across, bool store_across, long long ncol,
-                        long long nlines, int tail) {
+mixed_config make_mixed(int n, bool dbl, bool copy, bool load_across, bool store_across, long long nlines,
+                        int tail) {
     mixed_config c{};
     mixed_plan &g = c.plan;
     std::vector<int> rad = (copy || n == 1) ? std::vector<int>{} : mixed_radices(n, dbl);
@@ -192,8 +192,8 @@ mixed_config make_mixed(int n, bool dbl, bool copy, bool load_across, bool store
     int l2 = 0;
     while (l2 < 6 && (n * elem << (l2 + 1)) <= kMixedTile) l2++;
     while ((elem << l2) < 128 && bytes(2 << l2) <= (across ? kGenericMaxLds : kGenericMaxLds / 2)) l2++;
-    const long long cap = across ? ncol : nlines;
-    while (l2 > 0 && (1LL << (l2 - 1)) >= cap) l2--;
+    // few lines in all (nlines > 0): smaller tiles on more CUs, down to 64-byte chunks
+    while (nlines > 0 && l2 > (across ? (dbl ? 2 : 3) : 0) && (nlines >> l2) < kFewBlocks) l2--;
     g.log2t = l2;
     const int T = 1 << l2;
     g.pitch = walk && T > 1 ? T + 1 : T;

@@ -431,12 +431,13 @@ void fft_plan::configure(pass &p, bool dbl, bool sizes_only) const {
         return;
     }
     if (sizes_only) return;  // no step buffer: nothing else the workspace depends on
-    const long long ncol = std::max(p.lin.n[p.col], p.lout.n[p.col]);
     const int tail = (p.mode >= kModeDCT2 && p.mode <= kModeDST3) ? p.n : 0;
-    auto c = std::make_shared<mixed_config>(make_mixed(p.n, dbl, p.identity, p.load_colfast, p.store_colfast, ncol,
-                                                       ncol * std::max(p.lin.n[p.b1], p.lout.n[p.b1]), tail));
-    if (!c->ok) throw std::runtime_error("transform length " + std::to_string(p.n) + " has no single-pass plan");
-    p.lines = 1 << c->plan.log2t;
+    const long long lines = std::max(p.lin.n[p.col], p.lout.n[p.col]) * std::max(p.lin.n[p.b1], p.lout.n[p.b1]);
+    auto c = std::make_shared<std::array<mixed_config, 2>>();
+    for (int few = 0; few < 2; few++)
+        (*c)[few] = make_mixed(p.n, dbl, p.identity, p.load_colfast, p.store_colfast, few ? lines : 0, tail);
+    if (!(*c)[0].ok) throw std::runtime_error("transform length " + std::to_string(p.n) + " has no single-pass plan");
+    p.lines = 1 << (*c)[0].plan.log2t;
     p.mixed = c;
 }
 
@@ -584,7 +585,7 @@ const twiddles &fft_plan::get_twiddles(bool dbl, const pass &p, bool may_alloc) 
     if (p.mode == kModeR2C || p.mode == kModeC2R) { tail_count = n / 2; tail_mod = n; }
     if (p.mode >= kModeDCT2 && p.mode <= kModeDST3) { tail_count = n; tail_mod = 4LL * n; }
     if (p.mixed) {
-        const std::vector<unsigned char> v = mixed_table(p.mixed->plan, dbl, tail_mod);
+        const std::vector<unsigned char> v = mixed_table((*p.mixed)[0].plan, dbl, tail_mod);
         t.bytes = v.size();
         t.dev = upload_bytes(v.data(), t.bytes);
     } else if (dbl) {
@@ -763,10 +764,13 @@ void split_steps(const pass &p, const pass_args &base, bool dbl, int bt, void *t
 }
 
 namespace {
-void launch_mixed_pass(const pass &p, const pass_args &a, bool dbl, long long nblocks, hipStream_t s) {
-    mixed_plan g = p.mixed->plan;
+void launch_mixed_pass(const pass &p, const pass_args &a, bool dbl, hipStream_t s) {
+    const mixed_config *c = &(*p.mixed)[0];
+    if ((a.nlines >> c->plan.log2t) < kFewBlocks) c = &(*p.mixed)[1];
+    mixed_plan g = c->plan;
     mixed_launch_divs(g, a);
-    check_hip(launch_mixed(dbl, a, g, p.mixed->threads, nblocks, p.mixed->lds, s), "runtime-length FFT pass");
+    const long long nblocks = ((long long)a.nlines + (1 << g.log2t) - 1) >> g.log2t;
+    check_hip(launch_mixed(dbl, a, g, c->threads, nblocks, c->lds, s), "runtime-length FFT pass");
 }
 }  // namespace
 
@@ -780,7 +784,7 @@ void fft_plan::launch_split(const pass &p, const pass_args &base, bool dbl, int 
             st[i].tw = get_twiddles(dbl, q, false).dev;
             const long long nblocks = ((long long)st[i].nlines + q.lines - 1) / q.lines;
             if (q.fast) check_hip(q.fast->launch(st[i], nblocks, stream_), "split FFT pass");
-            else launch_mixed_pass(q, st[i], dbl, nblocks, stream_);
+            else launch_mixed_pass(q, st[i], dbl, stream_);
         }
     }
 }
@@ -881,7 +885,7 @@ void fft_plan::execute(int dir, bool dbl, bool in_real, bool out_real, int batch
         } else if (p.fast) {
             check_hip(p.fast->launch(a, nblocks, stream_), "fast FFT pass");
         } else {
-            launch_mixed_pass(p, a, dbl, nblocks, stream_);
+            launch_mixed_pass(p, a, dbl, stream_);
         }
         if (tprev) {
             const std::string name = pass_kernel_name(p, dbl, mfma, precision_, a);

@@ -69,7 +69,8 @@ struct pass {
     int mode = 0;           // kModeC2C, or kModeR2C / kModeC2R when the half-length kernel runs it
     // launch configuration
     const fast_kernel_info *fast = nullptr;
-    std::shared_ptr<const mixed_config> mixed;  // set: the runtime-length pass runs it
+    // set: the runtime-length pass runs it, with the second tile where a launch's lines are few
+    std::shared_ptr<const std::array<mixed_config, 2>> mixed;
     int lines = 1;  // lines (columns) per block
     // A length whose line does not fit one LDS tile runs as two passes (four-step), n = n1 n2,
     // position j = n2 j1 + j2, bin k = k1 + n1 k2: the first step takes the n1-point lines of
@@ -177,12 +178,12 @@ class fft_plan {
 };
 
 // Radix order of the runtime-length pass (empty: n has a prime factor above 13), and its tile for one
-// pass (copy: no transform, only the layout change; *_across: that side walks the column axis; ncol
-// columns, nlines lines in all; tail: real-data twiddles).  Device table: the later stages' entries,
+// pass (copy: no transform, only the layout change; *_across: that side walks the column axis; nlines:
+// lines of a launch with few of them, 0 for many; tail: real-data twiddles).  Device table: the later stages' entries,
 // the stage twiddles, w_{tail_mod}^k for k < tail, the chirp and its transform.
 std::vector<int> mixed_radices(int n, bool dbl);
-mixed_config make_mixed(int n, bool dbl, bool copy, bool load_across, bool store_across, long long ncol,
-                        long long nlines, int tail);
+mixed_config make_mixed(int n, bool dbl, bool copy, bool load_across, bool store_across, long long nlines,
+                        int tail);
 int mixed_post_offset(const std::vector<int> &radices);
 std::vector<unsigned char> mixed_table(const mixed_plan &g, bool dbl, long long tail_mod);
 // the divisors of one launch's line numbering

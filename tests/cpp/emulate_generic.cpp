@@ -60,7 +60,7 @@ template <typename R> int run_case(int n, int mode, int flags, int oi, int oo, i
     const sides si = layout_of(oi, nin, ncol, nb1), so = layout_of(oo, nout, ncol, nb1);
     const bool load_across = si.sa != 1 && nin > 1, store_across = so.sa != 1 && nout > 1;
     const int tail = (mode >= hmi::kModeDCT2 && mode <= hmi::kModeDST3) ? n : 0;
-    const hmi::mixed_config c = hmi::make_mixed(n, dbl, copy, load_across, store_across, ncol, (long long)ncol * nb1, tail);
+    const hmi::mixed_config c = hmi::make_mixed(n, dbl, copy, load_across, store_across, (flags & 1024) ? 0 : (long long)ncol * nb1, tail);
     what = "n=" + std::to_string(n) + (dbl ? " f64" : " f32") + " mode=" + std::to_string(mode) + " flags=" +
            std::to_string(flags) + " orders=" + std::to_string(oi) + std::to_string(oo) + " ncol=" + std::to_string(ncol) +
            " nb1=" + std::to_string(nb1) + " batch=" + std::to_string(batch);
@@ -179,6 +179,7 @@ int main(int argc, char **argv) {
     auto one = [&](bool dbl, int n, int mode, int flags, int oi, int oo, int ncol, int nb1, int batch) {
         if (at++ % shares != share) return;
         std::string what;
+        flags |= (at & 1) * 1024;  // both tiles of a plan
         const int bad = dbl ? run_case<double>(n, mode, flags, oi, oo, ncol, nb1, batch, at, what)
                             : run_case<float>(n, mode, flags, oi, oo, ncol, nb1, batch, at, what);
         cases++;

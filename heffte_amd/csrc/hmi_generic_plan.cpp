@@ -244,6 +244,43 @@ mixed_config make_mixed(int n, bool dbl, bool copy, bool load_across, bool store
     return c;
 }
 
+plane_config make_plane(int n0, int n1, long long nplanes, bool dbl) {
+    plane_config c{};
+    if (n0 < 2 || n1 < 2 || n0 > kPlaneMaxSide || n1 > kPlaneMaxSide) return c;
+    const long long elem = dbl ? 16 : 8, rp = n0 | 1, ps = rp * n1;
+    if (ps * elem > kPlaneBytes) return c;
+    const mixed_config c0 = make_mixed(n0, dbl, false, false, false, 0, 0), c1 = make_mixed(n1, dbl, false, false, false, 0, 0);
+    if (!c0.ok || !c1.ok) return c;
+    plane_args &a = c.args;
+    a.g0 = c0.plan;
+    a.g1 = c1.plan;
+    if (a.g0.chirp || a.g0.direct || a.g1.chirp || a.g1.direct) return c;
+    // planes per block: up to kPlaneTile bytes, as long as the launch keeps kFewBlocks blocks
+    int planes = 1;
+    while (2 * planes * ps * elem <= kPlaneTile && nplanes / (2 * planes) >= kFewBlocks) planes *= 2;
+    a.n0 = n0;
+    a.n1 = n1;
+    a.planes = planes;
+    a.rp = (int)rp;
+    a.ps = (int)ps;
+    a.rows = (unsigned)(planes * n1);
+    a.cols = (unsigned)(planes * n0);
+    a.by_rows = make_div(a.rows);
+    a.by_cols = make_div(a.cols);
+    a.by_n0 = make_div((unsigned)n0);
+    c.lds = (size_t)(planes * ps * elem);
+    // threads: about one round of the smallest stage, whole sets of four waves above 256
+    int top = 2;
+    for (const mixed_plan *g : {&a.g0, &a.g1})
+        for (int s = 0; s < g->nst; s++) top = std::max(top, g->radix[s]);
+    const long long units = (long long)planes * n0 * n1 / top;
+    c.threads = 64;
+    while (c.threads < 256 && c.threads < units) c.threads += 64;
+    if (units > 256 + 64) c.threads = kMixedThreads;
+    c.ok = true;
+    return c;
+}
+
 void mixed_launch_divs(mixed_plan &g, const pass_args &a) {
     g.by_ncol = make_div((unsigned)a.ncol);
     g.by_nb1 = make_div((unsigned)a.nb1);

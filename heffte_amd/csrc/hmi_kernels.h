@@ -35,6 +35,12 @@ const fast_kernel_info *find_fast_kernel(int n, bool dbl, bool wide);
 constexpr int kMixedThreads = 512;
 constexpr int kLightRadix = 10;
 constexpr long long kMixedTile = 16 * 1024;  // bytes a tile aims at
+// Fused two-axis pass: longest side (longer axes keep the compile-time and matrix-core passes), LDS
+// bytes of a plane and of a block's planes.  A plane that fills the LDS alone, one block per CU, still
+// beats two passes: complex<double> 16 x 100^3 286 -> 236 us, 90 x 100 x 108 32 -> 28 us, complex<float>
+// 4 x (120, 120, 64) 38 -> 30 us.
+constexpr int kPlaneMaxSide = 256;
+constexpr long long kPlaneBytes = kGenericMaxLds, kPlaneTile = 32 * 1024;
 // Launches of fewer blocks take smaller tiles on more CUs (r2c 20 x 14 x 12 float: 14.3 -> 13.1 us a
 // call, 60 x 60 x 40 pair 30.7 -> 28.0 us); many lines keep the full tile, which one transform's line
 // count used to cap also in a batch (one-dimensional lines: one line per block).
@@ -47,6 +53,10 @@ inline hipError_t launch_mixed(bool dbl, const pass_args &a, const mixed_plan &g
                                size_t lds_bytes, hipStream_t s) {
     return (dbl ? launch_mixed_f64 : launch_mixed_f32)(a, g, threads, nblocks, lds_bytes, s);
 }
+
+// Fused pass over the two fastest axes (hmi_plane.h).
+hipError_t launch_plane_f32(const plane_args &a, int threads, long long nblocks, size_t lds_bytes, hipStream_t s);
+hipError_t launch_plane_f64(const plane_args &a, int threads, long long nblocks, size_t lds_bytes, hipStream_t s);
 
 // Compile-time tile of the batched kernel for one length: lines per tile and LDS bytes
 // for each precision, and the complex-unit size of its stage twiddle table.

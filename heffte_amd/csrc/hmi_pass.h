@@ -130,6 +130,22 @@ struct mixed_stage {
 enum : int { kMixedHead = 192 };
 static_assert(sizeof(mixed_stage) * (kMixedStages - 1) <= kMixedHead, "the stages fit the table head");
 
+// Fused pass over the two fastest axes of a box (fft_plane): planes of n0 x n1 elements back to back,
+// `planes` of them per block, the same layout on both sides.
+struct plane_args {
+    const void *in;
+    void *out;
+    const void *mul;              // as pass_args::mul
+    const void *tw0, *tw1;        // runtime-length tables of n0 and n1
+    mixed_plan g0, g1;            // their radix plans (tile fields unused)
+    int n0, n1, nplanes, planes;
+    int rp, ps;                   // LDS strides of rows and planes (elements); rp is odd
+    unsigned rows, cols;          // planes n1, planes n0
+    fast_div by_rows, by_cols, by_n0;
+    int conj, stream;
+    double scale;
+};
+
 // Batched mixed-size transforms (one phase = one axis of every transform).
 // Every transform is a c2c box in order (0, 1, 2) at its own element offset.
 struct batch_xform {

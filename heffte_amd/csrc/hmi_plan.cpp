@@ -151,7 +151,9 @@ void fft_plan::prepare(bool dbl) {
     for_each_variant([&](int dir, bool ir, bool orl, bool ip) {
         const exec_plan &ep = get_exec_plan(dir, dbl, ir, orl, ip);
         for (const pass &p : ep.passes) {
-            if (p.split) {
+            if (p.plane) {
+                for (const mixed_plan *g : {&p.plane->args.g0, &p.plane->args.g1}) (void)get_plane_table(dbl, *g, true);
+            } else if (p.split) {
                 for (const pass &q : *p.split) (void)get_twiddles(dbl, q, true);
                 (void)get_split_table(dbl, p.n, true);
             } else {
@@ -363,6 +365,40 @@ exec_plan fft_plan::build(int dir, bool dbl, bool in_real, bool out_real, bool i
     } while (std::next_permutation(perm.begin(), perm.end()));
     if (!std::isfinite(best_cost)) throw std::runtime_error("no valid pass schedule for these boxes");
 
+    // The two fastest axes in one fused pass where a plane fits the LDS: same layout on both sides and
+    // plain complex data, so the passes are (fastest two: in -> out), (slowest: out, in place).
+    const int *o = bin.order;
+    if (!sizes_only && kind_ == kind::c2c && !in_real && !out_real && std::equal(o, o + 3, bout.order) && nin[o[0]] > 1 &&
+        nin[o[1]] > 1 && nin[o[0]] <= kPlaneMaxSide && nin[o[1]] <= kPlaneMaxSide) {
+        const plane_config c = make_plane((int)nin[o[0]], (int)nin[o[1]], nin[o[2]], dbl);
+        pass q;
+        q.axis = o[2];
+        q.col = o[0];
+        q.b1 = o[1];
+        q.n = q.store_len = (int)nin[o[2]];
+        q.src = buf::out;
+        q.lin = q.lout = Lout;
+        q.load_colfast = q.store_colfast = 1;
+        q.last = true;
+        // (a slowest axis with narrow column chunks is better off in the schedule above)
+        if (c.ok && narrow_chunk_cost(q, dbl) == 0.0) {
+            exec_plan ep;
+            pass p;
+            p.axis = o[0];
+            p.plane_axis = o[1];
+            p.col = o[1];
+            p.b1 = o[2];
+            p.n = p.store_len = (int)nin[o[0]];
+            p.lin = Lin;
+            p.lout = Lout;
+            p.last = nin[o[2]] == 1;
+            p.plane = std::make_shared<plane_config>(c);
+            ep.passes.push_back(p);
+            if (!p.last) ep.passes.push_back(q);
+            best = ep;
+        }
+    }
+
     for (pass &p : best.passes) configure(p, dbl, sizes_only);
     // the step buffer of split axes follows the intermediate arrays in the workspace
     long long split_elems = 0;
@@ -376,6 +412,7 @@ exec_plan fft_plan::build(int dir, bool dbl, bool in_real, bool out_real, bool i
 }
 
 void fft_plan::configure(pass &p, bool dbl, bool sizes_only) const {
+    if (p.plane) return;
     const size_t elem = dbl ? 16 : 8;
     const bool wide = p.load_colfast || p.store_colfast;
     if (p.mode >= kModeDCT2) {
@@ -552,7 +589,9 @@ namespace {
 std::string pass_kernel_name(const pass &p, bool dbl, bool mfma, int precision, const pass_args &a) {
     const char *R = dbl ? "double" : "float";
     std::string s;
-    if (p.split) {
+    if (p.plane) {
+        s = std::string("fft_plane<") + R + "> " + std::to_string(p.plane->args.n0) + " x " + std::to_string(p.plane->args.n1);
+    } else if (p.split) {
         s = std::string("split ") + R + " " + std::to_string(p.split_n1) + " x " + std::to_string(p.split_n2) +
             " (two launches per transform)";
     } else if (mfma) {
@@ -597,6 +636,20 @@ const twiddles &fft_plan::get_twiddles(bool dbl, const pass &p, bool may_alloc) 
         t.bytes = v.size() * sizeof(float);
         t.dev = upload_bytes(v.data(), t.bytes);
     }
+    return tw_.emplace(key, t).first->second;
+}
+
+const twiddles &fft_plan::get_plane_table(bool dbl, const mixed_plan &g, bool may_alloc) {
+    // (bit 57: the runtime-length table of a length that may have a compile-time tile as well)
+    const long long key = ((long long)g.n << 8) | (dbl ? 1 : 0) | (1LL << 57);
+    std::lock_guard<std::mutex> lock(mtx_);
+    auto it = tw_.find(key);
+    if (it != tw_.end()) return it->second;
+    if (!may_alloc) throw std::runtime_error(kNotResident);
+    const std::vector<unsigned char> v = mixed_table(g, dbl, 1);
+    twiddles t;
+    t.bytes = v.size();
+    t.dev = upload_bytes(v.data(), t.bytes);
     return tw_.emplace(key, t).first->second;
 }
 
@@ -774,6 +827,24 @@ void launch_mixed_pass(const pass &p, const pass_args &a, bool dbl, hipStream_t 
 }
 }  // namespace
 
+void fft_plan::launch_plane(const pass &p, const pass_args &base, bool dbl, int batch) {
+    const plane_config &c = *p.plane;
+    plane_args a = c.args;
+    a.in = base.in;
+    a.out = base.out;
+    a.mul = base.mul;
+    a.tw0 = get_plane_table(dbl, a.g0, false).dev;
+    a.tw1 = get_plane_table(dbl, a.g1, false).dev;
+    const long long nplanes = p.lin.n[p.b1] * batch;
+    if (nplanes > 0x7fffffffLL) throw std::runtime_error("too many planes in one pass");
+    a.nplanes = (int)nplanes;
+    a.conj = base.conj;
+    a.stream = base.stream;
+    a.scale = base.scale;
+    const long long nblocks = (nplanes + a.planes - 1) / a.planes;
+    check_hip((dbl ? launch_plane_f64 : launch_plane_f32)(a, c.threads, nblocks, c.lds, stream_), "fused two-axis FFT pass");
+}
+
 void fft_plan::launch_split(const pass &p, const pass_args &base, bool dbl, int batch, void *tmp) {
     for (int bt = 0; bt < batch; bt++) {
         pass_args st[2];
@@ -820,7 +891,11 @@ void fft_plan::execute(int dir, bool dbl, bool in_real, bool out_real, int batch
         const pass &p = ep.passes[i];
         const bool mfma = split && p.n == 512 && p.mode == kModeC2C && !p.identity && !p.in_real && !p.out_real &&
                           !p.herm_load && p.store_len == p.n && !(mul && i == 0);
-        if (p.split) {
+        if (p.plane) {
+            // both axes' tables (launch_plane uses them)
+            for (const mixed_plan *g : {&p.plane->args.g0, &p.plane->args.g1})
+                tables[i] = get_plane_table(dbl, *g, may_alloc).dev;
+        } else if (p.split) {
             // both steps' tables and the step twiddles, looked up now (launch_split uses them)
             for (const pass &q : *p.split) (void)get_twiddles(dbl, q, may_alloc);
             tables[i] = get_split_table(dbl, p.n, may_alloc).dev;
@@ -848,7 +923,7 @@ void fft_plan::execute(int dir, bool dbl, bool in_real, bool out_real, int batch
     };
     const bool debug = std::getenv("HMI_DEBUG_PLAN") != nullptr;
     // per-pass timing: one event before the first pass and one after each pass
-    std::unique_lock<std::mutex> tlock(mtx_, std::defer_lock);
+    std::unique_lock<std::mutex> tlock(timing_mtx_, std::defer_lock);
     hipEvent_t tprev = nullptr;
     if (timing_) {
         tlock.lock();
@@ -874,7 +949,9 @@ void fft_plan::execute(int dir, bool dbl, bool in_real, bool out_real, int batch
         const long long nblocks = ((long long)a.nlines + p.lines - 1) / p.lines;
         const bool mfma = split && p.n == 512 && p.mode == kModeC2C && !p.identity && !p.in_real && !p.out_real &&
                           !p.herm_load && p.store_len == p.n && !a.mul;
-        if (p.split) {
+        if (p.plane) {
+            launch_plane(p, a, dbl, batch);
+        } else if (p.split) {
             launch_split(p, a, dbl, batch, static_cast<char *>(ws) + (size_t)batch * p.split_ws * (dbl ? 16 : 8));
         } else if (mfma) {
             // the split-precision form: a.tw holds W512 and the split W32 / W16 operand tables
@@ -924,13 +1001,13 @@ void fft_plan::clear_timing() {
 }
 
 void fft_plan::set_timing(bool on) {
-    std::lock_guard<std::mutex> lock(mtx_);
+    std::lock_guard<std::mutex> lock(timing_mtx_);
     clear_timing();
     timing_ = on;
 }
 
 std::string fft_plan::timing_report() {
-    std::lock_guard<std::mutex> lock(mtx_);
+    std::lock_guard<std::mutex> lock(timing_mtx_);
     std::vector<long long> count(timing_names_.size(), 0);
     std::vector<double> total(timing_names_.size(), 0.0);
     for (const auto &rec : timing_launches_) {

@@ -56,6 +56,14 @@ struct mixed_config {
     size_t lds = 0;
 };
 
+// Tile and block of the fused pass over the two fastest axes.
+struct plane_config {
+    bool ok = false;
+    plane_args args{};  // radix plans, extents and strides; pointers and counts are set at the launch
+    int threads = 64;
+    size_t lds = 0;
+};
+
 struct pass {
     int axis = 0, n = 1;
     buf src = buf::in, dst = buf::out;
@@ -72,6 +80,9 @@ struct pass {
     // set: the runtime-length pass runs it, with the second tile where a launch's lines are few
     std::shared_ptr<const std::array<mixed_config, 2>> mixed;
     int lines = 1;  // lines (columns) per block
+    // set: axis and plane_axis (the two fastest axes of lin = lout) run as one fused pass
+    std::shared_ptr<const plane_config> plane;
+    int plane_axis = -1;
     // A length whose line does not fit one LDS tile runs as two passes (four-step), n = n1 n2,
     // position j = n2 j1 + j2, bin k = k1 + n1 k2: the first step takes the n1-point lines of
     // stride n2 (one per j2) into a buffer of the pass's input layout at position n2 k1 + j2,
@@ -154,7 +165,9 @@ class fft_plan {
     exec_plan build(int dir, bool dbl, bool in_real, bool out_real, bool in_place, bool sizes_only = false) const;
     void configure(pass &p, bool dbl, bool sizes_only = false) const;
     const twiddles &get_twiddles(bool dbl, const pass &p, bool may_alloc);
+    const twiddles &get_plane_table(bool dbl, const mixed_plan &g, bool may_alloc);
     const twiddles &get_split_table(bool dbl, int n, bool may_alloc);
+    void launch_plane(const pass &p, const pass_args &base, bool dbl, int batch);
     void launch_split(const pass &p, const pass_args &base, bool dbl, int batch, void *tmp);
     const twiddles &get_mfma_table(int prec, bool conj, bool may_alloc);
     template <typename F> void for_each_variant(F &&f) const;
@@ -170,6 +183,8 @@ class fft_plan {
     std::map<int, exec_plan> plans_;
     std::map<long long, twiddles> tw_;
     // per-pass timing records: launch i ran between events marks_[i].first and .second
+    // (a lock of their own: a timed call looks up tables while it records)
+    std::mutex timing_mtx_;
     bool timing_ = false;
     std::vector<std::string> timing_names_;
     std::vector<std::pair<int, std::pair<hipEvent_t, hipEvent_t>>> timing_launches_;
@@ -186,6 +201,9 @@ mixed_config make_mixed(int n, bool dbl, bool copy, bool load_across, bool store
                         int tail);
 int mixed_post_offset(const std::vector<int> &radices);
 std::vector<unsigned char> mixed_table(const mixed_plan &g, bool dbl, long long tail_mod);
+// Fused pass over planes of n0 x n1 elements (ok false: it does not take them), nplanes of them in one
+// transform.
+plane_config make_plane(int n0, int n1, long long nplanes, bool dbl);
 // the divisors of one launch's line numbering
 void mixed_launch_divs(mixed_plan &g, const pass_args &a);
 

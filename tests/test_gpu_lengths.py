@@ -62,3 +62,28 @@ def test_r2c_and_r2r_lengths(hmi, cuda, oracle, dtype, n):
             assert fc.rel_l2(fc.to_host(tr), fn(b, b, x, -1)) <= fc.TOL[dtype], (kind, size)
             rplan.backward(tr, tz, hmi.scale.full)
             assert fc.rel_l2(fc.to_host(tz), x) <= fc.TOL[dtype], (kind, size)
+
+
+@pytest.mark.parametrize("dtype", ["complex64", "complex128"])
+@pytest.mark.parametrize("size", [(2, 3, 1), (16, 16, 16), (7, 12, 5), (32, 30, 3), (81, 64, 2), (20, 256, 3), (100, 45, 7),
+                                  (3, 4, 900), (64, 1, 9), (98, 102, 4), (256, 19, 6)])
+def test_fused_planes(hmi, cuda, oracle, dtype, size):
+    """Boxes with one layout on both sides run their two fastest axes in one pass where a plane fits the
+    LDS: every order, in and out of place, a batch, both directions and the fused product."""
+    import torch
+    n = int(np.prod(size))
+    x = fc.uniform_complex(2 * n, n % 97)
+    for order in [(0, 1, 2), (2, 0, 1), (1, 0, 2)]:
+        box = hmi.box3d([0, 0, 0], [s - 1 for s in size], order)
+        plan = hmi.fft3d(hmi.backend.mi355, box, box)
+        b = oracle.Box.make((0, 0, 0), [s - 1 for s in size], order)
+        ref = oracle.fft3d_c2c(b, b, x, -1, 1.0, 2)
+        tx = fc.to_gpu(x, np.complex64 if dtype == "complex64" else np.complex128)
+        ty = torch.empty_like(tx)
+        plan.forward(tx, ty, hmi.scale.none, 2)
+        assert fc.rel_l2(fc.to_host(ty), ref) <= fc.TOL[dtype], order
+        plan.backward(ty, ty, hmi.scale.full, 2)
+        assert fc.rel_l2(fc.to_host(ty), x) <= fc.TOL[dtype], order
+        tz = torch.empty_like(tx)
+        plan.convolve(tx, ty, tz, None, hmi.scale.full, 2)
+        assert fc.rel_l2(fc.to_host(tz), oracle.convolve3d(b, b, x, x, 1.0 / n, 2)) <= 2 * fc.TOL[dtype], order

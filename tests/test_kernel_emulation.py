@@ -3,7 +3,8 @@
 The runtime-length pass takes every length without a compile-time tile in every form (complex, real
 sides, Hermitian load, partial store, fused product, split-axis twiddle, cosine and sine modes); its
 index arithmetic, radix plans and LDS layouts are checked against direct transforms for all orders
-of both sides, with arrays and LDS that end where the pass may last touch them.
+of both sides, with arrays and LDS that end where the pass may last touch them.  The fused two-axis
+pass likewise over many plane shapes.
 """
 import os
 import shutil
@@ -28,8 +29,9 @@ def build(tmp_path_factory, name, sources):
 
 
 @pytest.mark.skipif(CLANG is None, reason="clang++ not found")
-def test_runtime_length_pass(tmp_path_factory):
-    exe = build(tmp_path_factory, "emulate_generic", ["hmi_generic_plan.cpp"])
+@pytest.mark.parametrize("name", ["emulate_generic", "emulate_plane"])
+def test_kernel(tmp_path_factory, name):
+    exe = build(tmp_path_factory, name, ["hmi_generic_plan.cpp"])
     runs = [subprocess.Popen([exe, str(i), str(SHARES)], stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
             for i in range(SHARES)]
     for p in runs:

@@ -95,7 +95,11 @@ batch_plan::~batch_plan() {
         for (auto &ax : d.rest)
             for (auto *p : ax) (void)hipFree(p);
         for (auto *p : d.xy) (void)hipFree(p);
-        for (auto *p : d.zc) (void)hipFree(p);
+        (void)hipFree(d.zc);
+        (void)hipFree(d.fused);
+        (void)hipFree(d.mplans);
+        (void)hipFree(d.mtab);
+        (void)hipFree(d.mtoff);
         for (auto *p : d.zrest) (void)hipFree(p);
         (void)hipFree(d.plans);
         (void)hipFree(d.twoff);
@@ -144,86 +148,85 @@ void batch_plan::prepare(bool dbl) {
         plans.push_back(g);
         kids.push_back(kid);
     }
-    // Fused x-y phase: a transform whose x and y lengths both have compile-time tiles of register
-    // classes up to kXyMaxClass takes the 256-thread build when one plane fits its budget, else
-    // the 512-thread build when a plane fits that one; work item = as many consecutive z-planes
-    // as the budget holds (at least one).
+    // Fused phases (fft_batch_fused), for lengths with a runtime-length radix plan without prime factors
+    // above 13.  x-y: a padded plane fits the LDS; item = as many consecutive z-planes as fit the
+    // smallest block size that holds one.  z: item = as many consecutive (x, y) positions as fit the
+    // smallest block.  (nfused: the transforms of the sizes that fused_count() states.)
     const int pr = dbl ? 1 : 0;
     std::vector<int> xy_build(xf_.size(), -1);
+    std::vector<bool> zcol(xf_.size(), false);
     {
-        std::vector<batch_item> xy[kBatchClasses + 1];
-        long long held[kBatchClasses + 1] = {};
+        // radix plans and tables (no plan: one point, or a prime factor above 13)
+        std::vector<mixed_plan> mplans;
+        std::vector<unsigned char> mtab;
+        std::vector<int> mtoff;
+        for (size_t l = 0; l < lengths_.size(); l++) {
+            mixed_plan g{};
+            mtoff.push_back((int)mtab.size());
+            const int n = lengths_[l];
+            if (n > 1 && 2 * (size_t)n * elem <= (size_t)kGenericMaxLds)
+                g = make_mixed(n, dbl, false, false, false, 0, 0).plan;
+            if (g.chirp || g.direct) g = mixed_plan{};
+            if (g.n > 1) {
+                const std::vector<unsigned char> t = mixed_table(g, dbl, 1);
+                mtab.insert(mtab.end(), t.begin(), t.end());
+            }
+            mplans.push_back(g);
+        }
+        std::vector<batch_fused> fused(xf_.size());
+        std::vector<batch_item> xy[kFusedSizes], zc;
+        std::vector<long long> xy_elems(xf_.size(), 0), zc_elems(xf_.size(), 0);
+        d.nfused = 0;
         for (int i = 0; i < (int)xf_.size(); i++) {
             const batch_xform &x = xf_[i];
             const int k0 = kids[x.size_id[0]], k1 = kids[x.size_id[1]];
-            if (!batch_xy_supported(k0) || !batch_xy_supported(k1)) continue;
-            const int cls = std::max(batch_kernel_class(k0), batch_kernel_class(k1));
             const long long plane = (long long)xy_row_stride(x.n[0]) * x.n[1];  // LDS elements
-            int b = -1;
-            // the 256-thread build is one build carrying every tile (kXyMaxClass): one launch for
-            // the items of all classes (at 2 waves per SIMD and two blocks per CU the larger
-            // register budget costs nothing; separate launches per class added their tails)
-            if (cls <= kXyMaxClass[pr] && plane <= kXySmallBudget[pr]) b = kXyMaxClass[pr];
-            else if (cls <= kXyLargeMaxClass[pr] && plane <= kXyLargeBudget[pr]) b = kBatchClasses;
-            if (b < 0) continue;
-            xy_build[i] = b;
-            const long long budget = b == kBatchClasses ? kXyLargeBudget[pr] : kXySmallBudget[pr];
-            const long long g = std::max(1LL, budget / plane);
-            for (long long t = 0; t * g < x.n[2]; t++) xy[b].push_back({i, (int)t});
-            held[b] = std::max(held[b], std::min<long long>(g, x.n[2]) * plane);
+            batch_fused &f = fused[i];
+            if (mplans[x.size_id[0]].n > 1 && mplans[x.size_id[1]].n > 1 && plane * (long long)elem <= kGenericMaxLds) {
+                int b = 0;
+                while (plane * (long long)elem > kFusedLds[b]) b++;
+                f.planes = (int)std::min<long long>(x.n[2], kFusedLds[b] / (plane * (long long)elem));
+                f.by_rows = make_fast_div((unsigned)(f.planes * x.n[1]));
+                f.by_cols = make_fast_div((unsigned)(f.planes * x.n[0]));
+                f.by_n0 = make_fast_div((unsigned)x.n[0]);
+                xy_build[i] = b;
+                xy_elems[i] = f.planes * plane;
+                d.xy_lds[b] = std::max(d.xy_lds[b], (size_t)xy_elems[i] * elem);
+                for (long long t = 0; t * f.planes < x.n[2]; t++) xy[b].push_back({i, (int)t});
+            }
+            // the count the interface reports
+            if (k0 >= 0 && k1 >= 0) {
+                const int cls = std::max(batch_kernel_class(k0), batch_kernel_class(k1));
+                if ((cls <= kXyMaxClass[pr] && plane <= kXyBudget[pr]) || plane <= kXyLargeBudget[pr]) d.nfused++;
+            }
+            const long long cols = (long long)x.n[0] * x.n[1];
+            if (mplans[x.size_id[2]].n > 1 && (long long)elem * x.n[2] <= kFusedLds[0] && cols <= 0x7fffffffLL / 2) {
+                f.width = (int)std::min<long long>(cols, kFusedLds[0] / ((long long)elem * x.n[2]));
+                f.by_width = make_fast_div((unsigned)f.width);
+                zcol[i] = true;
+                zc_elems[i] = (long long)f.width * x.n[2];
+                d.zc_lds = std::max(d.zc_lds, (size_t)zc_elems[i] * elem);
+                for (long long t = 0; t * f.width < cols; t++) zc.push_back({i, (int)t});
+            }
         }
-        d.nfused = 0;
-        for (int b : xy_build) d.nfused += b >= 0 ? 1 : 0;
-        // largest items first (the blocks take them in list order, so the launch ends on small
-        // ones: 3.925 -> 3.910 ms per pair on the 1000-transform batch)
-        for (int b = 0; b <= kBatchClasses; b++) {
-            const long long budget = b == kBatchClasses ? kXyLargeBudget[pr] : kXySmallBudget[pr];
-            auto elems = [&](const batch_item &it) {
-                const batch_xform &x = xf_[it.xform];
-                const long long plane = (long long)x.n[0] * x.n[1];
-                const long long g = std::max(1LL, budget / ((long long)xy_row_stride(x.n[0]) * x.n[1]));
-                return std::min<long long>(g, x.n[2] - (long long)it.tile * g) * plane;
-            };
-            std::stable_sort(xy[b].begin(), xy[b].end(),
-                             [&](const batch_item &a, const batch_item &c) { return elems(a) > elems(c); });
-            if (xy[b].size() > 0x7fffffffULL) throw std::runtime_error("batch work list too long");
+        // largest items first (the blocks take them in list order, so a launch ends on small ones)
+        auto by_size = [](std::vector<batch_item> &v, const std::vector<long long> &e) {
+            std::stable_sort(v.begin(), v.end(),
+                             [&](const batch_item &a, const batch_item &b) { return e[a.xform] > e[b.xform]; });
+            if (v.size() > 0x7fffffffULL) throw std::runtime_error("batch work list too long");
+        };
+        for (int b = 0; b < kFusedSizes; b++) {
+            by_size(xy[b], xy_elems);
             d.nxy[b] = (int)xy[b].size();
             d.xy[b] = xy[b].empty() ? nullptr : upload(xy[b]);
-            d.xy_budget[b] = b == kBatchClasses ? kXyLargeBudget[pr] : kXySmallBudget[pr];
-            d.xy_lds[b] = (size_t)held[b] * elem;
         }
-    }
-    // Column-block z phase: a transform whose z length has a compile-time tile of a class the
-    // 256-thread builds run; work item = zcol_width(n2, budget, n0 n1) consecutive (x, y)
-    // positions.  The others keep the tiled z phase.
-    std::vector<bool> zcol(xf_.size(), false);
-    {
-        std::vector<batch_item> zc[kBatchClasses];
-        for (int i = 0; i < (int)xf_.size(); i++) {
-            const batch_xform &x = xf_[i];
-            const int kz = kids[x.size_id[2]];
-            if (!batch_xy_supported(kz)) continue;
-            const int cls = batch_kernel_class(kz);
-            if (cls > kXyMaxClass[pr] || (long long)x.n[2] > kXySmallBudget[pr]) continue;
-            const long long plane = (long long)x.n[0] * x.n[1];
-            if (plane > 0x7fffffffLL / 2) continue;
-            const long long w = zcol_width(x.n[2], kXySmallBudget[pr], (int)plane);
-            zcol[i] = true;
-            for (long long t = 0; t * w < plane; t++) zc[kXyMaxClass[pr]].push_back({i, (int)t});
-        }
-        for (int c = 0; c < kBatchClasses; c++) {
-            auto elems = [&](const batch_item &it) {
-                const batch_xform &x = xf_[it.xform];
-                const long long plane = (long long)x.n[0] * x.n[1];
-                const long long w = zcol_width(x.n[2], kXySmallBudget[pr], (int)plane);
-                return std::min<long long>(w, plane - (long long)it.tile * w) * x.n[2];
-            };
-            std::stable_sort(zc[c].begin(), zc[c].end(),
-                             [&](const batch_item &a, const batch_item &b) { return elems(a) > elems(b); });
-            if (zc[c].size() > 0x7fffffffULL) throw std::runtime_error("batch work list too long");
-            d.nzc[c] = (int)zc[c].size();
-            d.zc[c] = zc[c].empty() ? nullptr : upload(zc[c]);
-        }
+        by_size(zc, zc_elems);
+        d.nzc = (int)zc.size();
+        d.zc = zc.empty() ? nullptr : upload(zc);
+        d.fused = upload(fused);
+        d.mplans = upload(mplans);
+        d.mtab = upload(mtab);
+        d.mtoff = upload(mtoff);
     }
     // work lists: every tile of every transform, one list per axis and register class; for the
     // x and y axes also the lists without the transforms of the fused phase, for z the list
@@ -275,42 +278,33 @@ void batch_plan::launch_phases(int dir, bool dbl, const void *in, void *out, int
     b.twoff = d.twoff;
     b.kid = d.kid;
     b.conj = dir > 0 ? 1 : 0;
+    b.fused = d.fused;
+    b.mplans = d.mplans;
+    b.mtab = d.mtab;
+    b.mtoff = d.mtoff;
     // at most 2^32 - 1 work-items in a grid: beyond that the grid stride covers the rest
-    const int max_blocks = (int)(0xffffffffLL / kXyLargeThreads);
-    const bool fused = fused_ && d.nfused > 0;
+    const int max_blocks = (int)(0xffffffffLL / kMixedThreads);
+    const bool fused = fused_;
+    auto launch_fused = [&](bool xy, const batch_item *items, int nitems, int size, size_t lds) {
+        if (nitems == 0) return;
+        b.items = items;
+        b.nitems = nitems;
+        check_hip((dbl ? launch_batch_fused_f64 : launch_batch_fused_f32)(xy, b, kFusedThreads[size],
+                                                                          std::min(nitems, max_blocks), lds, s),
+                  "batched fused phase");
+    };
     if (fused) {
-        // fused x-y phase: reads the input arrays, writes the output arrays
-        b.axis = 0;
+        // reads the input arrays, writes the output arrays; the largest blocks first
         b.from_in = 1;
         b.scaling = 0;
-        for (int k = 0; k <= kBatchClasses; k++) {
-            b.items = d.xy[k];
-            b.nitems = d.nxy[k];
-            b.xy_budget = d.xy_budget[k];
-            const int nblocks = std::min(b.nitems, max_blocks);
-            if (nblocks > 0)
-                check_hip(launch_batched_xy(dbl, k == kBatchClasses, k == kBatchClasses ? kXyLargeMaxClass[0] : k, b,
-                                            nblocks, d.xy_lds[k], s),
-                          "batched fused x-y phase");
-        }
+        for (int k = kFusedSizes - 1; k >= 0; k--) launch_fused(true, d.xy[k], d.nxy[k], k, d.xy_lds[k]);
     }
     for (int ax = 0; ax < 3; ax++) {
         b.axis = ax;
         b.from_in = (ax == 0) ? 1 : 0;
         b.scaling = (ax == 2) ? scaling : 0;
-        if (fused && ax == 2) {
-            // column-block z phase: reads and writes the output arrays, applies the scale
-            b.xy_budget = kXySmallBudget[dbl ? 1 : 0];
-            for (int c = 0; c < kBatchClasses; c++) {
-                b.items = d.zc[c];
-                b.nitems = d.nzc[c];
-                const int nblocks = std::min(b.nitems, max_blocks);
-                if (nblocks > 0)
-                    check_hip(launch_batched_zcol(dbl, c, b, nblocks, (size_t)b.xy_budget * (dbl ? 16 : 8), s),
-                              "batched column-block z phase");
-            }
-        }
-        b.xy_budget = 0;
+        // reads and writes the output arrays, applies the scale
+        if (fused && ax == 2) launch_fused(false, d.zc, d.nzc, 0, d.zc_lds);
         for (int c = 0; c < kBatchClasses; c++) {
             const bool rest = fused;
             b.items = !rest ? d.items[ax][c] : (ax < 2 ? d.rest[ax][c] : d.zrest[c]);
@@ -476,6 +470,7 @@ double batch_tuner::time_choice(int n, bool dbl, const batch_choice &c) {
     batch_plan probe(1, sizes, nullptr, nullptr);
     probe.set_graph(false);
     probe.set_autotune(false);
+    probe.set_fused(false);  // the choice is of the separate phases' tile
     probe.forced_[n] = c;
     const size_t bytes = (size_t)n * n2 * m * (dbl ? 16 : 8);
     void *buf = nullptr;

@@ -51,8 +51,8 @@ class batch_plan {
     void set_autotune(bool on) { autotune_ = on; }
     // off: every transform takes the separate x and y phases (the fused x-y phase is on by default)
     void set_fused(bool on) { fused_ = on; }
-    // transforms the fused x-y phase takes (the work lists are built on the first execute of each
-    // precision; -1 before that)
+    // transforms of compile-time tile lengths and sizes that the fused x-y phase takes (kXyBudget; the
+    // work lists are built on the first execute of each precision; -1 before that)
     int fused_count(bool dbl) const { return dev_[dbl ? 1 : 0].ready ? dev_[dbl ? 1 : 0].nfused : -1; }
     int count() const { return (int)xf_.size(); }
     long long input_elems() const { return in_extent_; }
@@ -75,16 +75,18 @@ class batch_plan {
         // the x and y work lists restricted to the transforms the fused phase does not take
         batch_item *rest[2][kBatchClasses] = {};
         int nrest[2][kBatchClasses] = {};
-        // fused x-y work lists: one per small build (register class), the last for the
-        // 1024-thread build; planes per work item set by xy_budget, LDS bytes per block
-        batch_item *xy[kBatchClasses + 1] = {};
-        int nxy[kBatchClasses + 1] = {};
-        int xy_budget[kBatchClasses + 1] = {};
-        size_t xy_lds[kBatchClasses + 1] = {};
-        // column-block z phase: one list per register class (xy_budget = kXySmallBudget), and the
-        // z work list of the transforms it does not take
-        batch_item *zc[kBatchClasses] = {};
-        int nzc[kBatchClasses] = {};
+        // fused x-y and column-block z work lists, one per block size (kFusedLds), and what they need:
+        // one entry per transform, runtime-length plans and tables per length
+        batch_item *xy[kFusedSizes] = {};
+        int nxy[kFusedSizes] = {};
+        batch_item *zc = nullptr;
+        int nzc = 0;
+        size_t xy_lds[kFusedSizes] = {}, zc_lds = 0;
+        batch_fused *fused = nullptr;
+        mixed_plan *mplans = nullptr;
+        unsigned char *mtab = nullptr;
+        int *mtoff = nullptr;
+        // the z work list of the transforms the column-block phase does not take
         batch_item *zrest[kBatchClasses] = {};
         int nzrest[kBatchClasses] = {};
         int nfused = 0;

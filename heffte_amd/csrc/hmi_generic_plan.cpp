@@ -281,6 +281,8 @@ plane_config make_plane(int n0, int n1, long long nplanes, bool dbl) {
     return c;
 }
 
+fast_div make_fast_div(unsigned d) { return make_div(d); }
+
 void mixed_launch_divs(mixed_plan &g, const pass_args &a) {
     g.by_ncol = make_div((unsigned)a.ncol);
     g.by_nb1 = make_div((unsigned)a.nb1);

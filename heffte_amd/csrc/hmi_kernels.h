@@ -81,33 +81,19 @@ const char *kernels_build_stamp();
 // work items of one register class.
 hipError_t launch_batched(bool dbl, int cls, const batch_args &b, int nblocks, size_t lds_bytes, hipStream_t s);
 
-// Fused x-y phase of a batch: each work item loads whole x-y planes (contiguous) of one
-// transform into LDS (n1 rows of xy_row_stride(n0) elements per plane), runs the x-axis and
-// y-axis FFTs there and stores the planes back, so the x and y axes cost one read and one write
-// of the array instead of two each.  Transforms whose x and y lengths both have compile-time
-// tiles (batch_xy_supported) of a register class up to kXyMaxClass take it.  Builds: 256 threads
-// with planes of at most kXySmallBudget elements (one build, cls = kXyMaxClass, carrying every
-// tile of the classes up to it), and for complex<float> 512 threads with planes up to
-// kXyLargeBudget elements (tiles of the classes up to kXyLargeMaxClass; -1: no such build).
-constexpr int kXySmallThreads = 256, kXyLargeThreads = 512;
-constexpr int kXySmallBudget[2] = {10240, 5120};   // elements: 80 KiB of LDS (complex<float>, <double>)
-constexpr int kXyLargeBudget[2] = {20480, 0};      // elements: 160 KiB of LDS
-constexpr int kXyMaxClass[2] = {2, 0};             // register classes of the 256-thread build
-constexpr int kXyLargeMaxClass[2] = {2, -1};       // register classes the 512-thread build runs
-// Row stride (elements) of an x-y plane of rows of n0 elements in the LDS of the fused phase: odd,
-// so that 32 lanes reading one position of 32 consecutive rows hit distinct banks.
+// Fused phases of a batch (fft_batch_fused, hmi_plane.h): the x-y phase for planes that fit the LDS, the
+// column-block z phase.  Work items of three sizes, each with its own launch: kFusedLds[k] bytes of LDS
+// and kFusedThreads[k] threads per block.  The rest: the sizes heffte_mi355_batch_fused_count counts
+// (register classes and padded plane elements by precision).
+constexpr int kXyBudget[2] = {10240, 5120};
+constexpr int kXyLargeBudget[2] = {20480, 0};
+constexpr int kXyMaxClass[2] = {2, 0};
+constexpr int kFusedSizes = 3;
+constexpr int kFusedLds[kFusedSizes] = {40 * 1024, 80 * 1024, kGenericMaxLds};
+constexpr int kFusedThreads[kFusedSizes] = {256, 512, 512};
 constexpr int xy_row_stride(int n0) { return n0 | 1; }
-bool batch_xy_supported(int kid);
-hipError_t launch_batched_xy(bool dbl, bool large, int cls, const batch_args &b, int nblocks, size_t lds_bytes,
-                             hipStream_t s);
-
-// Column-block z phase of a batch (256 threads, one build: cls = kXyMaxClass, carrying every
-// tile up to it): items (transform, block of zcol_width(n2, budget, n0 n1) consecutive (x, y)
-// positions); b.xy_budget = LDS elements per item.
-constexpr int zcol_width(int n2, int budget, int plane) {
-    return budget / n2 < 1 ? 1 : (budget / n2 < plane ? budget / n2 : plane);
-}
-hipError_t launch_batched_zcol(bool dbl, int cls, const batch_args &b, int nblocks, size_t lds_bytes, hipStream_t s);
+hipError_t launch_batch_fused_f32(bool xy, const batch_args &b, int threads, int nblocks, size_t lds_bytes, hipStream_t s);
+hipError_t launch_batch_fused_f64(bool xy, const batch_args &b, int threads, int nblocks, size_t lds_bytes, hipStream_t s);
 
 // Precision forms of the c2c passes: plain FP32/FP64 vector ALU, or the 512-point
 // complex<float> pass on the matrix cores with split-precision operands.

@@ -800,425 +800,6 @@ hipError_t launch_batched(bool dbl, int cls, const batch_args &b, int nblocks, s
     return hipGetLastError();
 }
 
-// ------------------------------------------------------ batched, fused x-y
-
-// Where the column FFTs of the fused phases store their results: column c of block p of the
-// lines at dst + p plane + c, its rows row elements apart; each value becomes (x sc, sg y sc).
-template <typename C, typename R> struct col_store {
-    C *dst;
-    int row;
-    long long plane;
-    R sg, sc;
-    __device__ __forceinline__ C value(C v) const { return cmk<C>(v.x * sc, sg * v.y * sc); }
-};
-
-// Stockham stages of one n-point line held in LDS at lb[j * es], E elements per thread (P = n / E
-// threads per line); each exchange goes through the line's own slots.  Every thread of the block
-// calls it (the barriers are block-wide); threads without a line (valid = false) only take part
-// in the barriers.
-template <int S, typename RL, int E, int P, typename C>
-__device__ __forceinline__ void lds_line_stages(C (&v)[E], C *lb, int es, const C *__restrict__ tw, int t,
-                                                bool valid) {
-    constexpr int R = RL::at(S);
-    constexpr int Ls = RL::ls(S);
-    constexpr int NB = E / R;
-    constexpr bool last = (S + 1 == RL::count);
-    constexpr int TWO = RL::twoff(S);
-    static_assert(E % R == 0, "every radix must divide the elements per thread");
-#pragma unroll
-    for (int r = 0; r < NB; r++) {
-        const int b = t + P * r;
-        const int k = b % Ls;
-        C x[R];
-#pragma unroll
-        for (int p = 0; p < R; p++) x[p] = v[r + NB * p];
-        if constexpr (Ls > 1) {
-            const C *w = tw + TWO + k * (R - 1);
-#pragma unroll
-            for (int p = 1; p < R; p++) x[p] = cmul(x[p], w[p - 1]);
-        }
-        dft<R>::run(x);
-        if constexpr (last) {
-#pragma unroll
-            for (int q = 0; q < R; q++) v[r + NB * q] = x[q];
-        } else if (valid) {
-            const int base = (b / Ls) * Ls * R + k;
-#pragma unroll
-            for (int q = 0; q < R; q++) lb[(base + q * Ls) * es] = x[q];
-        }
-    }
-    if constexpr (!last) {
-        __syncthreads();
-        if (valid) {
-#pragma unroll
-            for (int e = 0; e < E; e++) v[e] = lb[(t + P * e) * es];
-        }
-        __syncthreads();
-        lds_line_stages<S + 1, RL, E, P>(v, lb, es, tw, t, valid);
-    }
-}
-
-// n-point FFTs of the lines of the x-y planes held in LDS (the dynamic shared memory of the
-// kernel): row r of plane p at (p n1 + r) rs, rs = xy_row_stride(n0) (odd), planes ps = n1 rs
-// apart.  ACROSS = false: the rows (line l at l rs, element stride 1); ACROSS = true: the columns
-// (line l = p n0 + c at p ps + c, element stride rs).  Consecutive lanes take consecutive lines
-// at one position t of their lines: the odd row stride puts the lanes of a row pass on distinct
-// LDS banks, consecutive columns are consecutive addresses.  NTH threads, rounds of NTH / P
-// lines.  The columns' results go from registers straight to global memory (col_store:
-// consecutive lanes store consecutive columns).
-template <typename RL, int E, int NTH, bool ACROSS, typename C, typename R>
-__device__ __forceinline__ void lds_lines_fft(int nlines, int n0, int rs, int ps, const C *__restrict__ tw,
-                                              const col_store<C, R> &cs) {
-    extern __shared__ __align__(16) unsigned char smem_raw[];
-    C *buf = reinterpret_cast<C *>(smem_raw);
-    constexpr int N = RL::n(), P = N / E, LPI = NTH / P;
-    static_assert(LPI >= 1, "a line needs at most the block's threads");
-    const int es = ACROSS ? rs : 1;
-    const int tid = threadIdx.x;
-    const int l0 = tid % LPI;
-    // with LPI a multiple of 64 a wave holds 64 consecutive lines at one position t: t, the
-    // twiddles and every element offset are uniform over the wave (scalar registers and loads)
-    int t = tid / LPI;
-    if constexpr (LPI % 64 == 0) t = __builtin_amdgcn_readfirstlane(t);
-    const bool inb = tid < LPI * P;
-    // a column line = (plane q, column r) of the planes, walked by LPI per round
-    int q = l0 / n0, r = l0 % n0;
-    const int dq = LPI / n0, dr = LPI % n0;
-    for (int first = 0; first < nlines; first += LPI) {
-        const int line = first + l0;
-        const bool valid = inb && line < nlines;
-        C *lb = buf + (!valid ? 0 : (ACROSS ? q * ps + r : line * rs));
-        C v[E];
-        if (valid) {
-#pragma unroll
-            for (int e = 0; e < E; e++) v[e] = lb[(t + P * e) * es];
-        }
-        __syncthreads();
-        lds_line_stages<0, RL, E, P>(v, lb, es, tw, t, valid);
-        if (valid) {
-            if constexpr (ACROSS) {
-                C *gb = cs.dst + q * cs.plane + r;
-#pragma unroll
-                for (int e = 0; e < E; e++) gb[(t + P * e) * cs.row] = cs.value(v[e]);
-            } else {
-#pragma unroll
-                for (int e = 0; e < E; e++) lb[(t + P * e) * es] = v[e];
-            }
-        }
-        __syncthreads();
-        q += dq;
-        r += dr;
-        if (r >= n0) r -= n0, q++;
-    }
-}
-
-// The stages of one line as lds_line_stages, for lengths whose radices do not all divide one
-// elements-per-thread count (105 = 3 5 7): each stage reads its butterflies' inputs from the
-// line's LDS slots (thread t takes butterflies t, t + P, ... < n / R), a barrier, then writes
-// their outputs; the last stage of a column (ACROSS) writes to global memory instead (gb: the
-// column's first element, rows cs.row apart).
-template <int S, typename RL, int P, bool ACROSS, typename C, typename R>
-__device__ __forceinline__ void staged_line_stages(C *lb, int es, const C *__restrict__ tw, int t, bool valid, C *gb,
-                                                   const col_store<C, R> &cs) {
-    constexpr int Rr = RL::at(S), Ls = RL::ls(S), N = RL::n(), NBT = N / Rr, NBS = (NBT + P - 1) / P;
-    constexpr bool last = (S + 1 == RL::count);
-    constexpr int TWO = RL::twoff(S);
-    C x[NBS][Rr];
-#pragma unroll
-    for (int j = 0; j < NBS; j++) {
-        const int b = t + P * j;
-        if (valid && b < NBT) {
-#pragma unroll
-            for (int p = 0; p < Rr; p++) x[j][p] = lb[(b + NBT * p) * es];
-            if constexpr (Ls > 1) {
-                const C *w = tw + TWO + (b % Ls) * (Rr - 1);
-#pragma unroll
-                for (int p = 1; p < Rr; p++) x[j][p] = cmul(x[j][p], w[p - 1]);
-            }
-            dft<Rr>::run(x[j]);
-        }
-    }
-    __syncthreads();  // every read of the stage before its writes
-#pragma unroll
-    for (int j = 0; j < NBS; j++) {
-        const int b = t + P * j;
-        if (valid && b < NBT) {
-            const int base = (b / Ls) * Ls * Rr + b % Ls;
-            if constexpr (last && ACROSS) {
-#pragma unroll
-                for (int q = 0; q < Rr; q++) gb[(base + q * Ls) * cs.row] = cs.value(x[j][q]);
-            } else {
-#pragma unroll
-                for (int q = 0; q < Rr; q++) lb[(base + q * Ls) * es] = x[j][q];
-            }
-        }
-    }
-    if constexpr (!last) {
-        __syncthreads();
-        staged_line_stages<S + 1, RL, P, ACROSS>(lb, es, tw, t, valid, gb, cs);
-    }
-}
-
-// lds_lines_fft for those lengths: P threads per line, lines and planes as there.
-template <typename RL, int P, int NTH, bool ACROSS, typename C, typename R>
-__device__ __forceinline__ void lds_lines_fft_staged(int nlines, int n0, int rs, int ps, const C *__restrict__ tw,
-                                                     const col_store<C, R> &cs) {
-    extern __shared__ __align__(16) unsigned char smem_raw[];
-    C *buf = reinterpret_cast<C *>(smem_raw);
-    constexpr int LPI = NTH / P;
-    static_assert(LPI >= 1, "a line needs at most the block's threads");
-    const int es = ACROSS ? rs : 1;
-    const int tid = threadIdx.x;
-    const int l0 = tid % LPI;
-    int t = tid / LPI;
-    if constexpr (LPI % 64 == 0) t = __builtin_amdgcn_readfirstlane(t);
-    const bool inb = tid < LPI * P;
-    // a column line = (plane q, column r) of the planes, walked by LPI per round
-    int q = l0 / n0, r = l0 % n0;
-    const int dq = LPI / n0, dr = LPI % n0;
-    for (int first = 0; first < nlines; first += LPI) {
-        const int line = first + l0;
-        const bool valid = inb && line < nlines;
-        C *lb = buf + (!valid ? 0 : (ACROSS ? q * ps + r : line * rs));
-        C *gb = (ACROSS && valid) ? cs.dst + q * cs.plane + r : cs.dst;
-        staged_line_stages<0, RL, P, ACROSS>(lb, es, tw, t, valid, gb, cs);
-        __syncthreads();
-        q += dq;
-        r += dr;
-        if (r >= n0) r -= n0, q++;
-    }
-}
-
-// threads per line of the staged lengths in the fused phase
-constexpr int kXyStagedThreads = 8;
-
-// Tiles the fused phase can run: every compile-time tile (register tiles through
-// lds_lines_fft, the staged tile through lds_lines_fft_staged)
-#define HMI_XY_OK(K, N, E, T, PS, ...) true,
-static const bool kXyOk[] = {HMI_BATCH_TABLE(HMI_XY_OK)};
-bool batch_xy_supported(int kid) { return kid >= 0 && kXyOk[kid]; }
-
-
-// the lines of one axis of the planes in LDS with the tile of length id kid (class <= CLS)
-template <typename R, int CLS, int NTH, bool ACROSS>
-__device__ __forceinline__ void xy_axis(int kid, int nlines, int n0, int rs, int ps, const typename cvec<R>::type *tw,
-                                        const col_store<typename cvec<R>::type, R> &cs) {
-#define HMI_XY_CASE(K, N, E, T, PS, ...)                                                        \
-    case K:                                                                                     \
-        if constexpr (E > 0 && batch_class_of(E) <= CLS && NTH / (N / (E > 0 ? E : 1)) >= 1)   \
-            lds_lines_fft<radices<__VA_ARGS__>, (E > 0 ? E : 1), NTH, ACROSS>(nlines, n0, rs, ps, tw, cs); \
-        else if constexpr (E == 0)                                                              \
-            lds_lines_fft_staged<radices<__VA_ARGS__>, kXyStagedThreads, NTH, ACROSS>(nlines, n0, rs, ps, tw, cs); \
-        break;
-    switch (kid) {
-        HMI_BATCH_TABLE(HMI_XY_CASE)
-        default: break;
-    }
-#undef HMI_XY_CASE
-}
-
-// Fused x-y phase: work item = (transform, group of G consecutive z-planes), G = max(1, budget /
-// (n1 rs)), rs = xy_row_stride(n0).  The planes are contiguous in memory: one coalesced load into
-// the padded rows in LDS (conjugated for the backward transform), the n0-point FFTs of the G n1
-// rows, the n1-point FFTs of the G n0 columns, whose results go from registers to global memory
-// (conjugated back; consecutive lanes write consecutive columns).  No scale: the z phase applies
-// it.
-template <typename R, int CLS, int NTH>
-__device__ __forceinline__ void xy_item(const batch_args &b, const batch_item &it, typename cvec<R>::type *buf) {
-    using C = typename cvec<R>::type;
-    const batch_xform x = b.xforms[it.xform];
-    const int n0 = x.n[0], n1 = x.n[1], n2 = x.n[2];
-    const int rs = xy_row_stride(n0), ps = n1 * rs;
-    const int G = b.xy_budget / ps > 1 ? b.xy_budget / ps : 1;
-    const int z0 = it.tile * G;
-    const int g = (n2 - z0) < G ? (n2 - z0) : G;
-    const int cnt = g * n1 * n0;
-    const long long zoff = (long long)z0 * n1 * n0;
-    const C *__restrict__ src = (b.from_in ? static_cast<const C *>(b.in) + x.in_off
-                                           : static_cast<const C *>(b.out) + x.out_off) + zoff;
-    C *__restrict__ dst = static_cast<C *>(b.out) + x.out_off + zoff;
-    const R sg = b.conj ? R(-1) : R(1);
-    // element i of the group sits in LDS row i / n0 (the g n1 rows back to back), column i % n0;
-    // walking i by NTH moves the pair by (NTH / n0, NTH % n0).  Loads go out U at a time before
-    // their LDS stores, so that U loads per thread are in flight.
-    constexpr int U = 24;
-    const int dr = NTH / n0, dc = NTH % n0;
-    const int r0 = (int)threadIdx.x / n0, c0 = (int)threadIdx.x % n0;
-    {
-        int r = r0, c = c0;
-        for (int i0 = threadIdx.x; i0 < cnt; i0 += U * NTH) {
-            C v[U];
-#pragma unroll
-            for (int u = 0; u < U; u++)
-                if (i0 + u * NTH < cnt) v[u] = src[i0 + u * NTH];
-#pragma unroll
-            for (int u = 0; u < U; u++) {
-                if (i0 + u * NTH < cnt) buf[r * rs + c] = cmk<C>(v[u].x, sg * v[u].y);
-                r += dr;
-                c += dc;
-                if (c >= n0) c -= n0, r++;
-            }
-        }
-    }
-    __syncthreads();
-    const C *__restrict__ tw = static_cast<const C *>(b.tw);
-    // x: g n1 rows of n0 points; y: g n0 columns of n1 points, stored from registers
-    const col_store<C, R> cs{dst, n0, (long long)n0 * n1, sg, R(1)};
-    xy_axis<R, CLS, NTH, false>(b.kid[x.size_id[0]], g * n1, n0, rs, ps, tw + b.twoff[x.size_id[0]], cs);
-    xy_axis<R, CLS, NTH, true>(b.kid[x.size_id[1]], g * n0, n0, rs, ps, tw + b.twoff[x.size_id[1]], cs);
-}
-
-// Every build at 2 waves per SIMD (up to 256 VGPRs): two 256-thread blocks per CU with 80 KiB of
-// LDS each, or one 512-thread block with up to 160 KiB.  The launchers use only the build of
-// class kXyMaxClass, which carries every tile.
-constexpr int kXyWaves[kBatchClasses][2] = {{2, 2}, {2, 2}, {2, 2}};
-
-template <typename R, int CLS>
-__global__ void __launch_bounds__(kXySmallThreads)
-__attribute__((amdgpu_waves_per_eu(kXyWaves[CLS][sizeof(R) == 8])))
-fft_batched_xy(batch_args b) {
-    using C = typename cvec<R>::type;
-    extern __shared__ __align__(16) unsigned char smem_raw[];
-    for (int i = blockIdx.x; i < b.nitems; i += gridDim.x)
-        xy_item<R, CLS, kXySmallThreads>(b, b.items[i], reinterpret_cast<C *>(smem_raw));
-}
-
-__global__ void __launch_bounds__(kXyLargeThreads) __attribute__((amdgpu_waves_per_eu(2)))
-fft_batched_xy_large(batch_args b) {
-    extern __shared__ __align__(16) unsigned char smem_raw[];
-    for (int i = blockIdx.x; i < b.nitems; i += gridDim.x)
-        xy_item<float, kXyLargeMaxClass[0], kXyLargeThreads>(b, b.items[i], reinterpret_cast<float2 *>(smem_raw));
-}
-static_assert(kXyLargeMaxClass[1] < 0, "the 1024-thread build is complex<float> only");
-
-// Column-block z phase: work item = (transform, block of w <= W = min(n0 n1, budget / n2)
-// consecutive (x, y) positions), the n2-point z lines of those positions: one load of the n2
-// rows of w contiguous elements (rows n0 n1 apart in memory) into LDS rows of w, the z FFTs with
-// consecutive lanes on consecutive positions (as the column FFTs of the x-y phase), results
-// stored from registers, scaled and conjugated back for the backward transform.
-template <typename R, int CLS, int NTH>
-__device__ __forceinline__ void zcol_item(const batch_args &b, const batch_item &it, typename cvec<R>::type *buf) {
-    using C = typename cvec<R>::type;
-    const batch_xform x = b.xforms[it.xform];
-    const int plane = x.n[0] * x.n[1], n2 = x.n[2];
-    const int W = zcol_width(n2, b.xy_budget, plane);
-    const int c0 = it.tile * W;
-    const int w = (plane - c0) < W ? (plane - c0) : W;
-    const int cnt = n2 * w;
-    const C *__restrict__ src = (b.from_in ? static_cast<const C *>(b.in) + x.in_off
-                                           : static_cast<const C *>(b.out) + x.out_off) + c0;
-    C *__restrict__ dst = static_cast<C *>(b.out) + x.out_off + c0;
-    const R sg = b.conj ? R(-1) : R(1);
-    const double ntot = (double)plane * (double)n2;
-    const R sc = (R)((b.scaling == 0) ? 1.0 : (b.scaling == 1 ? 1.0 / ntot : sqrt(1.0 / ntot)));
-    // element i of the block (row z = i / w, column c = i % w) sits at LDS i; walking i by NTH
-    // moves (z, c) by (NTH / w, NTH % w).  Loads go out U at a time before their LDS stores.
-    constexpr int U = 24;
-    const int dz = NTH / w, dc = NTH % w;
-    int z = (int)threadIdx.x / w, c = (int)threadIdx.x % w;
-    for (int i0 = threadIdx.x; i0 < cnt; i0 += U * NTH) {
-        C v[U];
-        int zz = z, cc = c;
-#pragma unroll
-        for (int u = 0; u < U; u++) {
-            if (i0 + u * NTH < cnt) v[u] = src[(long long)zz * plane + cc];
-            zz += dz;
-            cc += dc;
-            if (cc >= w) cc -= w, zz++;
-        }
-#pragma unroll
-        for (int u = 0; u < U; u++)
-            if (i0 + u * NTH < cnt) buf[i0 + u * NTH] = cmk<C>(v[u].x, sg * v[u].y);
-        z = zz;
-        c = cc;
-    }
-    __syncthreads();
-    const col_store<C, R> cs{dst, plane, 0, sg, sc};
-    xy_axis<R, CLS, NTH, true>(b.kid[x.size_id[2]], w, w, w, 0,
-                               static_cast<const C *>(b.tw) + b.twoff[x.size_id[2]], cs);
-}
-
-template <typename R, int CLS>
-__global__ void __launch_bounds__(kXySmallThreads)
-__attribute__((amdgpu_waves_per_eu(kXyWaves[CLS][sizeof(R) == 8])))
-fft_batched_zcol(batch_args b) {
-    using C = typename cvec<R>::type;
-    extern __shared__ __align__(16) unsigned char smem_raw[];
-    for (int i = blockIdx.x; i < b.nitems; i += gridDim.x)
-        zcol_item<R, CLS, kXySmallThreads>(b, b.items[i], reinterpret_cast<C *>(smem_raw));
-}
-
-template <typename R, int CLS>
-constexpr batched_fn zcol_build() {
-    if constexpr (CLS == kXyMaxClass[sizeof(R) == 8]) return &fft_batched_zcol<R, CLS>;
-    else return nullptr;
-}
-template <int... CS>
-static const batched_fn *batched_zcol_builds(bool dbl, std::integer_sequence<int, CS...>) {
-    static const batched_fn f[2][sizeof...(CS)] = {{zcol_build<float, CS>()...}, {zcol_build<double, CS>()...}};
-    return f[dbl ? 1 : 0];
-}
-
-hipError_t launch_batched_zcol(bool dbl, int cls, const batch_args &b, int nblocks, size_t lds_bytes, hipStream_t s) {
-    static const bool configured = [] {
-        for (int d = 0; d < 2; d++)
-            for (int c = 0; c < kBatchClasses; c++) {
-                const batched_fn fn = batched_zcol_builds(d != 0, std::make_integer_sequence<int, kBatchClasses>())[c];
-                if (fn)
-                    (void)hipFuncSetAttribute(reinterpret_cast<const void *>(fn),
-                                              hipFuncAttributeMaxDynamicSharedMemorySize, kGenericMaxLds);
-            }
-        return true;
-    }();
-    (void)configured;
-    if (cls < 0 || cls >= kBatchClasses || cls > kXyMaxClass[dbl ? 1 : 0]) return hipErrorInvalidValue;
-    if (lds_bytes > (size_t)kGenericMaxLds) return hipErrorInvalidValue;
-    const batched_fn fn = batched_zcol_builds(dbl, std::make_integer_sequence<int, kBatchClasses>())[cls];
-    if (!fn) return hipErrorInvalidValue;
-    fn<<<dim3((unsigned)nblocks), dim3(kXySmallThreads), lds_bytes, s>>>(b);
-    return hipGetLastError();
-}
-
-template <typename R, int CLS>
-constexpr batched_fn xy_build() {
-    if constexpr (CLS == kXyMaxClass[sizeof(R) == 8]) return &fft_batched_xy<R, CLS>;
-    else return nullptr;
-}
-template <int... CS>
-static const batched_fn *batched_xy_builds(bool dbl, std::integer_sequence<int, CS...>) {
-    static const batched_fn f[2][sizeof...(CS)] = {{xy_build<float, CS>()...}, {xy_build<double, CS>()...}};
-    return f[dbl ? 1 : 0];
-}
-
-hipError_t launch_batched_xy(bool dbl, bool large, int cls, const batch_args &b, int nblocks, size_t lds_bytes,
-                             hipStream_t s) {
-    static const bool configured = [] {
-        for (int d = 0; d < 2; d++)
-            for (int c = 0; c < kBatchClasses; c++) {
-                const batched_fn fn = batched_xy_builds(d != 0, std::make_integer_sequence<int, kBatchClasses>())[c];
-                if (fn)
-                    (void)hipFuncSetAttribute(reinterpret_cast<const void *>(fn),
-                                              hipFuncAttributeMaxDynamicSharedMemorySize, kGenericMaxLds);
-            }
-        (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&fft_batched_xy_large),
-                                  hipFuncAttributeMaxDynamicSharedMemorySize, kGenericMaxLds);
-        return true;
-    }();
-    (void)configured;
-    if (cls < 0 || cls >= kBatchClasses || cls > (large ? kXyLargeMaxClass : kXyMaxClass)[dbl ? 1 : 0])
-        return hipErrorInvalidValue;
-    if (!large && !batched_xy_builds(dbl, std::make_integer_sequence<int, kBatchClasses>())[cls])
-        return hipErrorInvalidValue;
-    if (lds_bytes > (size_t)kGenericMaxLds) return hipErrorInvalidValue;
-    if (large) {
-        fft_batched_xy_large<<<dim3((unsigned)nblocks), dim3(kXyLargeThreads), lds_bytes, s>>>(b);
-    } else {
-        const batched_fn fn = batched_xy_builds(dbl, std::make_integer_sequence<int, kBatchClasses>())[cls];
-        fn<<<dim3((unsigned)nblocks), dim3(kXySmallThreads), lds_bytes, s>>>(b);
-    }
-    return hipGetLastError();
-}
-
 // ------------------------------------------------------------- permutation
 
 // dst[i so_f + j so_m + k so_s] = src[i si_f + j si_m + k si_s] over a

@@ -159,6 +159,12 @@ struct batch_item {
     int tile;   // tile of lines along the phase axis
 };
 
+// How the fused phases run one transform: planes per x-y work item, columns per z work item.
+struct batch_fused {
+    int planes, width;
+    fast_div by_rows, by_cols, by_n0, by_width;
+};
+
 struct batch_args {
     const void *in;
     void *out;
@@ -173,8 +179,12 @@ struct batch_args {
     int from_in;    // 1: read the input arrays (first phase), 0: read the output arrays in place
     int conj;       // backward transform
     int scaling;    // 0 none, 1 full (1/N of each transform), 2 symmetric; applied by the last phase
-    int xy_budget;  // fused x-y phase: elements of the planes one work item holds in LDS (a work
-                    // item of a transform takes max(1, xy_budget / (n0 n1)) consecutive z-planes)
+    // fused phases: one entry per transform; runtime-length radix plans and tables (byte offsets into
+    // mtab) of each length
+    const batch_fused *fused;
+    const mixed_plan *mplans;
+    const unsigned char *mtab;
+    const int *mtoff;
 };
 
 }  // namespace hmi

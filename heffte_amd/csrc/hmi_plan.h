@@ -204,6 +204,7 @@ std::vector<unsigned char> mixed_table(const mixed_plan &g, bool dbl, long long 
 // Fused pass over planes of n0 x n1 elements (ok false: it does not take them), nplanes of them in one
 // transform.
 plane_config make_plane(int n0, int n1, long long nplanes, bool dbl);
+fast_div make_fast_div(unsigned d);
 // the divisors of one launch's line numbering
 void mixed_launch_divs(mixed_plan &g, const pass_args &a);
 

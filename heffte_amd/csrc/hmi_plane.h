@@ -171,6 +171,181 @@ template <typename R, bool HEAVY, int NTM> __global__ void __launch_bounds__(kMi
     HMI_MIXED_SWITCH(a.g1.last, HMI_PLANE_STORE)
 }
 
+// ---- batches: the same stages over work lists of transforms of different sizes
+
+// Copy of a device-resident radix plan (uniform over the block: scalar loads)
+__device__ __forceinline__ mixed_plan load_plan(const mixed_plan *p) {
+#ifdef HMI_EMULATE
+    return *p;
+#else
+    mixed_plan g;
+    const auto *src = (const __attribute__((address_space(4))) int *)(uintptr_t)p;
+    int *dst = reinterpret_cast<int *>(&g);
+#pragma unroll
+    for (unsigned i = 0; i < sizeof(mixed_plan) / 4; i++) dst[i] = src[i];
+    return g;
+#endif
+}
+
+// First stage of a column block, global memory -> LDS: position i of column l at src + i row + l.
+template <int RX, typename R, typename C>
+__device__ __forceinline__ void cols_load(const plane_args &a, const C *__restrict__ tw, const C *src, long long row, unsigned w,
+                                          C *lds) {
+    const int m = a.g1.m0;
+    const R sg = a.conj ? R(-1) : R(1);
+    for (unsigned idx = threadIdx.x; idx < a.cols * (unsigned)m; idx += blockDim.x) {
+        const unsigned j = fdiv(idx, a.by_cols), l = idx - j * a.cols;
+        if (l >= w) continue;
+        const C *sp = src + (long long)j * row + l;
+        const long long st = (long long)m * row;
+        C x[RX];
+#pragma unroll
+        for (int p = 0; p < RX; p++) x[p] = sp[p * st];
+#pragma unroll
+        for (int p = 0; p < RX; p++) x[p].y *= sg;
+        dft<RX>::run(x);
+        if (m > 1) {
+            const C *wt = tw + j * (RX - 1);
+#pragma unroll
+            for (int q = 1; q < RX; q++) x[q] = cmul(x[q], wt[q - 1]);
+        }
+        C *dp = lds + (int)j * a.rp + (int)l;
+#pragma unroll
+        for (int q = 0; q < RX; q++) dp[q * m * a.rp] = x[q];
+    }
+}
+
+// Last stage of a column block, LDS -> global memory.
+template <int RX, typename R, typename C>
+__device__ __forceinline__ void cols_store(const plane_args &a, C *dst, long long row, unsigned w, const C *lds) {
+    const unsigned nb = (unsigned)(a.g1.n / RX);
+    const R sc = (R)a.scale, sy = a.conj ? -sc : sc;
+    for (unsigned idx = threadIdx.x; idx < nb * a.cols; idx += blockDim.x) {
+        const unsigned u = fdiv(idx, a.by_cols), l = idx - u * a.cols;
+        if (l >= w) continue;
+        const C *sp = lds + (int)plane_block(u, a.g1) * RX * a.rp + (int)l;
+        C x[RX];
+#pragma unroll
+        for (int p = 0; p < RX; p++) x[p] = sp[p * a.rp];
+        dft<RX>::run(x);
+        C *dp = dst + (long long)u * row + l;
+        const long long st = (long long)nb * row;
+#pragma unroll
+        for (int q = 0; q < RX; q++) dp[q * st] = cmk<C>(x[q].x * sc, x[q].y * sy);
+    }
+}
+
+// One-stage lengths: the transformed columns back to global memory.
+template <typename R, typename C>
+__device__ __forceinline__ void cols_copy(const plane_args &a, C *dst, long long row, unsigned w, const C *lds) {
+    const R sc = (R)a.scale, sy = a.conj ? -sc : sc;
+    for (unsigned idx = threadIdx.x; idx < a.cols * (unsigned)a.g1.n; idx += blockDim.x) {
+        const unsigned k = fdiv(idx, a.by_cols), l = idx - k * a.cols;
+        if (l >= w) continue;
+        const C v = lds[(int)k * a.rp + (int)l];
+        dst[(long long)k * row + l] = cmk<C>(v.x * sc, v.y * sy);
+    }
+}
+
+// Fused phases of a batch.  XY: item = (transform, group of consecutive z-planes), both axes of the
+// planes in LDS, input to output arrays, no scale.  Otherwise: item = (transform, block of consecutive
+// (x, y) positions), their z lines, in place in the output arrays, with the scale.
+//
+// Bound: HBM bytes in the z phase, LDS and issue inside the blocks in the x-y phase.  1000 transforms of
+// sides 16 ... 128, complex<float>, 1.5 GB: x-y 0.79 ms (3.8 TB/s, in three launches by block size),
+// z 0.62 ms (4.8 TB/s) a direction, pair 3.69 -> 2.83 ms against compile-time tiles that held whole
+// butterfly chains per line in registers (two 256-thread blocks per CU; x-y 1.2 ms, z 0.75 ms).  Measured
+// around it: radices up to 10 only 3.10 ms; first block size 32, 24 or 52 KB 2.84-2.88; 512 threads in it
+// 3.00, 256 in the second 2.92; z blocks of 20 KB 2.94, of 80 KB with 512 threads 2.79.
+template <typename R, bool XY, int NTH> __global__ void __launch_bounds__(NTH) fft_batch_fused(batch_args b) {
+    using C = typename cvec<R>::type;
+    constexpr bool HEAVY = true;
+    constexpr int NTM = 0;
+    extern __shared__ __align__(16) unsigned char smem_raw[];
+    C *lds = reinterpret_cast<C *>(smem_raw);
+    for (int i = blockIdx.x; i < b.nitems; i += gridDim.x) {
+        const batch_item it = b.items[i];
+        const batch_xform x = b.xforms[it.xform];
+        const batch_fused f = b.fused[it.xform];
+        const int n0 = x.n[0], n1 = x.n[1], n2 = x.n[2];
+        plane_args a;
+        a.mul = nullptr;
+        a.conj = b.conj;
+        const C *in = b.from_in ? static_cast<const C *>(b.in) + x.in_off : static_cast<const C *>(b.out) + x.out_off;
+        C *out = static_cast<C *>(b.out) + x.out_off;
+        a.in = in;
+        a.out = out;
+        const int id1 = x.size_id[XY ? 1 : 2];
+        a.g1 = load_plan(b.mplans + id1);
+        const unsigned char *t1 = b.mtab + b.mtoff[id1];
+        const C *__restrict__ tw1 = reinterpret_cast<const C *>(t1 + kMixedHead);
+        const mixed_stage *st1 = reinterpret_cast<const mixed_stage *>(t1);
+        unsigned planes = 0, w = 0;
+        long long base = 0;
+        const long long row = (long long)n0 * n1;
+        if constexpr (XY) {
+            const int id0 = x.size_id[0];
+            a.g0 = load_plan(b.mplans + id0);
+            const unsigned char *t0 = b.mtab + b.mtoff[id0];
+            const C *__restrict__ tw0 = reinterpret_cast<const C *>(t0 + kMixedHead);
+            const mixed_stage *st0 = reinterpret_cast<const mixed_stage *>(t0);
+            const unsigned z0 = (unsigned)(it.tile * f.planes);
+            planes = (unsigned)(n2 - (int)z0 < f.planes ? n2 - (int)z0 : f.planes);
+            base = z0 * row;
+            a.n0 = n0;
+            a.n1 = n1;
+            a.rp = n0 | 1;
+            a.ps = n1 * a.rp;
+            a.rows = (unsigned)(f.planes * n1);
+            a.cols = (unsigned)(f.planes * n0);
+            a.by_rows = f.by_rows;
+            a.by_cols = f.by_cols;
+            a.by_n0 = f.by_n0;
+            a.scale = 1.0;
+            HMI_MIXED_SWITCH(a.g0.radix[0], HMI_PLANE_LOAD)
+            __syncthreads();
+            for (int s = 1; s < a.g0.nst; s++) {
+                const mixed_stage st = st0[s - 1];
+                HMI_MIXED_SWITCH(st.radix, HMI_PLANE_ROW)
+                __syncthreads();
+            }
+            if (a.g1.nst > 1) {
+                HMI_MIXED_SWITCH(a.g1.radix[0], HMI_PLANE_COL0)
+                __syncthreads();
+            }
+        } else {
+            const long long c0 = (long long)it.tile * f.width;
+            w = (unsigned)(row - c0 < f.width ? row - c0 : f.width);
+            a.n0 = f.width;
+            a.rp = f.width;
+            a.ps = 0;
+            a.cols = (unsigned)f.width;
+            a.by_cols = f.by_width;
+            a.by_n0 = f.by_width;
+            const double ntot = (double)row * (double)n2;
+            a.scale = (b.scaling == 0) ? 1.0 : (b.scaling == 1 ? 1.0 / ntot : sqrt(1.0 / ntot));
+            in += c0;
+            out += c0;
+#define HMI_COLS_LOAD(RX) case RX: cols_load<RX, R>(a, tw1, in, row, w, lds); break;
+            HMI_MIXED_SWITCH(a.g1.radix[0], HMI_COLS_LOAD)
+            __syncthreads();
+        }
+        for (int s = 1; s + 1 < a.g1.nst; s++) {
+            const mixed_stage st = st1[s - 1];
+            HMI_MIXED_SWITCH(st.radix, HMI_PLANE_COL)
+            __syncthreads();
+        }
+        if constexpr (XY) {
+            HMI_MIXED_SWITCH(a.g1.last, HMI_PLANE_STORE)
+        } else {
+#define HMI_COLS_STORE(RX) case RX: cols_store<RX, R>(a, out, row, w, lds); break;
+            if (a.g1.nst == 1) cols_copy<R>(a, out, row, w, lds);
+            else { HMI_MIXED_SWITCH(a.g1.last, HMI_COLS_STORE) }
+        }
+        __syncthreads();
+    }
+}
+
 template <typename R> struct plane_builds {
     using fn = void (*)(plane_args);
     static fn choose(const plane_args &a) {
@@ -206,5 +381,21 @@ template <typename R> struct plane_builds {
     }
 #endif
 };
+
+#ifndef HMI_EMULATE
+template <typename R> hipError_t launch_batch_builds(bool xy, const batch_args &b, int threads, int nblocks, size_t lds, hipStream_t s) {
+    static const bool configured = [] {
+        for (const void *f : {reinterpret_cast<const void *>(&fft_batch_fused<R, true, kMixedThreads>),
+                              reinterpret_cast<const void *>(&fft_batch_fused<R, false, kMixedThreads>)})
+            (void)hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, kGenericMaxLds);
+        return true;
+    }();
+    (void)configured;
+    if (threads > kMixedThreads || lds > (size_t)kGenericMaxLds) return hipErrorInvalidValue;
+    (xy ? &fft_batch_fused<R, true, kMixedThreads> : &fft_batch_fused<R, false, kMixedThreads>)
+        <<<dim3((unsigned)nblocks), dim3(threads), lds, s>>>(b);
+    return hipGetLastError();
+}
+#endif
 
 }  // namespace hmi

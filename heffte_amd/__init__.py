@@ -195,9 +195,9 @@ def _ptr(t):
     if t is None:
         return None
     if hasattr(t, "data_ptr"):
-        return ctypes.c_void_p(t.data_ptr())
+        return t.data_ptr()  # (the argument types convert an address)
     if isinstance(t, int):
-        return ctypes.c_void_p(t)
+        return t
     raise heffte_input_error("arrays must be torch tensors on the GPU or raw device addresses")
 
 
@@ -212,6 +212,10 @@ class fft_plan:
         self._h = handle
         self.kind = k
         self.use_r2c = (k == kind.r2c)
+        # extents never change; the entry point and workspace width of each pair of element types
+        # are looked up by name once (_entry)
+        self._sizes = (self.size_inbox(), self.size_outbox(), self.size_workspace())
+        self._entries = {}
 
     def __del__(self):
         h = getattr(self, "_h", None)
@@ -267,9 +271,8 @@ class fft_plan:
         s = getattr(stream, "cuda_stream", stream)
         _check(lib.heffte_mi355_set_stream(self._h, ctypes.c_void_p(s) if s else None), "set_stream")
 
-    def _call(self, direction, inarray, outarray, workspace, scaling, batch):
-        if scaling not in (0, 1, 2):
-            raise heffte_input_error(f"{direction}() called with invalid scaling")
+    def _entry(self, direction, inarray, outarray):
+        """(library function, bytes of a workspace element) for the arrays' element types."""
         ti, to = _dtype_name(inarray), _dtype_name(outarray)
         if self.kind in (kind.cos, kind.sin, kind.cos1):
             table = {("float32", "float32"): "s2s", ("float64", "float64"): "d2d"}
@@ -284,16 +287,27 @@ class fft_plan:
         key = table.get((ti, to))
         if key is None:
             raise heffte_input_error(f"{direction}() called with incompatible types {ti} -> {to}")
-        nin, nout = (self.size_inbox(), self.size_outbox()) if direction == "forward" else (
-            self.size_outbox(), self.size_inbox())
+        width = 16 if key in ("z2z", "d2z", "z2d") else 8 if key in ("c2c", "s2c", "c2s", "d2d") else 4
+        return getattr(lib, f"heffte_mi355_{direction}_{key}"), width
+
+    def _call(self, direction, inarray, outarray, workspace, scaling, batch):
+        if scaling not in (0, 1, 2):
+            raise heffte_input_error(f"{direction}() called with invalid scaling")
+        types = (direction, inarray.dtype, outarray.dtype)
+        entry = self._entries.get(types)
+        if entry is None:
+            entry = self._entries[types] = self._entry(direction, inarray, outarray)
+        fn, width = entry
+        nin, nout, nws = self._sizes
+        if direction != "forward":
+            nin, nout = nout, nin
         if inarray.numel() < batch * nin or outarray.numel() < batch * nout:
             raise heffte_input_error(f"{direction}() called with invalid array size")
-        if workspace is not None and workspace.numel() * workspace.element_size() < \
-                batch * self.size_workspace() * (16 if key in ("z2z", "d2z", "z2d") else
-                                                 8 if key in ("c2c", "s2c", "c2s", "d2d") else 4):
+        if workspace is not None and workspace.numel() * workspace.element_size() < batch * nws * width:
             raise heffte_input_error(f"{direction}() called with insufficient workspace size")
-        fn = getattr(lib, f"heffte_mi355_{direction}_{key}")
-        _check(fn(self._h, batch, _ptr(inarray), _ptr(outarray), _ptr(workspace), scaling), direction)
+        rc = fn(self._h, batch, _ptr(inarray), _ptr(outarray), _ptr(workspace), scaling)
+        if rc != 0:
+            _check(rc, direction)
 
     def forward(self, inarray, outarray, scaling=scale.none, batch=1):
         self._call("forward", inarray, outarray, None, scaling, batch)

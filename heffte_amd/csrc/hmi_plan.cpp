@@ -827,14 +827,14 @@ void launch_mixed_pass(const pass &p, const pass_args &a, bool dbl, hipStream_t 
 }
 }  // namespace
 
-void fft_plan::launch_plane(const pass &p, const pass_args &base, bool dbl, int batch) {
+void fft_plan::launch_plane(const pass &p, const pass_args &base, const void *table1, bool dbl, int batch) {
     const plane_config &c = *p.plane;
     plane_args a = c.args;
     a.in = base.in;
     a.out = base.out;
     a.mul = base.mul;
-    a.tw0 = get_plane_table(dbl, a.g0, false).dev;
-    a.tw1 = get_plane_table(dbl, a.g1, false).dev;
+    a.tw0 = base.tw;
+    a.tw1 = table1;
     const long long nplanes = p.lin.n[p.b1] * batch;
     if (nplanes > 0x7fffffffLL) throw std::runtime_error("too many planes in one pass");
     a.nplanes = (int)nplanes;
@@ -887,14 +887,15 @@ void fft_plan::execute(int dir, bool dbl, bool in_real, bool out_real, int batch
     constexpr size_t kMaxPasses = 8;
     if (ep.passes.size() > kMaxPasses) throw std::runtime_error("internal error: too many passes");
     std::array<const void *, kMaxPasses> tables{};
+    const void *second_table = nullptr;
     for (size_t i = 0; i < ep.passes.size(); i++) {
         const pass &p = ep.passes[i];
         const bool mfma = split && p.n == 512 && p.mode == kModeC2C && !p.identity && !p.in_real && !p.out_real &&
                           !p.herm_load && p.store_len == p.n && !(mul && i == 0);
         if (p.plane) {
-            // both axes' tables (launch_plane uses them)
-            for (const mixed_plan *g : {&p.plane->args.g0, &p.plane->args.g1})
-                tables[i] = get_plane_table(dbl, *g, may_alloc).dev;
+            // both axes' tables (at most one pass of a plan is fused)
+            tables[i] = get_plane_table(dbl, p.plane->args.g0, may_alloc).dev;
+            second_table = get_plane_table(dbl, p.plane->args.g1, may_alloc).dev;
         } else if (p.split) {
             // both steps' tables and the step twiddles, looked up now (launch_split uses them)
             for (const pass &q : *p.split) (void)get_twiddles(dbl, q, may_alloc);
@@ -921,7 +922,7 @@ void fft_plan::execute(int dir, bool dbl, bool in_real, bool out_real, int batch
         for (int d = 0; d < 3; d++) e += (L.n[d] - 1) * L.stride[d];
         return e + (long long)(batch - 1) * (L.n[0] * L.n[1] * L.n[2]) + 1;
     };
-    const bool debug = std::getenv("HMI_DEBUG_PLAN") != nullptr;
+    static const bool debug = std::getenv("HMI_DEBUG_PLAN") != nullptr;
     // per-pass timing: one event before the first pass and one after each pass
     std::unique_lock<std::mutex> tlock(timing_mtx_, std::defer_lock);
     hipEvent_t tprev = nullptr;
@@ -950,7 +951,7 @@ void fft_plan::execute(int dir, bool dbl, bool in_real, bool out_real, int batch
         const bool mfma = split && p.n == 512 && p.mode == kModeC2C && !p.identity && !p.in_real && !p.out_real &&
                           !p.herm_load && p.store_len == p.n && !a.mul;
         if (p.plane) {
-            launch_plane(p, a, dbl, batch);
+            launch_plane(p, a, second_table, dbl, batch);
         } else if (p.split) {
             launch_split(p, a, dbl, batch, static_cast<char *>(ws) + (size_t)batch * p.split_ws * (dbl ? 16 : 8));
         } else if (mfma) {

@@ -167,7 +167,7 @@ class fft_plan {
     const twiddles &get_twiddles(bool dbl, const pass &p, bool may_alloc);
     const twiddles &get_plane_table(bool dbl, const mixed_plan &g, bool may_alloc);
     const twiddles &get_split_table(bool dbl, int n, bool may_alloc);
-    void launch_plane(const pass &p, const pass_args &base, bool dbl, int batch);
+    void launch_plane(const pass &p, const pass_args &base, const void *table1, bool dbl, int batch);
     void launch_split(const pass &p, const pass_args &base, bool dbl, int batch, void *tmp);
     const twiddles &get_mfma_table(int prec, bool conj, bool may_alloc);
     template <typename F> void for_each_variant(F &&f) const;

@@ -115,6 +115,54 @@ __device__ __forceinline__ void run_stages(C (&v)[E], C *lds, const C *__restric
     }
 }
 
+// The stages of run_stages with the exchanges of the real and the imaginary parts one after the other
+// through an LDS tile of half the size (R values).
+template <int S, typename RL, int E, int P, int PS, typename LM, typename C, typename R>
+__device__ __forceinline__ void run_stages_halved(C (&v)[E], R *lds, const C *__restrict__ tw, int l, int t, int l2, int t2) {
+    constexpr int Rx = RL::at(S);
+    constexpr int Ls = RL::ls(S);
+    constexpr int NB = E / Rx;
+    constexpr bool last = (S + 1 == RL::count);
+    constexpr int TWO = RL::twoff(S);
+#pragma unroll
+    for (int r = 0; r < NB; r++) {
+        const int k = (t + P * r) % Ls;
+        C x[Rx];
+#pragma unroll
+        for (int p = 0; p < Rx; p++) x[p] = v[r + NB * p];
+        if constexpr (Ls > 1) {
+            const C *w = tw + TWO + k * (Rx - 1);
+#pragma unroll
+            for (int p = 1; p < Rx; p++) x[p] = cmul(x[p], w[p - 1]);
+        }
+        dft<Rx>::run(x);
+#pragma unroll
+        for (int q = 0; q < Rx; q++) v[r + NB * q] = x[q];
+    }
+    if constexpr (!last) {
+        auto put = [&](auto part) {
+#pragma unroll
+            for (int r = 0; r < NB; r++) {
+                const int b = t + P * r, base = (b / Ls) * Ls * Rx + b % Ls;
+#pragma unroll
+                for (int q = 0; q < Rx; q++) lds[LM::idx(l, base + q * Ls)] = part(v[r + NB * q]);
+            }
+        };
+        R re[E];
+        put([](const C &c) { return c.x; });
+        __syncthreads();
+#pragma unroll
+        for (int e = 0; e < E; e++) re[e] = lds[LM::idx(l2, t2 + P * e)];
+        __syncthreads();
+        put([](const C &c) { return c.y; });
+        __syncthreads();
+#pragma unroll
+        for (int e = 0; e < E; e++) v[e] = cmk<C>(re[e], lds[LM::idx(l2, t2 + P * e)]);
+        __syncthreads();
+        run_stages_halved<S + 1, RL, E, P, PS, LM>(v, lds, tw, l2, t2, l2, t2);
+    }
+}
+
 // Offset of line L (column-fastest numbering of column x b1 x batch).
 __device__ __forceinline__ long long line_offset(unsigned L, const pass_args &a, bool out) {
     const unsigned q = L / (unsigned)a.ncol;
@@ -136,6 +184,7 @@ __device__ __forceinline__ unsigned line_index(unsigned L, const pass_args &a, i
 // One tile (T lines) of an n-point pass; the block has exactly (n / E) * T threads.
 template <typename R, typename RL, int E, int T, int PS, int NTM = 0>
 __device__ __forceinline__ void uniform_tile(const pass_args &a, unsigned tile, typename cvec<R>::type *lds) {
+    constexpr bool HALVED = (NTM & 4) != 0;
     using C = typename cvec<R>::type;
     constexpr int N = RL::n();
     constexpr int P = N / E;
@@ -161,7 +210,7 @@ __device__ __forceinline__ void uniform_tile(const pass_args &a, unsigned tile, 
         const unsigned L = tile * T + l;
         const bool valid = active && L < (unsigned)a.nlines;
         const long long base = valid ? line_offset(L, a, false) : 0;
-        if (a.mode == kModeR2C) {
+        if (!HALVED && a.mode == kModeR2C) {
             // real line of 2N values read as N complex pairs z[m] = x[2m] + i x[2m+1]; a contiguous
             // line (even offsets: every other stride is a multiple of 2N) of an array aligned to
             // the pair size is read pairwise
@@ -178,7 +227,7 @@ __device__ __forceinline__ void uniform_tile(const pass_args &a, unsigned tile, 
                                  : cmk<C>(R(0), R(0));
                 }
             }
-        } else if (a.mode == kModeC2R) {
+        } else if (!HALVED && a.mode == kModeC2R) {
             // half spectrum X[0..N] of a real line of 2N values -> Z[k] = (X[k] + conj X[N-k])
             //   + i w^{-k} (X[k] - conj X[N-k]), the spectrum of z[m] = x[2m] + i x[2m+1];
             // the imaginary parts of X[0] and X[N] do not contribute to a real signal
@@ -282,7 +331,8 @@ __device__ __forceinline__ void uniform_tile(const pass_args &a, unsigned tile, 
         }
     }
 
-    run_stages<0, RL, E, P, RS, PS>(v, lds, tw, l, t, l2, t2);
+    if constexpr (HALVED) run_stages_halved<0, RL, E, P, PS, LM>(v, reinterpret_cast<R *>(lds), tw, l, t, l2, t2);
+    else run_stages<0, RL, E, P, RS, PS>(v, lds, tw, l, t, l2, t2);
     if constexpr (RL::count == 1) {
         if (a.load_colfast != a.store_colfast) {
 #pragma unroll
@@ -298,7 +348,7 @@ __device__ __forceinline__ void uniform_tile(const pass_args &a, unsigned tile, 
     const bool svalid = active && L2 < (unsigned)a.nlines;
     const R s = (R)a.scale;
     const long long obase = svalid ? line_offset(L2, a, true) : 0;
-    if (a.mode == kModeR2C) {
+    if (!HALVED && a.mode == kModeR2C) {
         // Z = DFT_N(z); X[k] = E[k] + w^k O[k], E = (Z[k] + conj Z[N-k]) / 2, O = -i (Z[k] - conj Z[N-k]) / 2
 #pragma unroll
         for (int e = 0; e < E; e++) lds[LM::idx(l2, t2 + P * e)] = v[e];
@@ -345,7 +395,7 @@ __device__ __forceinline__ void uniform_tile(const pass_args &a, unsigned tile, 
 #pragma unroll
         for (int e = 0; e < E; e++)
             if (t2 + P * e < a.store_len) stg<NTS>(&dst[obase + (long long)(t2 + P * e) * a.out_sa], v[e].x * f);
-    } else if (a.mode == kModeC2R) {
+    } else if (!HALVED && a.mode == kModeC2R) {
         R *__restrict__ dst = static_cast<R *>(a.out);
         if (a.out_sa == 1 && (reinterpret_cast<size_t>(a.out) & (sizeof(C) - 1)) == 0) {
 #pragma unroll
@@ -388,13 +438,13 @@ __device__ __forceinline__ void uniform_tile(const pass_args &a, unsigned tile, 
     }
 }
 
-// NTM: bit 0 = non-temporal stores, bit 1 = non-temporal loads of the pass data
+// NTM: bit 0 = non-temporal stores, bit 1 = non-temporal loads of the pass data, bit 2 = exchanges in halves
 template <typename R, typename RL, int E, int T, int PS, int NTM>
 __global__ void __launch_bounds__((RL::n() / E) * T) fft_uniform(pass_args a) {
     using C = typename cvec<R>::type;
     constexpr int RS = lds_map<RL::n(), E, PS, sizeof(C)>::RS;
     constexpr int CHUNK = T * (int)sizeof(C);
-    __shared__ C lds[T * RS];
+    __shared__ C lds[(NTM & 4) ? (T * RS + 1) / 2 : T * RS];
     unsigned tile = blockIdx.x;
     if (a.load_colfast || a.store_colfast) {
         if constexpr (CHUNK >= 128 || CHUNK <= 32) {
@@ -841,8 +891,23 @@ __global__ void __launch_bounds__(256) permute_kernel(const E *__restrict__ src,
 
 // ----------------------------------------------------------- fast registry
 
+// Real-to-real passes in complex<double> of 256 and more points, 8 elements per thread: their loads and
+// stores move half the bytes of a complex tile, so the pass is bound by latency, and its LDS holds a CU
+// to half the waves that its registers would allow.  Exchanging the parts one after the other in a tile
+// of half the size: 256^3 double DCT-II / III pair 465 -> 438 us, the results bit for bit the same.  The
+// complex passes stay as they are (512^3 complex<double> 768 -> 787 us per pass, 256^3 109 -> 108).
+constexpr bool halved_tile(int n, int e, int bytes) { return n >= 256 && bytes == 16 && e <= 8; }
+
 #define HMI_FAST(TYPE, N, E, T, PS, ...)                                                                  \
     static hipError_t launch_##TYPE##_##N##_##T(const pass_args &a, long long nblocks, hipStream_t s) {    \
+        if constexpr (halved_tile(N, E, 2 * sizeof(TYPE))) {                                               \
+            if (a.mode >= kModeDCT2) {                                                                     \
+                (a.stream ? &fft_uniform<TYPE, radices<__VA_ARGS__>, E, T, PS, 7>                          \
+                          : &fft_uniform<TYPE, radices<__VA_ARGS__>, E, T, PS, 4>)                         \
+                    <<<dim3((unsigned)nblocks), dim3((N / E) * T), 0, s>>>(a);                             \
+                return hipGetLastError();                                                                  \
+            }                                                                                              \
+        }                                                                                                  \
         if (a.stream == kStreamStores)                                                                     \
             fft_uniform<TYPE, radices<__VA_ARGS__>, E, T, PS, kStreamStores>                               \
                 <<<dim3((unsigned)nblocks), dim3((N / E) * T), 0, s>>>(a);                                 \

@@ -165,7 +165,7 @@ void batch_plan::prepare(bool dbl) {
             mtoff.push_back((int)mtab.size());
             const int n = lengths_[l];
             if (n > 1 && 2 * (size_t)n * elem <= (size_t)kGenericMaxLds)
-                g = make_mixed(n, dbl, false, false, false, 0, 0).plan;
+                g = make_mixed(n, dbl, false, true, true, 0, 0).plan;
             if (g.chirp || g.direct) g = mixed_plan{};
             if (g.n > 1) {
                 const std::vector<unsigned char> t = mixed_table(g, dbl, 1);

@@ -81,7 +81,7 @@ fast_div make_div(unsigned d) {
 // k_0 m_0 pitch + k_0 pad + (rest); the LDS serves `group` lanes at once from
 // `group` element slots (32 of 8 bytes over its 64 banks, 16 of 16 bytes).
 int read_conflicts(const mixed_plan &g, int pad, int group) {
-    const int nb = g.n / g.last, lanes = std::min(nb, 4 * group);
+    const int nb = g.n / g.last, lanes = std::min(nb, 2 * group);
     int total = 0;
     for (int u0 = 0; u0 < lanes; u0 += group) {
         int used[32] = {}, worst = 0;
@@ -249,7 +249,8 @@ plane_config make_plane(int n0, int n1, long long nplanes, bool dbl) {
     if (n0 < 2 || n1 < 2 || n0 > kPlaneMaxSide || n1 > kPlaneMaxSide) return c;
     const long long elem = dbl ? 16 : 8, rp = n0 | 1, ps = rp * n1;
     if (ps * elem > kPlaneBytes) return c;
-    const mixed_config c0 = make_mixed(n0, dbl, false, false, false, 0, 0), c1 = make_mixed(n1, dbl, false, false, false, 0, 0);
+    // (only the radix plans are used: the orientation with the least work)
+    const mixed_config c0 = make_mixed(n0, dbl, false, true, true, 0, 0), c1 = make_mixed(n1, dbl, false, true, true, 0, 0);
     if (!c0.ok || !c1.ok) return c;
     plane_args &a = c.args;
     a.g0 = c0.plan;
@@ -319,9 +320,13 @@ std::vector<unsigned char> mixed_table(const mixed_plan &g, bool dbl, long long 
             std::memcpy(&out[at], v, sizeof(v));
         }
     };
-    std::vector<cld> wn;
-    if (g.nst > 1)
-        for (int t = 0; t < g.n; t++) wn.push_back(root(t, g.n));
+    // w_n^t, the upper half and (n even) the second quarter by symmetry
+    std::vector<cld> wn(g.nst > 1 ? g.n : 0);
+    for (int t = 0; t < (int)wn.size(); t++) {
+        if (2 * t > g.n) wn[t] = std::conj(wn[g.n - t]);
+        else if (g.n % 2 == 0 && 4 * t > g.n) wn[t] = -std::conj(wn[g.n / 2 - t]);
+        else wn[t] = root(t, g.n);
+    }
     long long len = g.n, off = 0, blocks = 1;
     for (int s = 0; s < g.nst; s++) {
         const int r = g.radix[s];

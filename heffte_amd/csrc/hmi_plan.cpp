@@ -243,6 +243,8 @@ exec_plan fft_plan::build(int dir, bool dbl, bool in_real, bool out_real, bool i
                 buf cur_buf = buf::in;
                 int lcode = li, bcode = bi;
                 for (int i = 0; i < k && ok; i++) {
+                    // every pass still to come costs at least 1: no cheaper than the best one so far
+                    if (cost + (k - i) > best_cost + 1e-9) { ok = false; break; }
                     const candidate_pass &cp = seq[i];
                     pass p;
                     p.axis = cp.axis;
@@ -327,8 +329,6 @@ exec_plan fft_plan::build(int dir, bool dbl, bool in_real, bool out_real, bool i
                     if (!cp.identity && (p.load_colfast || p.store_colfast)) cost += narrow_chunk_cost(p, dbl);
                     // a copy pass runs one LDS tile per line: not along an axis too long for one
                     if (cp.identity) cost += 0.5 + (2 * dims[cp.axis] * (dbl ? 16 : 8) > kGenericMaxLds ? 100.0 : 0.0);
-                    // costs only grow along the sequence: not cheaper than the best one so far
-                    if (cost >= best_cost) { ok = false; break; }
                     ep.passes.push_back(p);
                     cur = p.lout;
                     cur_buf = p.dst;

@@ -27,7 +27,7 @@ bool is_permutation(const int o[3]) {
 
 const int kOrders[6][3] = {{0, 1, 2}, {0, 2, 1}, {1, 0, 2}, {1, 2, 0}, {2, 0, 1}, {2, 1, 0}};
 
-// Radix decomposition of the generic pass: 8s, then 4, 2, then odd primes.
+// Radix decomposition of the batched kernel's runtime-plan tile: 8s, then 4, 2, then odd primes.
 std::vector<int> factorize(int n) {
     std::vector<int> r;
     int m = n;
@@ -365,6 +365,8 @@ exec_plan fft_plan::build(int dir, bool dbl, bool in_real, bool out_real, bool i
     } while (std::next_permutation(perm.begin(), perm.end()));
     if (!std::isfinite(best_cost)) throw std::runtime_error("no valid pass schedule for these boxes");
 
+    const long long axes_ws = best.ws_elems;
+
     // The two fastest axes in one fused pass where a plane fits the LDS: same layout on both sides and
     // plain complex data, so the passes are (fastest two: in -> out), (slowest: out, in place).
     const int *o = bin.order;
@@ -408,6 +410,7 @@ exec_plan fft_plan::build(int dir, bool dbl, bool in_real, bool out_real, bool i
             split_elems = std::max(split_elems, p.lin.n[0] * p.lin.n[1] * p.lin.n[2]);
         }
     best.ws_elems += split_elems;
+    best.limit_elems = axes_ws + split_elems;
     return best;
 }
 
@@ -836,7 +839,8 @@ void fft_plan::launch_plane(const pass &p, const pass_args &base, const void *ta
     a.tw0 = base.tw;
     a.tw1 = table1;
     const long long nplanes = p.lin.n[p.b1] * batch;
-    if (nplanes > 0x7fffffffLL) throw std::runtime_error("too many planes in one pass");
+    // the limit on lines of one-axis passes, for either axis of the planes
+    if (nplanes * std::max(a.n0, a.n1) > 0x7fffffffLL) throw std::runtime_error("too many lines in one pass");
     a.nplanes = (int)nplanes;
     a.conj = base.conj;
     a.stream = base.stream;
@@ -869,12 +873,12 @@ void fft_plan::execute(int dir, bool dbl, bool in_real, bool out_real, int batch
     if (no_alloc) {
         // the workspace is the static scratch of this device (one per GPU, shared by every call)
         if (ws) throw std::invalid_argument("the no-allocation call takes no workspace (it uses the static scratch)");
-        const unsigned long long need = (unsigned long long)ep.ws_elems * (unsigned long long)batch * (dbl ? 16 : 8);
+        const unsigned long long need = (unsigned long long)ep.limit_elems * (unsigned long long)batch * (dbl ? 16 : 8);
         if (need > kScratchBytes)
             throw std::invalid_argument("the workspace of this call (" + std::to_string(need) +
                                         " bytes) exceeds the static scratch of the no-allocation entry point (" +
                                         std::to_string(kScratchBytes) + " bytes)");
-        if (need > 0) ws = scratch_address();
+        if (ep.ws_elems > 0) ws = scratch_address();
     }
     // the device tables must be resident before anything is launched when the call may not
     // allocate: look them all up first (a missing one throws here, with nothing enqueued)

@@ -97,6 +97,9 @@ struct pass {
 struct exec_plan {
     std::vector<pass> passes;
     long long ws_elems = 0;  // workspace needed per transform, in complex elements
+    // what one pass per axis would need: the scratch limit of the no-allocation call counts this, so
+    // whether a call fits does not depend on which passes are fused
+    long long limit_elems = 0;
 };
 
 // Device twiddle tables for one length and precision.

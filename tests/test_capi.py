@@ -241,3 +241,24 @@ def test_matrix_core_pass_count(hmi):
     assert (m, t) == (1, 3)
     with pytest.raises(hmi.heffte_input_error):
         plan.matrix_core_passes(0)
+
+
+@pytest.mark.parametrize("size", [(64, 64, 64), (90, 100, 108), (128, 128, 16), (2, 256, 33), (100, 64, 9000)])
+@pytest.mark.parametrize("dbl", [0, 1])
+def test_scratch_limit_does_not_depend_on_fused_passes(hmi, size, dbl):
+    # one layout on both sides: the fused two-axis pass needs no workspace, yet the no-allocation call
+    # takes exactly the batches whose batch * size_workspace fits its 64 MiB.  Every call is refused before
+    # a launch (no table is resident), so the arrays are never touched.
+    box = hmi.box3d([0, 0, 0], [s - 1 for s in size])
+    plan = hmi.fft3d(hmi.backend.mi355, box, box)
+    need = plan.size_workspace() * (16 if dbl else 8)
+    fits = (64 << 20) // need
+    x, y = ctypes.c_void_p(1 << 20), ctypes.c_void_p(1 << 40)
+    call = hmi.lib.heffte_mi355_execute_c2c_noalloc
+    for direction in (-1, 1):
+        for out in (x, y):
+            assert call(plan._h, direction, dbl, fits + 1, x, out, 0) != 0
+            assert "exceeds the static scratch" in hmi.last_error()
+            if fits > 0:
+                assert call(plan._h, direction, dbl, fits, x, out, 0) != 0
+                assert "static scratch" not in hmi.last_error()

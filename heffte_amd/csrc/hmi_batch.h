@@ -1,8 +1,9 @@
 // Batch of independent c2c 3D transforms of different sizes, run as phases over device work
-// lists (one launch per register class of tile), optionally replayed from a captured hipGraph:
-// the fused x-y phase for the transforms whose planes and tiles allow it, the x and y phases for
-// the others, then the z phase for all.  There is no counterpart in heFFTe, whose
-// batches share one geometry (include/heffte_fft3d.h:392-402).
+// lists (one launch per block size, or per register class of tile), optionally replayed from a
+// captured hipGraph: the fused x-y phase for the transforms whose planes and lengths allow it, the
+// x and y phases for the others, then the column-block z phase or, for lengths with large primes,
+// the tiled one.  There is no counterpart in heFFTe, whose batches share one geometry
+// (include/heffte_fft3d.h:392-402).
 #pragma once
 #include <hip/hip_runtime.h>
 

@@ -6,8 +6,8 @@
 //    one used for the global store are chosen independently (walk the FFT axis
 //    or walk the column axis), which is how a layout permutation is fused into
 //    a pass with coalesced HBM traffic on both sides.
-//  * fft_generic<R>: runtime radix plan (any length whose tile fits in LDS,
-//    any prime factor), Stockham ping-pong in LDS.
+//  * fft_batched<R>: one axis of a mixed-size batch over a device work list, by compile-time tiles or a
+//    runtime radix plan (generic_tile: Stockham ping-pong in LDS).
 //  * permute_kernel: heFFTe's in-node reshape (transpose_unpacker,
 //    src/heffte_backend_rocm.hip.cpp:91-134) as an LDS-tiled permutation.
 //
@@ -464,7 +464,7 @@ __global__ void __launch_bounds__((RL::n() / E) * T) fft_uniform(pass_args a) {
     uniform_tile<R, RL, E, T, PS, NTM>(a, tile, lds);
 }
 
-// ---------------------------------------------------------------- generic pass
+// ------------------------------------------- runtime-plan tile of the batched kernel
 
 template <int R, typename C>
 __device__ __forceinline__ void generic_bfly(const C *sp, int istride, C *dp, int ostride, const C *w, bool twiddle) {

@@ -67,7 +67,7 @@ struct pass_args {
     int tw4_dim;
 };
 
-// Runtime radix plan used by the generic (any length) pass.
+// Runtime radix plan of the batched kernel's runtime-plan tile (any length).
 struct generic_plan {
     int n;
     int nstages;

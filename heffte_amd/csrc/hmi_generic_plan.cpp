@@ -256,30 +256,56 @@ plane_config make_plane(int n0, int n1, long long nplanes, bool dbl) {
     a.g0 = c0.plan;
     a.g1 = c1.plan;
     if (a.g0.chirp || a.g0.direct || a.g1.chirp || a.g1.direct) return c;
-    // planes per block: up to kPlaneTile bytes, as long as the launch keeps kFewBlocks blocks
-    int planes = 1;
-    while (2 * planes * ps * elem <= kPlaneTile && nplanes / (2 * planes) >= kFewBlocks) planes *= 2;
     a.n0 = n0;
     a.n1 = n1;
-    a.planes = planes;
     a.rp = (int)rp;
     a.ps = (int)ps;
-    a.rows = (unsigned)(planes * n1);
-    a.cols = (unsigned)(planes * n0);
+    a.by_n0 = make_div((unsigned)n0);
+    c.ok = true;
+    group_planes(c, nplanes, dbl);
+    return c;
+}
+
+void group_planes(plane_config &c, long long nplanes, bool dbl) {
+    plane_args &a = c.args;
+    const long long elem = dbl ? 16 : 8;
+    // planes per block: up to kPlaneTile bytes, as long as the launch keeps kFewBlocks blocks
+    int planes = 1;
+    while (2 * planes * a.ps * elem <= kPlaneTile && nplanes / (2 * planes) >= kFewBlocks) planes *= 2;
+    a.planes = planes;
+    a.rows = (unsigned)(planes * a.n1);
+    a.cols = (unsigned)(planes * a.n0);
     a.by_rows = make_div(a.rows);
     a.by_cols = make_div(a.cols);
-    a.by_n0 = make_div((unsigned)n0);
-    c.lds = (size_t)(planes * ps * elem);
+    a.nplanes = (int)nplanes;
+    c.lds = (size_t)(planes * a.ps * elem);
+    c.nblocks = (nplanes + planes - 1) / planes;
     // threads: about one round of the smallest stage, whole sets of four waves above 256
     int top = 2;
     for (const mixed_plan *g : {&a.g0, &a.g1})
         for (int s = 0; s < g->nst; s++) top = std::max(top, g->radix[s]);
-    const long long units = (long long)planes * n0 * n1 / top;
+    const long long units = (long long)planes * a.n0 * a.n1 / top;
     c.threads = 64;
     while (c.threads < 256 && c.threads < units) c.threads += 64;
     if (units > 256 + 64) c.threads = kMixedThreads;
-    c.ok = true;
-    return c;
+    c.threads = launch_threads(c.threads, c.nblocks);
+}
+
+// A plane of more than 64 KiB has a CU to itself, and a launch of few of them leaves most CUs idle
+// while one pass per axis spreads their lines.  One pass for both axes over one pass for each, us of a
+// whole transform, complex<float> 128 x 128 x 1 12.7 / 8.8, x 64 22.3 / 21.3, x 128 25.2 / 27.5; 200 x 100 x 64
+// 28.2 / 25.1, x 128 32.9 / 34.4; 100 x 100 x 8 12.1 / 11.5, x 32 13.7 / 13.8; complex<double> 100 x 100 x 32
+// 19.5 / 18.8, x 64 23.3 / 25.0; 80 x 80 x 16 14.3 / 13.3, x 32 15.1 / 15.7; 64 x 64 (65 KiB) x 1 7.0 / 7.0, x 4
+// 10.5 / 10.4, x 32 11.5 / 12.9.  Planes of 64 KiB and less win from the first one on (64 x 64 x 1 complex<float>
+// 5.2 / 7.0).
+long long min_planes(int n0, int n1, bool dbl) {
+    const long long elem = dbl ? 16 : 8, above = (long long)(n0 | 1) * n1 - 64 * 1024 / elem;
+    return above <= 0 ? 1 : 1 + above / 96;
+}
+
+int launch_threads(int threads, long long nblocks) {
+    while (threads > 64 && nblocks * threads > 0xffffffffLL) threads -= 64;
+    return threads;
 }
 
 fast_div make_fast_div(unsigned d) { return make_div(d); }

@@ -128,7 +128,7 @@ fft_plan::fft_plan(kind k, const box3 &inbox, const box3 &outbox, int r2c_dir)
     long long ws = 0;
     // (a length may be split in one precision only: lines of complex<double> fill LDS sooner)
     for (bool dbl : {false, true})
-        for_each_variant([&](int dir, bool ir, bool orl, bool ip) { ws = std::max(ws, build(dir, dbl, ir, orl, ip, true).ws_elems); });
+        for_each_variant([&](int dir, bool ir, bool orl, bool ip) { ws = std::max(ws, build(dir, dbl, ir, orl, ip, true).axes.ws_elems); });
     ws_elems_ = ws;
 }
 
@@ -149,21 +149,12 @@ template <typename F> void fft_plan::for_each_variant(F &&f) const {
 
 void fft_plan::prepare(bool dbl) {
     for_each_variant([&](int dir, bool ir, bool orl, bool ip) {
-        const exec_plan &ep = get_exec_plan(dir, dbl, ir, orl, ip);
-        for (const pass &p : ep.passes) {
-            if (p.plane) {
-                for (const mixed_plan *g : {&p.plane->args.g0, &p.plane->args.g1}) (void)get_plane_table(dbl, *g, true);
-            } else if (p.split) {
-                for (const pass &q : *p.split) (void)get_twiddles(dbl, q, true);
-                (void)get_split_table(dbl, p.n, true);
-            } else {
-                (void)get_twiddles(dbl, p, true);
-            }
-        }
+        const exec_choice &c = get_choice(dir, dbl, ir, orl, ip);
+        upload_tables(c, dbl, [](const pass &) { return false; });
     });
     if (!dbl && precision_ != kPrecPlain && kind_ == kind::c2c) {
-        (void)get_mfma_table(precision_, false, true);
-        (void)get_mfma_table(precision_, true, true);
+        upload_mfma_table(precision_, false);
+        upload_mfma_table(precision_, true);
     }
 }
 
@@ -191,7 +182,7 @@ double fft_plan::scale_factor(int scaling) const {
     return s;
 }
 
-const exec_plan &fft_plan::get_exec_plan(int dir, bool dbl, bool in_real, bool out_real, bool in_place) {
+const exec_choice &fft_plan::get_choice(int dir, bool dbl, bool in_real, bool out_real, bool in_place) {
     const int key = ((dir > 0) << 4) | (dbl << 3) | (in_real << 2) | (out_real << 1) | (int)in_place;
     std::lock_guard<std::mutex> lock(mtx_);
     auto it = plans_.find(key);
@@ -199,7 +190,11 @@ const exec_plan &fft_plan::get_exec_plan(int dir, bool dbl, bool in_real, bool o
     return it->second;
 }
 
-exec_plan fft_plan::build(int dir, bool dbl, bool in_real, bool out_real, bool in_place, bool sizes_only) const {
+const exec_plan &fft_plan::get_exec_plan(int dir, bool dbl, bool in_real, bool out_real, bool in_place, long long batch) {
+    return get_choice(dir, dbl, in_real, out_real, in_place).pick(batch);
+}
+
+exec_choice fft_plan::build(int dir, bool dbl, bool in_real, bool out_real, bool in_place, bool sizes_only) const {
     const bool fwd = dir < 0;
     const box3 &bin = fwd ? inbox_ : outbox_;
     const box3 &bout = fwd ? outbox_ : inbox_;
@@ -365,14 +360,16 @@ exec_plan fft_plan::build(int dir, bool dbl, bool in_real, bool out_real, bool i
     } while (std::next_permutation(perm.begin(), perm.end()));
     if (!std::isfinite(best_cost)) throw std::runtime_error("no valid pass schedule for these boxes");
 
-    const long long axes_ws = best.ws_elems;
+    exec_choice c;
+    finish(best, dbl, sizes_only);
+    c.axes = best;
 
     // The two fastest axes in one fused pass where a plane fits the LDS: same layout on both sides and
     // plain complex data, so the passes are (fastest two: in -> out), (slowest: out, in place).
     const int *o = bin.order;
     if (!sizes_only && kind_ == kind::c2c && !in_real && !out_real && std::equal(o, o + 3, bout.order) && nin[o[0]] > 1 &&
         nin[o[1]] > 1 && nin[o[0]] <= kPlaneMaxSide && nin[o[1]] <= kPlaneMaxSide) {
-        const plane_config c = make_plane((int)nin[o[0]], (int)nin[o[1]], nin[o[2]], dbl);
+        const plane_config pc = make_plane((int)nin[o[0]], (int)nin[o[1]], nin[o[2]], dbl);
         pass q;
         q.axis = o[2];
         q.col = o[0];
@@ -383,35 +380,38 @@ exec_plan fft_plan::build(int dir, bool dbl, bool in_real, bool out_real, bool i
         q.load_colfast = q.store_colfast = 1;
         q.last = true;
         // (a slowest axis with narrow column chunks is better off in the schedule above)
-        if (c.ok && narrow_chunk_cost(q, dbl) == 0.0) {
-            exec_plan ep;
+        if (pc.ok && narrow_chunk_cost(q, dbl) == 0.0) {
             pass p;
             p.axis = o[0];
-            p.plane_axis = o[1];
             p.col = o[1];
             p.b1 = o[2];
             p.n = p.store_len = (int)nin[o[0]];
             p.lin = Lin;
             p.lout = Lout;
             p.last = nin[o[2]] == 1;
-            p.plane = std::make_shared<plane_config>(c);
-            ep.passes.push_back(p);
-            if (!p.last) ep.passes.push_back(q);
-            best = ep;
+            p.plane = std::make_shared<plane_config>(pc);
+            c.fused.passes.push_back(p);
+            if (!p.last) c.fused.passes.push_back(q);
+            finish(c.fused, dbl, sizes_only);
+            c.fused.limit_elems = c.axes.limit_elems;
+            c.planes = nin[o[2]];
+            c.at_least = min_planes((int)nin[o[0]], (int)nin[o[1]], dbl);
         }
     }
+    return c;
+}
 
-    for (pass &p : best.passes) configure(p, dbl, sizes_only);
+void fft_plan::finish(exec_plan &ep, bool dbl, bool sizes_only) const {
+    for (pass &p : ep.passes) configure(p, dbl, sizes_only);
     // the step buffer of split axes follows the intermediate arrays in the workspace
     long long split_elems = 0;
-    for (pass &p : best.passes)
+    for (pass &p : ep.passes)
         if (p.split) {
-            p.split_ws = best.ws_elems;
+            p.split_ws = ep.ws_elems;
             split_elems = std::max(split_elems, p.lin.n[0] * p.lin.n[1] * p.lin.n[2]);
         }
-    best.ws_elems += split_elems;
-    best.limit_elems = axes_ws + split_elems;
-    return best;
+    ep.ws_elems += split_elems;
+    ep.limit_elems = ep.ws_elems;
 }
 
 void fft_plan::configure(pass &p, bool dbl, bool sizes_only) const {
@@ -612,81 +612,75 @@ std::string pass_kernel_name(const pass &p, bool dbl, bool mfma, int precision, 
 }
 }  // namespace
 
-const twiddles &fft_plan::get_twiddles(bool dbl, const pass &p, bool may_alloc) {
-    const int n = p.n;
-    const long long key = ((long long)n << 8) | (dbl ? 1 : 0) | (p.fast ? 2 : 0) | (p.identity ? 4 : 0) |
-                          ((long long)p.mode << 3) | (p.fast ? (long long)p.fast->T << 40 : 0);
-    std::lock_guard<std::mutex> lock(mtx_);
-    auto it = tw_.find(key);
-    if (it != tw_.end()) return it->second;
-    if (!may_alloc) throw std::runtime_error(kNotResident);
-    twiddles t;
+namespace {
+// Keys of the plan's device tables.  The table of a runtime-length complex pass depends on the length
+// alone, so the fused pass shares it; a split axis has bit 7 set, out of the range of the mode bits.
+long long mixed_key(bool dbl, int n) { return ((long long)n << 8) | (dbl ? 1 : 0); }
+long long pass_key(bool dbl, const pass &p) {
+    return mixed_key(dbl, p.n) | (p.fast ? 2 : 0) | (p.identity ? 4 : 0) | ((long long)p.mode << 3) |
+           (p.fast ? (long long)p.fast->T << 40 : 0);
+}
+long long split_key(bool dbl, int n) { return mixed_key(dbl, n) | 0x80; }
+
+template <typename R> std::vector<unsigned char> as_bytes(const std::vector<R> &v) {
+    const unsigned char *p = reinterpret_cast<const unsigned char *>(v.data());
+    return std::vector<unsigned char>(p, p + v.size() * sizeof(R));
+}
+
+std::vector<unsigned char> table_bytes(bool dbl, const int *radix, int nstages, int tail_count, long long tail_mod) {
+    return dbl ? as_bytes(make_table<double>(radix, nstages, false, tail_count, tail_mod))
+               : as_bytes(make_table<float>(radix, nstages, false, tail_count, tail_mod));
+}
+
+std::vector<unsigned char> pass_table(bool dbl, const pass &p) {
     // r2c / c2r: w_n^k for k < n/2 (n = real line length); r2r: w_{4n}^k for k < n
     int tail_count = 0;
     long long tail_mod = 1;
-    if (p.mode == kModeR2C || p.mode == kModeC2R) { tail_count = n / 2; tail_mod = n; }
-    if (p.mode >= kModeDCT2 && p.mode <= kModeDST3) { tail_count = n; tail_mod = 4LL * n; }
-    if (p.mixed) {
-        const std::vector<unsigned char> v = mixed_table((*p.mixed)[0].plan, dbl, tail_mod);
+    if (p.mode == kModeR2C || p.mode == kModeC2R) { tail_count = p.n / 2; tail_mod = p.n; }
+    if (p.mode >= kModeDCT2 && p.mode <= kModeDST3) { tail_count = p.n; tail_mod = 4LL * p.n; }
+    if (p.mixed) return mixed_table((*p.mixed)[0].plan, dbl, tail_mod);
+    return table_bytes(dbl, p.fast->radix, p.fast->nstages, tail_count, tail_mod);
+}
+}  // namespace
+
+const void *fft_plan::find_table(long long key) const {
+    auto it = tw_.find(key);
+    return it == tw_.end() ? nullptr : it->second.dev;
+}
+
+void fft_plan::upload_tables(const exec_choice &c, bool dbl, const std::function<bool(const pass &)> &skip) {
+    std::lock_guard<std::mutex> lock(mtx_);
+    auto need = [&](long long key, auto &&bytes) {
+        if (tw_.count(key)) return;
+        const std::vector<unsigned char> v = bytes();
+        twiddles t;
         t.bytes = v.size();
         t.dev = upload_bytes(v.data(), t.bytes);
-    } else if (dbl) {
-        std::vector<double> v = make_table<double>(p.fast->radix, p.fast->nstages, false, tail_count, tail_mod);
-        t.bytes = v.size() * sizeof(double);
-        t.dev = upload_bytes(v.data(), t.bytes);
-    } else {
-        std::vector<float> v = make_table<float>(p.fast->radix, p.fast->nstages, false, tail_count, tail_mod);
-        t.bytes = v.size() * sizeof(float);
-        t.dev = upload_bytes(v.data(), t.bytes);
-    }
-    return tw_.emplace(key, t).first->second;
+        tw_.emplace(key, t);
+    };
+    for (const exec_plan *ep : {&c.axes, &c.fused})
+        for (const pass &p : ep->passes) {
+            if (p.plane) {
+                for (const mixed_plan *g : {&p.plane->args.g0, &p.plane->args.g1})
+                    need(mixed_key(dbl, g->n), [&] { return mixed_table(*g, dbl, 1); });
+            } else if (p.split) {
+                for (const pass &q : *p.split) need(pass_key(dbl, q), [&] { return pass_table(dbl, q); });
+                // w_n^m, m < n
+                need(split_key(dbl, p.n), [&] { return table_bytes(dbl, nullptr, 0, p.n, p.n); });
+            } else if (!skip(p)) {
+                need(pass_key(dbl, p), [&] { return pass_table(dbl, p); });
+            }
+        }
 }
 
-const twiddles &fft_plan::get_plane_table(bool dbl, const mixed_plan &g, bool may_alloc) {
-    // (bit 57: the runtime-length table of a length that may have a compile-time tile as well)
-    const long long key = ((long long)g.n << 8) | (dbl ? 1 : 0) | (1LL << 57);
-    std::lock_guard<std::mutex> lock(mtx_);
-    auto it = tw_.find(key);
-    if (it != tw_.end()) return it->second;
-    if (!may_alloc) throw std::runtime_error(kNotResident);
-    const std::vector<unsigned char> v = mixed_table(g, dbl, 1);
-    twiddles t;
-    t.bytes = v.size();
-    t.dev = upload_bytes(v.data(), t.bytes);
-    return tw_.emplace(key, t).first->second;
-}
-
-const twiddles &fft_plan::get_mfma_table(int prec, bool conj, bool may_alloc) {
+void fft_plan::upload_mfma_table(int prec, bool conj) {
     // W512 and the split W32 / W16 operand tables of one precision form and direction
     std::lock_guard<std::mutex> lock(mtx_);
-    twiddles &mt = mfma_tw_[prec == kSplitF16 ? 0 : 1][conj ? 1 : 0];
-    if (!mt.dev) {
-        if (!may_alloc) throw std::runtime_error(kNotResident);
-        std::vector<unsigned char> t = mfma512_operand_table(prec, conj);
-        mt.dev = upload_bytes(t.data(), t.size());
-        mt.bytes = t.size();
-    }
-    return mt;
-}
-
-const twiddles &fft_plan::get_split_table(bool dbl, int n, bool may_alloc) {
-    // w_n^m, m < n, of a split axis (key: bit 7 set, out of the range of the pass keys' mode bits)
-    const long long key = ((long long)n << 8) | (dbl ? 1 : 0) | 0x80;
-    std::lock_guard<std::mutex> lock(mtx_);
-    auto it = tw_.find(key);
-    if (it != tw_.end()) return it->second;
-    if (!may_alloc) throw std::runtime_error(kNotResident);
-    twiddles t;
-    if (dbl) {
-        std::vector<double> v = make_table<double>(nullptr, 0, false, n, n);
-        t.bytes = v.size() * sizeof(double);
-        t.dev = upload_bytes(v.data(), t.bytes);
-    } else {
-        std::vector<float> v = make_table<float>(nullptr, 0, false, n, n);
-        t.bytes = v.size() * sizeof(float);
-        t.dev = upload_bytes(v.data(), t.bytes);
-    }
-    return tw_.emplace(key, t).first->second;
+    twiddles &mt = mfma_table(prec, conj);
+    if (mt.dev) return;
+    std::vector<unsigned char> t = mfma512_operand_table(prec, conj);
+    mt.dev = upload_bytes(t.data(), t.size());
+    mt.bytes = t.size();
 }
 
 pass_args pass_launch_args(kind k, const exec_plan &ep, const pass &p, int dir, bool dbl, int batch, const void *in,
@@ -826,37 +820,42 @@ void launch_mixed_pass(const pass &p, const pass_args &a, bool dbl, hipStream_t 
     mixed_plan g = c->plan;
     mixed_launch_divs(g, a);
     const long long nblocks = ((long long)a.nlines + (1 << g.log2t) - 1) >> g.log2t;
-    check_hip(launch_mixed(dbl, a, g, c->threads, nblocks, c->lds, s), "runtime-length FFT pass");
+    check_hip(launch_mixed(dbl, a, g, launch_threads(c->threads, nblocks), nblocks, c->lds, s), "runtime-length FFT pass");
 }
 }  // namespace
 
 void fft_plan::launch_plane(const pass &p, const pass_args &base, const void *table1, bool dbl, int batch) {
-    const plane_config &c = *p.plane;
-    plane_args a = c.args;
+    plane_config c = *p.plane;
+    plane_args &a = c.args;
+    const long long nplanes = p.lin.n[p.b1] * batch;
+    // the limit on lines of one-axis passes, for either axis of the planes
+    if (nplanes * std::max(a.n0, a.n1) > 0x7fffffffLL) throw std::runtime_error("too many lines in one pass");
+    if (batch > 1) group_planes(c, nplanes, dbl);  // (planned for the planes of one transform)
     a.in = base.in;
     a.out = base.out;
     a.mul = base.mul;
     a.tw0 = base.tw;
     a.tw1 = table1;
-    const long long nplanes = p.lin.n[p.b1] * batch;
-    // the limit on lines of one-axis passes, for either axis of the planes
-    if (nplanes * std::max(a.n0, a.n1) > 0x7fffffffLL) throw std::runtime_error("too many lines in one pass");
-    a.nplanes = (int)nplanes;
     a.conj = base.conj;
     a.stream = base.stream;
     a.scale = base.scale;
-    const long long nblocks = (nplanes + a.planes - 1) / a.planes;
-    check_hip((dbl ? launch_plane_f64 : launch_plane_f32)(a, c.threads, nblocks, c.lds, stream_), "fused two-axis FFT pass");
+    check_hip((dbl ? launch_plane_f64 : launch_plane_f32)(a, c.threads, c.nblocks, c.lds, stream_), "fused two-axis FFT pass");
 }
 
 void fft_plan::launch_split(const pass &p, const pass_args &base, bool dbl, int batch, void *tmp) {
+    const void *step_w[2], *split_w;
+    {
+        std::lock_guard<std::mutex> lock(mtx_);
+        split_w = find_table(split_key(dbl, p.n));
+        for (int i = 0; i < 2; i++) step_w[i] = find_table(pass_key(dbl, (*p.split)[i]));
+    }
     for (int bt = 0; bt < batch; bt++) {
         pass_args st[2];
         split_steps(p, base, dbl, bt, tmp, st);
-        st[0].tw4 = get_split_table(dbl, p.n, false).dev;
+        st[0].tw4 = split_w;
         for (int i = 0; i < 2; i++) {
             const pass &q = (*p.split)[i];
-            st[i].tw = get_twiddles(dbl, q, false).dev;
+            st[i].tw = step_w[i];
             const long long nblocks = ((long long)st[i].nlines + q.lines - 1) / q.lines;
             if (q.fast) check_hip(q.fast->launch(st[i], nblocks, stream_), "split FFT pass");
             else launch_mixed_pass(q, st[i], dbl, stream_);
@@ -869,7 +868,8 @@ void fft_plan::execute(int dir, bool dbl, bool in_real, bool out_real, int batch
     if (batch < 1) throw std::invalid_argument("batch size must be positive");
     if (!in || !out) throw std::invalid_argument("null input or output array");
     const bool in_place = (in == out);
-    const exec_plan &ep = get_exec_plan(dir, dbl, in_real, out_real, in_place);
+    const exec_choice &choice = get_choice(dir, dbl, in_real, out_real, in_place);
+    const exec_plan &ep = choice.pick(batch);
     if (no_alloc) {
         // the workspace is the static scratch of this device (one per GPU, shared by every call)
         if (ws) throw std::invalid_argument("the no-allocation call takes no workspace (it uses the static scratch)");
@@ -892,21 +892,38 @@ void fft_plan::execute(int dir, bool dbl, bool in_real, bool out_real, int batch
     if (ep.passes.size() > kMaxPasses) throw std::runtime_error("internal error: too many passes");
     std::array<const void *, kMaxPasses> tables{};
     const void *second_table = nullptr;
-    for (size_t i = 0; i < ep.passes.size(); i++) {
-        const pass &p = ep.passes[i];
-        const bool mfma = split && p.n == 512 && p.mode == kModeC2C && !p.identity && !p.in_real && !p.out_real &&
-                          !p.herm_load && p.store_len == p.n && !(mul && i == 0);
-        if (p.plane) {
-            // both axes' tables (at most one pass of a plan is fused)
-            tables[i] = get_plane_table(dbl, p.plane->args.g0, may_alloc).dev;
-            second_table = get_plane_table(dbl, p.plane->args.g1, may_alloc).dev;
-        } else if (p.split) {
-            // both steps' tables and the step twiddles, looked up now (launch_split uses them)
-            for (const pass &q : *p.split) (void)get_twiddles(dbl, q, may_alloc);
-            tables[i] = get_split_table(dbl, p.n, may_alloc).dev;
-        } else {
-            tables[i] = mfma ? get_mfma_table(precision_, dir > 0, may_alloc).dev : get_twiddles(dbl, p, may_alloc).dev;
+    auto on_mfma = [&](const pass &p) {
+        return split && p.n == 512 && p.mode == kModeC2C && !p.identity && !p.in_real && !p.out_real && !p.herm_load &&
+               p.store_len == p.n && !(mul && p.src == buf::in);
+    };
+    auto resident = [&] {
+        std::lock_guard<std::mutex> lock(mtx_);
+        bool all = true;
+        for (size_t i = 0; i < ep.passes.size(); i++) {
+            const pass &p = ep.passes[i];
+            if (p.plane) {
+                // both axes' tables (at most one pass of a plan is fused)
+                tables[i] = find_table(mixed_key(dbl, p.plane->args.g0.n));
+                second_table = find_table(mixed_key(dbl, p.plane->args.g1.n));
+                all = all && second_table;
+            } else if (p.split) {
+                // the steps' tables too (launch_split looks them up again)
+                tables[i] = find_table(split_key(dbl, p.n));
+                for (const pass &q : *p.split) all = all && find_table(pass_key(dbl, q));
+            } else {
+                tables[i] = on_mfma(p) ? mfma_table(precision_, dir > 0).dev : find_table(pass_key(dbl, p));
+            }
+            all = all && tables[i];
         }
+        return all;
+    };
+    if (!resident()) {
+        if (!may_alloc) throw std::runtime_error(kNotResident);
+        // the tables of either schedule, so that a later call over another batch finds them
+        bool mfma = false;
+        upload_tables(choice, dbl, [&](const pass &p) { const bool m = on_mfma(p); mfma = mfma || m; return m; });
+        if (mfma) upload_mfma_table(precision_, dir > 0);
+        if (!resident()) throw std::runtime_error("internal error: a table of the plan is missing");
     }
     void *tmp = nullptr;
     if (ep.ws_elems > 0 && !ws) {
@@ -952,8 +969,7 @@ void fft_plan::execute(int dir, bool dbl, bool in_real, bool out_real, int batch
         pass_args a = pass_launch_args(kind_, ep, p, dir, dbl, batch, in, out, ws, tables[&p - &ep.passes.front()],
                                        scale, mul);
         const long long nblocks = ((long long)a.nlines + p.lines - 1) / p.lines;
-        const bool mfma = split && p.n == 512 && p.mode == kModeC2C && !p.identity && !p.in_real && !p.out_real &&
-                          !p.herm_load && p.store_len == p.n && !a.mul;
+        const bool mfma = on_mfma(p);
         if (p.plane) {
             launch_plane(p, a, second_table, dbl, batch);
         } else if (p.split) {

@@ -10,6 +10,7 @@
 #include <hip/hip_runtime.h>
 
 #include <array>
+#include <functional>
 #include <map>
 #include <memory>
 #include <mutex>
@@ -59,9 +60,10 @@ struct mixed_config {
 // Tile and block of the fused pass over the two fastest axes.
 struct plane_config {
     bool ok = false;
-    plane_args args{};  // radix plans, extents and strides; pointers and counts are set at the launch
+    plane_args args{};  // radix plans, extents and strides; group_planes sets the counts, a launch the pointers
     int threads = 64;
     size_t lds = 0;
+    long long nblocks = 0;
 };
 
 struct pass {
@@ -80,9 +82,8 @@ struct pass {
     // set: the runtime-length pass runs it, with the second tile where a launch's lines are few
     std::shared_ptr<const std::array<mixed_config, 2>> mixed;
     int lines = 1;  // lines (columns) per block
-    // set: axis and plane_axis (the two fastest axes of lin = lout) run as one fused pass
+    // set: axis and col (the two fastest axes of lin = lout) run as one fused pass
     std::shared_ptr<const plane_config> plane;
-    int plane_axis = -1;
     // A length whose line does not fit one LDS tile runs as two passes (four-step), n = n1 n2,
     // position j = n2 j1 + j2, bin k = k1 + n1 k2: the first step takes the n1-point lines of
     // stride n2 (one per j2) into a buffer of the pass's input layout at position n2 k1 + j2,
@@ -100,6 +101,16 @@ struct exec_plan {
     // what one pass per axis would need: the scratch limit of the no-allocation call counts this, so
     // whether a call fits does not depend on which passes are fused
     long long limit_elems = 0;
+};
+
+// The schedules of one variant of a plan.
+struct exec_choice {
+    exec_plan axes;   // one pass per axis
+    exec_plan fused;  // the two fastest axes in one pass (no passes: not taken)
+    long long planes = 0, at_least = 0;  // of one transform; of a launch that takes the fused schedule
+    const exec_plan &pick(long long batch) const {
+        return !fused.passes.empty() && planes * batch >= at_least ? fused : axes;
+    }
 };
 
 // Device twiddle tables for one length and precision.
@@ -152,8 +163,8 @@ class fft_plan {
     // ws holds batch * size_workspace() elements or is null; out must not alias yhat.
     void convolve_spectrum(bool dbl, int batch, const void *x, const void *yhat, void *out, void *ws, int scaling);
 
-    // Plan (without running it): exposed for tests of the planner.
-    const exec_plan &get_exec_plan(int dir, bool dbl, bool in_real, bool out_real, bool in_place);
+    // Plan of a call over `batch` transforms (without running it): exposed for tests of the planner.
+    const exec_plan &get_exec_plan(int dir, bool dbl, bool in_real, bool out_real, bool in_place, long long batch = 1);
 
     // Per-pass timing: while on, every call records a hipEvent on the plan's stream before its
     // first pass and after each pass, so the time between two consecutive events is the
@@ -165,14 +176,18 @@ class fft_plan {
 
   private:
     // sizes_only: enough of the plan for its workspace (the constructor asks for every variant's)
-    exec_plan build(int dir, bool dbl, bool in_real, bool out_real, bool in_place, bool sizes_only = false) const;
+    exec_choice build(int dir, bool dbl, bool in_real, bool out_real, bool in_place, bool sizes_only = false) const;
+    void finish(exec_plan &ep, bool dbl, bool sizes_only) const;
     void configure(pass &p, bool dbl, bool sizes_only = false) const;
-    const twiddles &get_twiddles(bool dbl, const pass &p, bool may_alloc);
-    const twiddles &get_plane_table(bool dbl, const mixed_plan &g, bool may_alloc);
-    const twiddles &get_split_table(bool dbl, int n, bool may_alloc);
+    const exec_choice &get_choice(int dir, bool dbl, bool in_real, bool out_real, bool in_place);
+    // device table by its key (null: not resident; the caller holds mtx_); uploads what both schedules
+    // of a variant need, without the passes that skip() names
+    const void *find_table(long long key) const;
+    void upload_tables(const exec_choice &c, bool dbl, const std::function<bool(const pass &)> &skip);
     void launch_plane(const pass &p, const pass_args &base, const void *table1, bool dbl, int batch);
     void launch_split(const pass &p, const pass_args &base, bool dbl, int batch, void *tmp);
-    const twiddles &get_mfma_table(int prec, bool conj, bool may_alloc);
+    twiddles &mfma_table(int prec, bool conj) { return mfma_tw_[prec == kSplitF16 ? 0 : 1][conj ? 1 : 0]; }
+    void upload_mfma_table(int prec, bool conj);
     template <typename F> void for_each_variant(F &&f) const;
 
     kind kind_;
@@ -183,7 +198,7 @@ class fft_plan {
     int precision_ = kPrecPlain;
     std::mutex mtx_;
     twiddles mfma_tw_[2][2] = {};  // [split FP16, split BF16][forward, backward]
-    std::map<int, exec_plan> plans_;
+    std::map<int, exec_choice> plans_;
     std::map<long long, twiddles> tw_;
     // per-pass timing records: launch i ran between events marks_[i].first and .second
     // (a lock of their own: a timed call looks up tables while it records)
@@ -204,9 +219,16 @@ mixed_config make_mixed(int n, bool dbl, bool copy, bool load_across, bool store
                         int tail);
 int mixed_post_offset(const std::vector<int> &radices);
 std::vector<unsigned char> mixed_table(const mixed_plan &g, bool dbl, long long tail_mod);
-// Fused pass over planes of n0 x n1 elements (ok false: it does not take them), nplanes of them in one
-// transform.
+// Fused pass over planes of n0 x n1 elements (ok false: it does not take them), grouped for a launch of
+// nplanes of them.
 plane_config make_plane(int n0, int n1, long long nplanes, bool dbl);
+// Groups the planes of one launch (of a whole batch): planes and threads per block, blocks.
+void group_planes(plane_config &c, long long nplanes, bool dbl);
+// Planes a launch needs for the fused pass to beat one pass per axis.
+long long min_planes(int n0, int n1, bool dbl);
+// Largest count of threads per block, at most `threads`, with fewer than 2^32 in the grid (the kernels
+// walk their work with a stride of the block's threads, a multiple of 64).
+int launch_threads(int threads, long long nblocks);
 fast_div make_fast_div(unsigned d);
 // the divisors of one launch's line numbering
 void mixed_launch_divs(mixed_plan &g, const pass_args &a);

@@ -21,7 +21,9 @@ using cld = std::complex<long double>;
 
 template <typename R> bool run_case(int n0, int n1, int nplanes, bool inverse, int product, unsigned seed) {
     const bool dbl = sizeof(R) == 8;
-    const hmi::plane_config c = hmi::make_plane(n0, n1, nplanes, dbl);
+    // as a launch does: planned for the planes of one transform, grouped for those of the batch
+    hmi::plane_config c = hmi::make_plane(n0, n1, 1 + nplanes / 8, dbl);
+    if (c.ok) hmi::group_planes(c, nplanes, dbl);
     const std::string what = std::to_string(n0) + " x " + std::to_string(n1) + " planes " + std::to_string(nplanes) +
                              (dbl ? " f64" : " f32") + (inverse ? " inverse" : "") + " product " + std::to_string(product);
     if (!c.ok) { std::printf("FAIL %s: no plan\n", what.c_str()); return false; }
@@ -37,10 +39,9 @@ template <typename R> bool run_case(int n0, int n1, int nplanes, bool inverse, i
     hmi::plane_args a = c.args;
     a.in = in; a.out = out; a.tw0 = d0; a.tw1 = d1;
     a.mul = product == 0 ? nullptr : product == 1 ? (const void *)mul : in;
-    a.nplanes = nplanes;
     a.conj = inverse; a.scale = 0.5;
     auto kernel = hmi::plane_builds<R>::choose(a);
-    emulate::run_blocks((nplanes + a.planes - 1) / a.planes, c.threads, hmi::smem_raw, sizeof(hmi::smem_raw), c.lds,
+    emulate::run_blocks(c.nblocks, c.threads, hmi::smem_raw, sizeof(hmi::smem_raw), c.lds,
                         [&] { kernel(a); });
     const long double pi = 3.141592653589793238462643383279502884L;
     auto root = [&](long long t, long long n) {
@@ -80,10 +81,41 @@ template <typename R> bool run_case(int n0, int n1, int nplanes, bool inverse, i
     return true;
 }
 
+// The grid of any launch stays below 2^32 threads, and many small planes share blocks: nplanes as
+// many as the limit on lines of a pass, or the memory of one GPU, allows.
+int check_grids() {
+    int fails = 0;
+    for (bool dbl : {false, true})
+        for (int n0 = 2; n0 <= hmi::kPlaneMaxSide; n0++)
+            for (int n1 : {2, 3, 4, 5, 8, 10, 16, 24, 27, 45, 64, 77, 100, 128, 200, 256}) {
+                hmi::plane_config c = hmi::make_plane(n0, n1, 1, dbl);
+                if (!c.ok) continue;
+                const long long elem = dbl ? 16 : 8, most = std::min(0x7fffffffLL / std::max(n0, n1), (288LL << 30) / (elem * n0 * n1));
+                for (long long nplanes : {1LL, 255LL, 4096LL * n0, most}) {
+                    if (nplanes > most) continue;
+                    hmi::group_planes(c, nplanes, dbl);
+                    const long long bytes = (long long)c.args.ps * elem;
+                    const bool bad = c.nblocks * c.threads > 0xffffffffLL || c.threads < 64 || c.threads % 64 ||
+                                     c.nblocks * c.args.planes < nplanes || (c.nblocks - 1) * c.args.planes >= nplanes ||
+                                     c.lds != (size_t)(c.args.planes * bytes) ||
+                                     (nplanes >= 1LL << 20 && 2 * (c.args.planes + 1) * bytes <= hmi::kPlaneTile);
+                    if (bad) std::printf("FAIL grid %d x %d planes %lld\n", n0, n1, nplanes), fails++;
+                }
+            }
+    for (int threads : {64, 128, 320, 512})
+        for (long long nblocks : {1LL, 1LL << 22, 1LL << 23, (1LL << 26) - 1}) {
+            const int t = hmi::launch_threads(threads, nblocks);
+            const bool most = t == threads || nblocks * (t + 64) > 0xffffffffLL;
+            if (t < 64 || t % 64 || t > threads || nblocks * t > 0xffffffffLL || !most)
+                std::printf("FAIL threads %d blocks %lld\n", threads, nblocks), fails++;
+        }
+    return fails;
+}
+
 int main(int argc, char **argv) {
     const int share = argc > 1 ? std::atoi(argv[1]) : 0, shares = argc > 2 ? std::atoi(argv[2]) : 1;
     std::mt19937 rng(3);
-    int cases = 0, fails = 0, at = 0;
+    int cases = 0, fails = share == 0 ? check_grids() : 0, at = 0;
     auto one = [&](bool dbl, int n0, int n1, int nplanes) {
         const bool inverse = rng() & 1;
         const int product = (int)(rng() % 4) % 3;

@@ -87,3 +87,56 @@ def test_fused_planes(hmi, cuda, oracle, dtype, size):
         tz = torch.empty_like(tx)
         plan.convolve(tx, ty, tz, None, hmi.scale.full, 2)
         assert fc.rel_l2(fc.to_host(tz), oracle.convolve3d(b, b, x, x, 1.0 / n, 2)) <= 2 * fc.TOL[dtype], order
+
+
+def passes_of(plan):
+    return " ".join(plan.timing())
+
+
+@pytest.mark.parametrize("dtype", ["complex64", "complex128"])
+@pytest.mark.parametrize("size,batch", [((2, 3, 1), 700), ((4, 4, 4), 300), ((5, 7, 3), 401), ((8, 8, 8), 129), ((16, 16, 16), 70),
+                                        ((32, 30, 3), 90), ((81, 64, 2), 60), ((20, 256, 3), 20), ((100, 45, 7), 10),
+                                        ((98, 100, 4), 30), ((256, 20, 6), 9)])
+def test_fused_planes_of_a_batch(hmi, cuda, oracle, dtype, size, batch):
+    """The planes of a whole batch are grouped into blocks, and planes that fill a CU take the fused pass
+    only where the batch holds enough of them: both schedules of one plan, one transform and the batch."""
+    import torch
+    n = int(np.prod(size))
+    x = fc.uniform_complex(batch * n, n % 89)
+    box = hmi.box3d([0, 0, 0], [s - 1 for s in size])
+    plan = hmi.fft3d(hmi.backend.mi355, box, box)
+    b = oracle.Box.make((0, 0, 0), [s - 1 for s in size], (0, 1, 2))
+    ref = oracle.fft3d_c2c(b, b, x, -1, 1.0, batch)
+    tx = fc.to_gpu(x, np.complex64 if dtype == "complex64" else np.complex128)
+    ty, tz = torch.empty_like(tx), torch.empty(n, dtype=tx.dtype, device=cuda)
+    plan.set_timing(True)
+    plan.forward(tx, ty, hmi.scale.none, batch)
+    assert "fft_plane" in passes_of(plan)
+    assert fc.rel_l2(fc.to_host(ty), ref) <= fc.TOL[dtype]
+    plan.set_timing(True)
+    plan.forward(tx, tz)
+    # one transform: planes above 64 KiB in a CU each would leave the others idle
+    wide = (size[0] | 1) * size[1] * tx.element_size() > 64 * 1024 + 8192
+    assert ("fft_plane" in passes_of(plan)) == (not wide)
+    plan.set_timing(False)
+    assert fc.rel_l2(fc.to_host(tz), ref[:n]) <= fc.TOL[dtype]
+    plan.backward(ty, ty, hmi.scale.full, batch)
+    assert fc.rel_l2(fc.to_host(ty), x) <= fc.TOL[dtype]
+
+
+def test_sixteen_million_small_boxes(hmi, cuda, oracle):
+    """2^24 boxes of 4 x 4 x 4 in one call, in place (8.6 GB): one plane per block would ask for 2^32
+    threads, more than a launch takes."""
+    import torch
+    few, n = 64, 64
+    x = fc.uniform_complex(few * n, 3)
+    box = hmi.box3d([0, 0, 0], [3, 3, 3])
+    plan = hmi.fft3d(hmi.backend.mi355, box, box)
+    b = oracle.Box.make((0, 0, 0), (3, 3, 3), (0, 1, 2))
+    ref = oracle.fft3d_c2c(b, b, x, -1, 1.0, few)
+    tx = fc.to_gpu(x, np.complex64)
+    many = tx.repeat((1 << 24) // few)
+    plan.forward(many, many, hmi.scale.none, 1 << 24)
+    many = many.view(-1, few * n)
+    assert fc.rel_l2(fc.to_host(many[0]), ref) <= fc.TOL["complex64"]
+    assert all(torch.equal(rows, many[:1].expand_as(rows)) for rows in many.split(1 << 16))

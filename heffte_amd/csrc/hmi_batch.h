@@ -67,7 +67,9 @@ class batch_plan {
 
   private:
     struct device_state {
-        void *tw = nullptr;
+        void *tables = nullptr;  // the allocation that holds everything below
+        float *tw_f32 = nullptr;
+        double *tw_f64 = nullptr;
         batch_xform *xf = nullptr;
         // work lists per axis and register class of tile (batch_kernel_class), each run by its
         // own build of the batched kernel

@@ -199,7 +199,8 @@ class fft_plan {
     std::mutex mtx_;
     twiddles mfma_tw_[2][2] = {};  // [split FP16, split BF16][forward, backward]
     std::map<int, exec_choice> plans_;
-    std::map<long long, twiddles> tw_;
+    std::map<long long, twiddles> tw_;  // within the allocations tables_
+    std::vector<void *> tables_;
     // per-pass timing records: launch i ran between events marks_[i].first and .second
     // (a lock of their own: a timed call looks up tables while it records)
     std::mutex timing_mtx_;

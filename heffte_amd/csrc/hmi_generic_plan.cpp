@@ -64,11 +64,20 @@ bool is_prime(int p) {
     return true;
 }
 
-// Largest prime run as a direct stage.  A direct sum's error grows with the prime, a chirp
-// convolution's hardly with the length; measured against 64 bits on single primes, direct / chirp:
-// 17 points 0.85e-7 / 1.30e-7 (complex<double> 2.1e-16 / 2.9e-16), 47: 1.33e-7 / 1.35e-7 (2.9e-16 /
-// 2.9e-16), 97: 1.83e-7 / 1.46e-7 (3.7e-16 / 3.0e-16).
-constexpr int kMaxDirect = 61;
+// Largest prime factor that runs as a direct stage in a length of `cofactor` times that prime.  The error
+// of a direct stage grows with its prime alone, that of a chirp convolution with the whole length, whose
+// transforms it needs twice.  Relative errors against long double, direct stage / chirp / one direct sum
+// without shared pairs:
+//   complex<double>  67 points 2.11e-16 / 2.56e-16 / 2.88e-16, 4 x 67 2.32 / 3.45 / 3.01, 6 x 67 2.42 / 3.80 / 3.16
+//   complex<float>   30 x 67 1.41e-7 / 1.91e-7 / 1.78e-7, 4 x 101 1.45 / 1.62 / 1.93
+// A prime alone is direct up to 61 (67 points 1.0 to 1.2 times the chirp's time, 127 points 1.5 to 2.6), and
+// with a cofactor up to where the chirp would be less exact than that plain direct sum (complex<double>
+// 3 x 71 ... 30 x 107, complex<float> 4 x 67, 60 x 83, 56 x 89; of all lengths of one tile): there the direct
+// stage takes 0.5 to 1.4 times the chirp's time.
+int max_direct(int cofactor, bool dbl) {
+    if (dbl) return cofactor < 3 ? 61 : 107;
+    return cofactor < 4 ? 61 : cofactor < 24 ? 73 : cofactor < 48 ? 83 : 107;
+}
 
 fast_div make_div(unsigned d) {
     unsigned s = 0;
@@ -104,8 +113,12 @@ int read_conflicts(const mixed_plan &g, int pad, int group) {
 }  // namespace
 
 std::vector<int> mixed_radices(int n, bool dbl) {
+    int largest = n;  // prime factor
+    for (int p = 2; p * p <= largest; p++)
+        while (largest % p == 0 && largest > p) largest /= p;
+    const int top = max_direct(n / largest, dbl);
     std::vector<int> direct;
-    for (int p = 17; p <= kMaxDirect; p += 2)
+    for (int p = 17; p <= top; p += 2)
         while (is_prime(p) && n % p == 0) {
             direct.push_back(p);
             n /= p;

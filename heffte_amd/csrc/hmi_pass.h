@@ -92,8 +92,8 @@ struct fast_div {
 // k_0 m_0 + k_1 m_1 + ...  Element (line l, position i) of a tile sits at
 // i pitch + (i / m_0) pad + l.
 //
-// Prime factors from 17 to 61 are direct stages, behind the others: an output pair (q, p - q) sums the
-// (p - 1) / 2 input pairs (k, p - k) against the table w_p^t.  The last stage takes them from LDS to
+// Prime factors from 17 to 61 (to 107 beside other factors, max_direct) are direct stages, behind the
+// others: an output pair (q, p - q) sums the (p - 1) / 2 input pairs (k, p - k) against the table w_p^t.  The last stage takes them from LDS to
 // global memory; a length with two or three such factors runs the earlier ones from one LDS buffer
 // to a second one.
 //

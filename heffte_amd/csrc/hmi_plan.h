@@ -211,8 +211,8 @@ class fft_plan {
     void clear_timing();
 };
 
-// Radix order of the runtime-length pass (empty: n has a prime factor above 13), and its tile for one
-// pass (copy: no transform, only the layout change; *_across: that side walks the column axis; nlines:
+// Radix order of the runtime-length pass (empty: n has a prime factor beyond the direct stages and runs as
+// a chirp convolution), and its tile for one pass (copy: no transform, only the layout change; *_across: that side walks the column axis; nlines:
 // lines of a launch with few of them, 0 for many; tail: real-data twiddles).  Device table: the later stages' entries,
 // the stage twiddles, w_{tail_mod}^k for k < tail, the chirp and its transform.
 std::vector<int> mixed_radices(int n, bool dbl);

@@ -10,7 +10,7 @@ pytestmark = pytest.mark.gpu
 
 LENGTHS = [2, 3, 7, 10, 11, 13, 14, 15, 18, 22, 25, 26, 36, 49, 50, 60, 72, 81, 90, 91, 100, 121, 125, 143, 150, 169, 180,
            225, 240, 250, 320, 343, 384, 400, 625, 768, 1000, 1331, 2187, 2400, 3125, 5000,
-           17, 19, 34, 37, 51, 61, 186, 289, 323, 4913, 67, 127, 158, 199, 254, 509, 2003, 4999]
+           17, 19, 34, 37, 51, 61, 186, 289, 323, 4913, 67, 127, 158, 199, 254, 509, 2003, 4999, 201, 268, 402, 2010, 4489]
 
 
 @pytest.mark.parametrize("dtype", ["complex64", "complex128"])

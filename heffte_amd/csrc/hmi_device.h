@@ -78,6 +78,8 @@ template <typename C> __device__ __forceinline__ C csub(C a, C b) { return cmk<C
 template <typename C> __device__ __forceinline__ C cmul(C a, C b) {
     return cmk<C>(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
 }
+__device__ __forceinline__ float fmad(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+__device__ __forceinline__ double fmad(double a, double b, double c) { return __builtin_fma(a, b, c); }
 // a * (-i)
 template <typename C> __device__ __forceinline__ C cmul_mi(C a) { return cmk<C>(a.y, -a.x); }
 // a * (+i)
@@ -283,10 +285,26 @@ template <> struct dft<12> : dft_coprime<4, 3> {};
 template <> struct dft<14> : dft_coprime<2, 7> {};
 template <> struct dft<15> : dft_coprime<3, 5> {};
 
+// a w for a constant w = (c, s) given with the parts that its rounding drops: two roundings, as a product
+// with a table entry, and no error of the constant
+template <typename C>
+__device__ __forceinline__ C cmul_exact(C a, decltype(C::x) c, decltype(C::x) c_lo, decltype(C::x) s, decltype(C::x) s_lo) {
+    const auto re = a.x * c_lo - a.y * s_lo, im = a.x * s_lo + a.y * c_lo;
+    return cmk<C>(fmad(a.x, c, fmad(-a.y, s, re)), fmad(a.x, s, fmad(a.y, c, im)));
+}
+// what rounding a constant to T drops (lo: what its double literal drops)
+template <typename T> constexpr T const_lo(double v, double lo) { return (T)((v - (double)(T)v) + lo); }
+
 // 9 = 3 x 3: DFT3 over h of x[p + 3h], twiddle by w9^{p m}, DFT3 over p.
 template <> struct dft<9> {
-    template <typename C> __device__ __forceinline__ static void run(C *x) {
+    template <bool EXACT, typename C>
+    __device__ __forceinline__ static C rotate(C a, double c, double c_lo, double s, double s_lo) {
         using T = decltype(C::x);
+        if constexpr (EXACT) return cmul_exact(a, (T)c, const_lo<T>(c, c_lo), (T)s, const_lo<T>(s, s_lo));
+        return cmul(a, cmk<C>((T)c, (T)s));
+    }
+    // EXACT: without the rounding errors of the constants
+    template <bool EXACT = false, typename C> __device__ __forceinline__ static void run(C *x) {
         C y[3][3];
 #pragma unroll
         for (int p = 0; p < 3; p++) {
@@ -294,10 +312,10 @@ template <> struct dft<9> {
             for (int h = 0; h < 3; h++) y[p][h] = x[p + 3 * h];
             dft<3>::run(y[p]);
         }
-        y[1][1] = cmul(y[1][1], cmk<C>((T)0.76604444311897803520, (T)-0.64278760968653932632));
-        y[1][2] = cmul(y[1][2], cmk<C>((T)0.17364817766693034885, (T)-0.98480775301220805937));
-        y[2][1] = cmul(y[2][1], cmk<C>((T)0.17364817766693034885, (T)-0.98480775301220805937));
-        y[2][2] = cmul(y[2][2], cmk<C>((T)-0.93969262078590838405, (T)-0.34202014332566873304));
+        y[1][1] = rotate<EXACT>(y[1][1], 0.76604444311897803520, 2.175071174208104540e-17, -0.64278760968653932632, 3.659607900790949073e-17);
+        y[1][2] = rotate<EXACT>(y[1][2], 0.17364817766693034885, -1.009049335084363263e-17, -0.98480775301220805937, -3.905108875799298123e-17);
+        y[2][1] = rotate<EXACT>(y[2][1], 0.17364817766693034885, -1.009049335084363263e-17, -0.98480775301220805937, -3.905108875799298123e-17);
+        y[2][2] = rotate<EXACT>(y[2][2], -0.93969262078590838405, 4.385093284002041579e-17, -0.34202014332566873304, -2.013601653464464493e-17);
 #pragma unroll
         for (int m = 0; m < 3; m++) {
             C z[3] = {y[0][m], y[1][m], y[2][m]};
@@ -307,5 +325,11 @@ template <> struct dft<9> {
         }
     }
 };
+
+// Butterfly of one stage; EXACT: its radix-9 constants without their rounding errors.
+template <int RX, bool EXACT, typename C> __device__ __forceinline__ void butterfly(C *x) {
+    if constexpr (RX == 9) dft<9>::run<EXACT>(x);
+    else dft<RX>::run(x);
+}
 
 }  // namespace hmi

@@ -215,7 +215,7 @@ __device__ __forceinline__ C mixed_element(const pass_args &a, const mixed_plan 
 }
 
 // Stage 0: global memory -> LDS.
-template <int RX, int FORM, int NTM, typename R, typename C>
+template <int RX, int SET, int FORM, int NTM, typename R, typename C>
 __device__ __forceinline__ void mixed_first(const pass_args &a, const mixed_plan &g, unsigned tile, C *lds) {
     const int T = 1 << g.log2t, m = g.m0, nth = blockDim.x;
     const int stride = m * g.pitch + g.pad;
@@ -250,7 +250,7 @@ __device__ __forceinline__ void mixed_first(const pass_args &a, const mixed_plan
         } else {
             mixed_load<RX, FORM, NTM, R>(x, a, g, ln, j, m);
         }
-        dft<RX>::run(x);
+        butterfly<RX, SET == kSetOdd>(x);
         if (m > 1) {
             const C *w = tw + j * (RX - 1);
 #pragma unroll
@@ -263,7 +263,7 @@ __device__ __forceinline__ void mixed_first(const pass_args &a, const mixed_plan
 }
 
 // A stage between two others, in place in LDS; BACK: its transpose (twiddles before the butterfly).
-template <int RX, bool BACK, typename R, typename C>
+template <int RX, int SET, bool BACK, typename R, typename C>
 __device__ __forceinline__ void mixed_middle(const pass_args &a, const mixed_plan &g, const mixed_stage &st, C *lds) {
     const int T = 1 << g.log2t, m = st.m, nth = blockDim.x;
     const int stride = m * g.pitch;
@@ -283,7 +283,7 @@ __device__ __forceinline__ void mixed_middle(const pass_args &a, const mixed_pla
 #pragma unroll
             for (int q = 1; q < RX; q++) x[q] = cmul(x[q], w[q - 1]);
         }
-        dft<RX>::run(x);
+        butterfly<RX, SET == kSetOdd>(x);
         if (!BACK) {
 #pragma unroll
             for (int q = 1; q < RX; q++) x[q] = cmul(x[q], w[q - 1]);
@@ -295,7 +295,7 @@ __device__ __forceinline__ void mixed_middle(const pass_args &a, const mixed_pla
 
 // Chirp passes: the last stage, the product with the transformed chirp and the first transposed
 // stage, which works on the same elements.
-template <int RX, typename R, typename C>
+template <int RX, int SET, typename R, typename C>
 __device__ __forceinline__ void mixed_center(const pass_args &a, const mixed_plan &g, const mixed_stage &st, C *lds) {
     const int T = 1 << g.log2t, nth = blockDim.x;
     const unsigned nb = (unsigned)g.n / RX;
@@ -307,20 +307,20 @@ __device__ __forceinline__ void mixed_center(const pass_args &a, const mixed_pla
         C x[RX];
 #pragma unroll
         for (int p = 0; p < RX; p++) x[p] = dp[p * g.pitch];
-        dft<RX>::run(x);
+        butterfly<RX, SET == kSetOdd>(x);
 #pragma unroll
         for (int q = 0; q < RX; q++) {
             const C v = cmul(x[q], hat[c * RX + q]);
             x[q] = cmk<C>(v.x, -v.y);
         }
-        dft<RX>::run(x);
+        butterfly<RX, SET == kSetOdd>(x);
 #pragma unroll
         for (int q = 0; q < RX; q++) dp[q * g.pitch] = x[q];
     }
 }
 
 // Chirp passes: the transpose of stage 0, LDS -> global memory.
-template <int RX, int NTM, typename R, typename C>
+template <int RX, int SET, int NTM, typename R, typename C>
 __device__ __forceinline__ void mixed_chirp_last(const pass_args &a, const mixed_plan &g, unsigned tile, const C *lds) {
     const int T = 1 << g.log2t, m = g.m0, nth = blockDim.x;
     const int stride = m * g.pitch + g.pad;
@@ -347,7 +347,7 @@ __device__ __forceinline__ void mixed_chirp_last(const pass_args &a, const mixed
         for (int q = 0; q < RX; q++) x[q] = sp[q * stride];
 #pragma unroll
         for (int q = 1; q < RX; q++) x[q] = cmul(x[q], w[q - 1]);
-        dft<RX>::run(x);
+        butterfly<RX, SET == kSetOdd>(x);
 #pragma unroll
         for (int p = 0; p < RX; p++) {
             const int k = j + p * m;
@@ -360,7 +360,7 @@ __device__ __forceinline__ void mixed_chirp_last(const pass_args &a, const mixed
 }
 
 // The last stage: LDS -> global memory.
-template <int RX, int FORM, int NTM, typename R, typename C>
+template <int RX, int SET, int FORM, int NTM, typename R, typename C>
 __device__ __forceinline__ void mixed_last(const pass_args &a, const mixed_plan &g, unsigned tile, const C *lds) {
     const int T = 1 << g.log2t, nth = blockDim.x;
     const unsigned nb = (unsigned)g.n / RX;
@@ -395,7 +395,7 @@ __device__ __forceinline__ void mixed_last(const pass_args &a, const mixed_plan 
         C x[RX];
 #pragma unroll
         for (int p = 0; p < RX; p++) x[p] = sp[p * g.pitch];
-        dft<RX>::run(x);
+        butterfly<RX, SET == kSetOdd>(x);
         mixed_store<RX, FORM, NTM, R>(x, a, g, ln, (int)u, (int)nb);
     }
 }
@@ -527,11 +527,13 @@ __device__ __forceinline__ void mixed_direct_last(const pass_args &a, const mixe
     }
 }
 
-// Radices of the light build (every thread holds at most kLightRadix values) and of the full one.
+// Radices of the light build (every thread holds at most kLightRadix values), what the full one adds, and
+// those of the odd one.
 #define HMI_MIXED_LIGHT(X) X(2) X(3) X(4) X(5) X(6) X(7) X(8) X(9) X(10)
 #define HMI_MIXED_HEAVY(X) X(11) X(12) X(13) X(14) X(15) X(16)
+#define HMI_MIXED_ODD(X) X(3) X(5) X(7) X(9)
 
-template <typename R, bool HEAVY, int FORM, int NTM>
+template <typename R, int SET, int FORM, int NTM>
 __global__ void __launch_bounds__(kMixedThreads) fft_generic(pass_args a, mixed_plan g) {
     using C = typename cvec<R>::type;
     extern __shared__ __align__(16) unsigned char smem_raw[];
@@ -548,15 +550,17 @@ __global__ void __launch_bounds__(kMixedThreads) fft_generic(pass_args a, mixed_
                  : chunk == 16 ? xcd_grouped_tile<8>(tile, gridDim.x) : xcd_grouped_tile<16>(tile, gridDim.x);
         }
     }
-#define HMI_MIXED_FIRST(RX) case RX: mixed_first<RX, FORM, NTM, R>(a, g, tile, lds); break;
-#define HMI_MIXED_MID(RX) case RX: mixed_middle<RX, false, R>(a, g, st, lds); break;
-#define HMI_MIXED_BACK(RX) case RX: mixed_middle<RX, true, R>(a, g, st, lds); break;
-#define HMI_MIXED_CENTER(RX) case RX: mixed_center<RX, R>(a, g, st, lds); break;
-#define HMI_MIXED_LAST(RX) case RX: mixed_last<RX, FORM, NTM, R>(a, g, tile, lds); break;
-#define HMI_MIXED_CHIRP_LAST(RX) case RX: mixed_chirp_last<RX, NTM, R>(a, g, tile, lds); break;
+#define HMI_MIXED_FIRST(RX) case RX: mixed_first<RX, SET, FORM, NTM, R>(a, g, tile, lds); break;
+#define HMI_MIXED_MID(RX) case RX: mixed_middle<RX, SET, false, R>(a, g, st, lds); break;
+#define HMI_MIXED_BACK(RX) case RX: mixed_middle<RX, SET, true, R>(a, g, st, lds); break;
+#define HMI_MIXED_CENTER(RX) case RX: mixed_center<RX, SET, R>(a, g, st, lds); break;
+#define HMI_MIXED_LAST(RX) case RX: mixed_last<RX, SET, FORM, NTM, R>(a, g, tile, lds); break;
+#define HMI_MIXED_CHIRP_LAST(RX) case RX: mixed_chirp_last<RX, SET, NTM, R>(a, g, tile, lds); break;
 #define HMI_MIXED_SWITCH(R, CASE)                                                     \
-    if constexpr (HEAVY) {                                                            \
+    if constexpr (SET == kSetFull) {                                                  \
         switch (R) { HMI_MIXED_LIGHT(CASE) HMI_MIXED_HEAVY(CASE) }                    \
+    } else if constexpr (SET == kSetOdd) {                                            \
+        switch (R) { HMI_MIXED_ODD(CASE) }                                            \
     } else {                                                                          \
         switch (R) { HMI_MIXED_LIGHT(CASE) }                                          \
     }
@@ -606,22 +610,23 @@ __global__ void __launch_bounds__(kMixedThreads) fft_generic(pass_args a, mixed_
 
 template <typename R> struct generic_builds {
     using fn = void (*)(pass_args, mixed_plan);
-    // [full radix set][kFormAny, kFormPlain, kFormPlain32, kFormChirp, kFormDirect][non-temporal: none, stores, both]
-    static fn pick(bool heavy, int form, int stream) {
+    // [radix set][kFormAny, kFormPlain, kFormPlain32, kFormChirp, kFormDirect][non-temporal: none, stores, both]
+    static fn pick(int set, int form, int stream) {
 #ifdef HMI_EMULATE  // the CPU tests run the kernels without the non-temporal hints
-#define HMI_MIXED_BUILDS(H, F) {&fft_generic<R, H, F, 0>, nullptr, nullptr}
+#define HMI_MIXED_BUILDS(S, F) {&fft_generic<R, S, F, 0>, nullptr, nullptr}
 #else
-#define HMI_MIXED_BUILDS(H, F) \
-    {&fft_generic<R, H, F, 0>, &fft_generic<R, H, F, kStreamStores>, &fft_generic<R, H, F, kStreamLoadsStores>}
+#define HMI_MIXED_BUILDS(S, F) \
+    {&fft_generic<R, S, F, 0>, &fft_generic<R, S, F, kStreamStores>, &fft_generic<R, S, F, kStreamLoadsStores>}
 #endif
         static const fn f[2][5][3] = {
-            {HMI_MIXED_BUILDS(false, 0), HMI_MIXED_BUILDS(false, 1), HMI_MIXED_BUILDS(false, 2), HMI_MIXED_BUILDS(false, 3), HMI_MIXED_BUILDS(false, 4)},
-            {HMI_MIXED_BUILDS(true, 0), HMI_MIXED_BUILDS(true, 1), HMI_MIXED_BUILDS(true, 2), HMI_MIXED_BUILDS(true, 3), HMI_MIXED_BUILDS(true, 4)}};
-        return f[heavy ? 1 : 0][form][stream == 0 ? 0 : (stream == kStreamStores ? 1 : 2)];
+            {HMI_MIXED_BUILDS(kSetLight, 0), HMI_MIXED_BUILDS(kSetLight, 1), HMI_MIXED_BUILDS(kSetLight, 2), HMI_MIXED_BUILDS(kSetLight, 3), HMI_MIXED_BUILDS(kSetLight, 4)},
+            {HMI_MIXED_BUILDS(kSetFull, 0), HMI_MIXED_BUILDS(kSetFull, 1), HMI_MIXED_BUILDS(kSetFull, 2), HMI_MIXED_BUILDS(kSetFull, 3), HMI_MIXED_BUILDS(kSetFull, 4)}};
+        // (a plan of the odd set has neither a chirp nor direct stages)
+        static const fn odd[3][3] = {HMI_MIXED_BUILDS(kSetOdd, 0), HMI_MIXED_BUILDS(kSetOdd, 1), HMI_MIXED_BUILDS(kSetOdd, 2)};
+        const int at = stream == 0 ? 0 : (stream == kStreamStores ? 1 : 2);
+        return set == kSetOdd ? odd[form][at] : f[set][form][at];
     }
     static fn choose(const pass_args &a, const mixed_plan &g) {
-        int top = 0;
-        for (int i = 0; i < g.nst; i++) top = g.radix[i] <= 16 ? std::max(top, g.radix[i]) : top;
         const bool plain = a.mode == kModeC2C && !a.in_real && !a.out_real && !a.herm_load && !a.mul && !a.tw4 &&
                            a.store_len == g.len;
         // elements up to the furthest one of either side (no stride is negative)
@@ -631,17 +636,17 @@ template <typename R> struct generic_builds {
         const long long most = std::max(span(a.in_sa, a.in_sc, a.in_sb1, a.in_sb2),
                                         span(a.out_sa, a.out_sc, a.out_sb1, a.out_sb2));
         const bool near = most * (long long)sizeof(typename cvec<R>::type) <= (1LL << 32);
-        return pick(top > kLightRadix, g.chirp ? kFormChirp : g.direct ? kFormDirect : !plain ? kFormAny : (near ? kFormPlain32 : kFormPlain), a.stream);
+        return pick(g.set, g.chirp ? kFormChirp : g.direct ? kFormDirect : !plain ? kFormAny : (near ? kFormPlain32 : kFormPlain), a.stream);
     }
 #ifndef HMI_EMULATE
     static hipError_t launch(const pass_args &a, const mixed_plan &g, int threads, long long nblocks, size_t lds,
                              hipStream_t s) {
         // once per process, thread-safe (static initialisation)
         static const bool configured = [] {
-            for (bool heavy : {false, true})
-                for (int form = 0; form < 5; form++)
+            for (int set : {kSetLight, kSetFull, kSetOdd})
+                for (int form = 0; form < (set == kSetOdd ? 3 : 5); form++)
                     for (int st : {0, (int)kStreamStores, (int)kStreamLoadsStores})
-                        (void)hipFuncSetAttribute(reinterpret_cast<const void *>(pick(heavy, form, st)),
+                        (void)hipFuncSetAttribute(reinterpret_cast<const void *>(pick(set, form, st)),
                                                   hipFuncAttributeMaxDynamicSharedMemorySize, kGenericMaxLds);
             return true;
         }();

@@ -103,10 +103,13 @@ struct fast_div {
 // stages above transform x_j c_j, the last one multiplies by the transform of conj(c) (in position
 // order, times 1 / n) and conjugates, and the transposed stages S-1 ... 0 lead back to natural order.
 enum : int { kMixedStages = 6 };
+// Radices up to kLightRadix, all up to 16, and 3, 5, 7 and 9 with exact constants of radix 9.
+enum : int { kSetLight = 0, kSetFull = 1, kSetOdd = 2 };
 struct mixed_plan {
     int n, nst;
     int len;                         // points of a line (n, unless chirp)
     int chirp, direct;               // direct: number of direct stages
+    int set;                         // build of the kernels that runs it (kSetLight, ...)
     int log2t, pitch, pad;           // lines per tile 2^log2t, LDS strides (elements)
     int radix[kMixedStages];
     int m0;                          // the first stage's twiddles w_n^{j q}: table[j (r_0 - 1) + q - 1]

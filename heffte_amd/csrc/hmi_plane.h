@@ -43,7 +43,7 @@ __device__ __forceinline__ int plane_position(unsigned k, const mixed_plan &g) {
 
 // One axis of the plane: stage s of every line of the block in place in LDS.  A line is a row (stride
 // rp between rows, elements 1 apart) or a column (columns 1 apart, planes ps apart, elements rp apart).
-template <int RX, bool COLS, typename C>
+template <int RX, int SET, bool COLS, typename C>
 __device__ __forceinline__ void plane_stage(const plane_args &a, const mixed_plan &g, const C *__restrict__ tw, int m,
                                             const fast_div &by_m, C *lds) {
     const unsigned nb = (unsigned)(g.n / RX), nlines = COLS ? a.cols : a.rows;
@@ -64,7 +64,7 @@ __device__ __forceinline__ void plane_stage(const plane_args &a, const mixed_pla
         C x[RX];
 #pragma unroll
         for (int p = 0; p < RX; p++) x[p] = dp[p * stride];
-        dft<RX>::run(x);
+        butterfly<RX, SET == kSetOdd>(x);
         if (m > 1) {
             const C *w = tw + j * (RX - 1);
 #pragma unroll
@@ -76,7 +76,7 @@ __device__ __forceinline__ void plane_stage(const plane_args &a, const mixed_pla
 }
 
 // First row stage, global memory -> LDS (lanes walk the rows).
-template <int RX, int NTM, typename R, typename C>
+template <int RX, int SET, int NTM, typename R, typename C>
 __device__ __forceinline__ void plane_load(const plane_args &a, const C *__restrict__ tw, long long base, unsigned rows, C *lds) {
     constexpr bool NTL = (NTM & 2) != 0;
     const int m = a.g0.m0;
@@ -99,7 +99,7 @@ __device__ __forceinline__ void plane_load(const plane_args &a, const C *__restr
         }
 #pragma unroll
         for (int p = 0; p < RX; p++) x[p].y *= sg;
-        dft<RX>::run(x);
+        butterfly<RX, SET == kSetOdd>(x);
         if (m > 1) {
             const C *w = tw + j * (RX - 1);
 #pragma unroll
@@ -112,7 +112,7 @@ __device__ __forceinline__ void plane_load(const plane_args &a, const C *__restr
 }
 
 // Last column stage, LDS -> global memory (lanes walk the columns in frequency order).
-template <int RX, int NTM, typename R, typename C>
+template <int RX, int SET, int NTM, typename R, typename C>
 __device__ __forceinline__ void plane_store(const plane_args &a, long long base, unsigned cols, const C *lds) {
     constexpr bool NTS = (NTM & 1) != 0;
     const unsigned nb = (unsigned)(a.g1.n / RX);
@@ -128,7 +128,7 @@ __device__ __forceinline__ void plane_store(const plane_args &a, long long base,
         C x[RX];
 #pragma unroll
         for (int p = 0; p < RX; p++) x[p] = sp[p * a.rp];
-        dft<RX>::run(x);
+        butterfly<RX, SET == kSetOdd>(x);
         const unsigned off = (pl * (unsigned)a.n1 + u) * (unsigned)a.n0 + k0;
         const unsigned st = nb * (unsigned)a.n0;
 #pragma unroll
@@ -136,7 +136,7 @@ __device__ __forceinline__ void plane_store(const plane_args &a, long long base,
     }
 }
 
-template <typename R, bool HEAVY, int NTM> __global__ void __launch_bounds__(kMixedThreads) fft_plane(plane_args a) {
+template <typename R, int SET, int NTM> __global__ void __launch_bounds__(kMixedThreads) fft_plane(plane_args a) {
     using C = typename cvec<R>::type;
     extern __shared__ __align__(16) unsigned char smem_raw[];
     C *lds = reinterpret_cast<C *>(smem_raw);
@@ -146,11 +146,11 @@ template <typename R, bool HEAVY, int NTM> __global__ void __launch_bounds__(kMi
     const C *__restrict__ tw0 = reinterpret_cast<const C *>(static_cast<const char *>(a.tw0) + kMixedHead);
     const C *__restrict__ tw1 = reinterpret_cast<const C *>(static_cast<const char *>(a.tw1) + kMixedHead);
     const mixed_stage *st0 = static_cast<const mixed_stage *>(a.tw0), *st1 = static_cast<const mixed_stage *>(a.tw1);
-#define HMI_PLANE_LOAD(RX) case RX: plane_load<RX, NTM, R>(a, tw0, base, planes * (unsigned)a.n1, lds); break;
-#define HMI_PLANE_ROW(RX) case RX: plane_stage<RX, false>(a, a.g0, tw0 + st.twoff, st.m, st.by_m, lds); break;
-#define HMI_PLANE_COL0(RX) case RX: plane_stage<RX, true>(a, a.g1, tw1, a.g1.m0, a.g1.by_m0, lds); break;
-#define HMI_PLANE_COL(RX) case RX: plane_stage<RX, true>(a, a.g1, tw1 + st.twoff, st.m, st.by_m, lds); break;
-#define HMI_PLANE_STORE(RX) case RX: plane_store<RX, NTM, R>(a, base, planes * (unsigned)a.n0, lds); break;
+#define HMI_PLANE_LOAD(RX) case RX: plane_load<RX, SET, NTM, R>(a, tw0, base, planes * (unsigned)a.n1, lds); break;
+#define HMI_PLANE_ROW(RX) case RX: plane_stage<RX, SET, false>(a, a.g0, tw0 + st.twoff, st.m, st.by_m, lds); break;
+#define HMI_PLANE_COL0(RX) case RX: plane_stage<RX, SET, true>(a, a.g1, tw1, a.g1.m0, a.g1.by_m0, lds); break;
+#define HMI_PLANE_COL(RX) case RX: plane_stage<RX, SET, true>(a, a.g1, tw1 + st.twoff, st.m, st.by_m, lds); break;
+#define HMI_PLANE_STORE(RX) case RX: plane_store<RX, SET, NTM, R>(a, base, planes * (unsigned)a.n0, lds); break;
     // (a partial group leaves the rows and columns of the missing planes untransformed garbage in LDS)
     HMI_MIXED_SWITCH(a.g0.radix[0], HMI_PLANE_LOAD)
     __syncthreads();
@@ -188,7 +188,7 @@ __device__ __forceinline__ mixed_plan load_plan(const mixed_plan *p) {
 }
 
 // First stage of a column block, global memory -> LDS: position i of column l at src + i row + l.
-template <int RX, typename R, typename C>
+template <int RX, int SET, typename R, typename C>
 __device__ __forceinline__ void cols_load(const plane_args &a, const C *__restrict__ tw, const C *src, long long row, unsigned w,
                                           C *lds) {
     const int m = a.g1.m0;
@@ -203,7 +203,7 @@ __device__ __forceinline__ void cols_load(const plane_args &a, const C *__restri
         for (int p = 0; p < RX; p++) x[p] = sp[p * st];
 #pragma unroll
         for (int p = 0; p < RX; p++) x[p].y *= sg;
-        dft<RX>::run(x);
+        butterfly<RX, SET == kSetOdd>(x);
         if (m > 1) {
             const C *wt = tw + j * (RX - 1);
 #pragma unroll
@@ -216,7 +216,7 @@ __device__ __forceinline__ void cols_load(const plane_args &a, const C *__restri
 }
 
 // Last stage of a column block, LDS -> global memory.
-template <int RX, typename R, typename C>
+template <int RX, int SET, typename R, typename C>
 __device__ __forceinline__ void cols_store(const plane_args &a, C *dst, long long row, unsigned w, const C *lds) {
     const unsigned nb = (unsigned)(a.g1.n / RX);
     const R sc = (R)a.scale, sy = a.conj ? -sc : sc;
@@ -227,7 +227,7 @@ __device__ __forceinline__ void cols_store(const plane_args &a, C *dst, long lon
         C x[RX];
 #pragma unroll
         for (int p = 0; p < RX; p++) x[p] = sp[p * a.rp];
-        dft<RX>::run(x);
+        butterfly<RX, SET == kSetOdd>(x);
         C *dp = dst + (long long)u * row + l;
         const long long st = (long long)nb * row;
 #pragma unroll
@@ -259,7 +259,7 @@ __device__ __forceinline__ void cols_copy(const plane_args &a, C *dst, long long
 // 3.00, 256 in the second 2.92; z blocks of 20 KB 2.94, of 80 KB with 512 threads 2.79.
 template <typename R, bool XY, int NTH> __global__ void __launch_bounds__(NTH) fft_batch_fused(batch_args b) {
     using C = typename cvec<R>::type;
-    constexpr bool HEAVY = true;
+    constexpr int SET = kSetFull;
     constexpr int NTM = 0;
     extern __shared__ __align__(16) unsigned char smem_raw[];
     C *lds = reinterpret_cast<C *>(smem_raw);
@@ -326,7 +326,7 @@ template <typename R, bool XY, int NTH> __global__ void __launch_bounds__(NTH) f
             a.scale = (b.scaling == 0) ? 1.0 : (b.scaling == 1 ? 1.0 / ntot : sqrt(1.0 / ntot));
             in += c0;
             out += c0;
-#define HMI_COLS_LOAD(RX) case RX: cols_load<RX, R>(a, tw1, in, row, w, lds); break;
+#define HMI_COLS_LOAD(RX) case RX: cols_load<RX, SET, R>(a, tw1, in, row, w, lds); break;
             HMI_MIXED_SWITCH(a.g1.radix[0], HMI_COLS_LOAD)
             __syncthreads();
         }
@@ -338,7 +338,7 @@ template <typename R, bool XY, int NTH> __global__ void __launch_bounds__(NTH) f
         if constexpr (XY) {
             HMI_MIXED_SWITCH(a.g1.last, HMI_PLANE_STORE)
         } else {
-#define HMI_COLS_STORE(RX) case RX: cols_store<RX, R>(a, out, row, w, lds); break;
+#define HMI_COLS_STORE(RX) case RX: cols_store<RX, SET, R>(a, out, row, w, lds); break;
             if (a.g1.nst == 1) cols_copy<R>(a, out, row, w, lds);
             else { HMI_MIXED_SWITCH(a.g1.last, HMI_COLS_STORE) }
         }
@@ -349,15 +349,16 @@ template <typename R, bool XY, int NTH> __global__ void __launch_bounds__(NTH) f
 template <typename R> struct plane_builds {
     using fn = void (*)(plane_args);
     static fn choose(const plane_args &a) {
-        int top = 0;
-        for (int i = 0; i < a.g0.nst; i++) top = std::max(top, a.g0.radix[i]);
-        for (int i = 0; i < a.g1.nst; i++) top = std::max(top, a.g1.radix[i]);
+        // both axes in one set: the odd one only for two plans of it (its radices are light ones too)
+        const int set = a.g0.set == kSetFull || a.g1.set == kSetFull ? kSetFull : a.g0.set == a.g1.set ? a.g0.set : kSetLight;
 #ifdef HMI_EMULATE
-        return top > kLightRadix ? &fft_plane<R, true, 0> : &fft_plane<R, false, 0>;
+        static const fn f[3] = {&fft_plane<R, kSetLight, 0>, &fft_plane<R, kSetFull, 0>, &fft_plane<R, kSetOdd, 0>};
+        return f[set];
 #else
-        static const fn f[2][2] = {{&fft_plane<R, false, 0>, &fft_plane<R, false, kStreamLoadsStores>},
-                                   {&fft_plane<R, true, 0>, &fft_plane<R, true, kStreamLoadsStores>}};
-        return f[top > kLightRadix ? 1 : 0][a.stream ? 1 : 0];
+        static const fn f[3][2] = {{&fft_plane<R, kSetLight, 0>, &fft_plane<R, kSetLight, kStreamLoadsStores>},
+                                   {&fft_plane<R, kSetFull, 0>, &fft_plane<R, kSetFull, kStreamLoadsStores>},
+                                   {&fft_plane<R, kSetOdd, 0>, &fft_plane<R, kSetOdd, kStreamLoadsStores>}};
+        return f[set][a.stream ? 1 : 0];
 #endif
     }
 #ifndef HMI_EMULATE
@@ -365,10 +366,9 @@ template <typename R> struct plane_builds {
         // once per process, thread-safe (static initialisation)
         static const bool configured = [] {
             for (int stream : {0, (int)kStreamLoadsStores})
-                for (int r : {2, 16}) {
+                for (int set : {kSetLight, kSetFull, kSetOdd}) {
                     plane_args p{};
-                    p.g0.nst = 1;
-                    p.g0.radix[0] = r;
+                    p.g0.set = p.g1.set = set;
                     p.stream = stream;
                     (void)hipFuncSetAttribute(reinterpret_cast<const void *>(choose(p)),
                                               hipFuncAttributeMaxDynamicSharedMemorySize, kGenericMaxLds);

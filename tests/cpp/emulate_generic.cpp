@@ -219,6 +219,10 @@ int main(int argc, char **argv) {
     const struct { bool dbl; int n; double plain; } exact[] = {
         {true, 213, 3.13e-16}, {true, 268, 3.01e-16}, {true, 402, 3.16e-16}, {true, 404, 3.60e-16}, {true, 536, 3.11e-16},
         {false, 268, 1.63e-7}, {false, 670, 1.70e-7}, {false, 2010, 1.78e-7}, {false, 4984, 1.97e-07}};
+    // odd lengths with several stages of radix 9: no less exact than with stages of radix 3
+    const struct { bool dbl; int n; double plain; } nines[] = {
+        {false, 81, 1.010e-7}, {false, 729, 1.282e-7}, {true, 81, 2.032e-16}};
+    for (const auto &e : nines) one(e.dbl, e.n, hmi::kModeC2C, 0, 0, 2, 80000 / e.n, 1, 1, e.plain);
     for (const auto &e : exact) one(e.dbl, e.n, hmi::kModeC2C, 0, 0, 2, e.n < 1000 ? 40 : 5, 1, 1, e.plain);
     std::printf("%s %d\n", fails ? "failed" : "ok", cases);
     return fails ? 1 : 0;

@@ -13,7 +13,7 @@ constexpr int kGenericMaxLds = 160 * 1024;
 // pass outputs above this size use non-temporal stores (larger than the MALL), and their loads
 // too when a side of the pass walks the column axis (pass_args::stream)
 constexpr long long kStreamBytes = 256LL << 20;
-enum : int { kStreamStores = 1, kStreamLoadsStores = 3 };
+enum : int { kStreamStores = 1, kStreamLoadsStores = 3, kHalvedTile = 4 };
 
 using fast_launcher = hipError_t (*)(const pass_args &, long long nblocks, hipStream_t);
 
@@ -23,6 +23,7 @@ struct fast_kernel_info {
     int n, E, T, PS;
     int radix[8];
     int nstages;
+    bool halved;  // real-to-real modes exchange in halves (kHalvedTile)
     fast_launcher launch;
 };
 

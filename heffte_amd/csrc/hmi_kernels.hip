@@ -184,7 +184,7 @@ __device__ __forceinline__ unsigned line_index(unsigned L, const pass_args &a, i
 // One tile (T lines) of an n-point pass; the block has exactly (n / E) * T threads.
 template <typename R, typename RL, int E, int T, int PS, int NTM = 0>
 __device__ __forceinline__ void uniform_tile(const pass_args &a, unsigned tile, typename cvec<R>::type *lds) {
-    constexpr bool HALVED = (NTM & 4) != 0;
+    constexpr bool HALVED = (NTM & kHalvedTile) != 0;
     using C = typename cvec<R>::type;
     constexpr int N = RL::n();
     constexpr int P = N / E;
@@ -444,7 +444,7 @@ __global__ void __launch_bounds__((RL::n() / E) * T) fft_uniform(pass_args a) {
     using C = typename cvec<R>::type;
     constexpr int RS = lds_map<RL::n(), E, PS, sizeof(C)>::RS;
     constexpr int CHUNK = T * (int)sizeof(C);
-    __shared__ C lds[(NTM & 4) ? (T * RS + 1) / 2 : T * RS];
+    __shared__ C lds[(NTM & kHalvedTile) ? (T * RS + 1) / 2 : T * RS];
     unsigned tile = blockIdx.x;
     if (a.load_colfast || a.store_colfast) {
         if constexpr (CHUNK >= 128 || CHUNK <= 32) {
@@ -894,7 +894,9 @@ __global__ void __launch_bounds__(256) permute_kernel(const E *__restrict__ src,
 // Real-to-real passes in complex<double> of 256 and more points, 8 elements per thread: their loads and
 // stores move half the bytes of a complex tile, so the pass is bound by latency, and its LDS holds a CU
 // to half the waves that its registers would allow.  Exchanging the parts one after the other in a tile
-// of half the size: 256^3 double DCT-II / III pair 465 -> 438 us, the results bit for bit the same.  The
+// of half the size: 256^3 double DCT-II / III pair 465 -> 438 us, the results bit for bit the same; above the
+// Infinity Cache with the streaming form of the pass (512 x 256 x 512, the contiguous axis 244 us with
+// non-temporal loads and stores, 231 with stores only).  The
 // complex passes stay as they are (512^3 complex<double> 768 -> 787 us per pass, 256^3 109 -> 108).
 constexpr bool halved_tile(int n, int e, int bytes) { return n >= 256 && bytes == 16 && e <= 8; }
 
@@ -902,8 +904,10 @@ constexpr bool halved_tile(int n, int e, int bytes) { return n >= 256 && bytes =
     static hipError_t launch_##TYPE##_##N##_##T(const pass_args &a, long long nblocks, hipStream_t s) {    \
         if constexpr (halved_tile(N, E, 2 * sizeof(TYPE))) {                                               \
             if (a.mode >= kModeDCT2) {                                                                     \
-                (a.stream ? &fft_uniform<TYPE, radices<__VA_ARGS__>, E, T, PS, 7>                          \
-                          : &fft_uniform<TYPE, radices<__VA_ARGS__>, E, T, PS, 4>)                         \
+                (a.stream == 0 ? &fft_uniform<TYPE, radices<__VA_ARGS__>, E, T, PS, kHalvedTile>           \
+                 : a.stream == kStreamStores                                                               \
+                     ? &fft_uniform<TYPE, radices<__VA_ARGS__>, E, T, PS, kHalvedTile | kStreamStores>     \
+                     : &fft_uniform<TYPE, radices<__VA_ARGS__>, E, T, PS, kHalvedTile | kStreamLoadsStores>) \
                     <<<dim3((unsigned)nblocks), dim3((N / E) * T), 0, s>>>(a);                             \
                 return hipGetLastError();                                                                  \
             }                                                                                              \
@@ -971,7 +975,8 @@ constexpr bool halved_tile(int n, int e, int bytes) { return n >= 256 && bytes =
 HMI_FAST_TABLE(HMI_FAST)
 
 #define HMI_FAST_ENTRY(TYPE, N, E, T, PS, ...) \
-    {sizeof(TYPE) == 8, N, E, T, PS, {__VA_ARGS__}, radices<__VA_ARGS__>::count, &launch_##TYPE##_##N##_##T},
+    {sizeof(TYPE) == 8, N, E, T, PS, {__VA_ARGS__}, radices<__VA_ARGS__>::count, \
+     halved_tile(N, E, 2 * sizeof(TYPE)), &launch_##TYPE##_##N##_##T},
 
 static const fast_kernel_info kFast[] = {HMI_FAST_TABLE(HMI_FAST_ENTRY)};
 

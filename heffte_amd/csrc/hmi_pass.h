@@ -145,7 +145,7 @@ struct plane_args {
     int rp, ps;                   // LDS strides of rows and planes (elements); rp is odd
     unsigned rows, cols;          // planes n1, planes n0
     fast_div by_rows, by_cols, by_n0;
-    int conj, stream;
+    int conj;
     double scale;
 };
 

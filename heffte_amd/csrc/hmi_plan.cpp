@@ -603,7 +603,8 @@ std::string pass_kernel_name(const pass &p, bool dbl, bool mfma, int precision, 
         s = std::string("fft_uniform<") + R + ", radices<";
         for (int i = 0; i < p.fast->nstages; i++) s += (i ? ", " : "") + std::to_string(p.fast->radix[i]);
         s += ">, " + std::to_string(p.fast->E) + ", " + std::to_string(p.fast->T) + ", " +
-             std::to_string(p.fast->PS) + ", " + std::to_string(a.stream) + ">";
+             std::to_string(p.fast->PS) + ", " +
+             std::to_string(a.stream | (p.fast->halved && p.mode >= kModeDCT2 ? kHalvedTile : 0)) + ">";
     } else {
         s = std::string("fft_generic<") + R + "> n=" + std::to_string(p.n);
     }
@@ -844,7 +845,6 @@ void fft_plan::launch_plane(const pass &p, const pass_args &base, const void *ta
     a.tw0 = base.tw;
     a.tw1 = table1;
     a.conj = base.conj;
-    a.stream = base.stream;
     a.scale = base.scale;
     check_hip((dbl ? launch_plane_f64 : launch_plane_f32)(a, c.threads, c.nblocks, c.lds, stream_), "fused two-axis FFT pass");
 }

@@ -10,7 +10,11 @@
 // Bound: LDS and issue latency inside the block (2.7-3.8 TB/s of its own read + write), still less than
 // the pass over the array and the launch it saves.  Two passes against three, us a transform: 32^3
 // complex<float> 12.0 -> 9.1, 64^3 13.2 -> 10.0, 256 x 64^3 596 -> 379, 16 x 100^3 133 -> 96, 40 x
-// (48, 60, 72) 73 -> 58; complex<double> 256 x 64^3 1095 -> 731, 8 x (70, 70, 256) 204 -> 123.
+// (48, 60, 72) 73 -> 58; complex<double> 256 x 64^3 1095 -> 731, 8 x (70, 70, 256) 204 -> 123.  Its accesses take
+// the caches' default policy at any size: outputs above the Infinity Cache, default / non-temporal stores /
+// non-temporal loads and stores, us of a whole transform, complex<float> 512 x 64^3 729 / 742 / 759, 400 x
+// (48, 60, 72) 507 / 520 / 603, 32768 x 16^3 825 / 814 / 1582, 262144 x 8^3 686 / 717 / 1018, complex<double>
+// 40 x 100^3 511 / 520 / 534.
 #pragma once
 #include "hmi_generic.h"
 
@@ -75,10 +79,11 @@ __device__ __forceinline__ void plane_stage(const plane_args &a, const mixed_pla
     }
 }
 
-// First row stage, global memory -> LDS (lanes walk the rows).
-template <int RX, int SET, int NTM, typename R, typename C>
+// First row stage, global memory -> LDS (lanes walk the rows).  (Values through ldg: where the choice below is
+// one between addresses, the compiler turns every access into flat and scratch ones, 745 -> 1077 us for
+// 512 x 64^3 complex<float>.)
+template <int RX, int SET, typename R, typename C>
 __device__ __forceinline__ void plane_load(const plane_args &a, const C *__restrict__ tw, long long base, unsigned rows, C *lds) {
-    constexpr bool NTL = (NTM & 2) != 0;
     const int m = a.g0.m0;
     const R sg = a.conj ? R(-1) : R(1);
     const C *in = static_cast<const C *>(a.in) + base;
@@ -89,11 +94,11 @@ __device__ __forceinline__ void plane_load(const plane_args &a, const C *__restr
         const unsigned off = row * (unsigned)a.n0 + (unsigned)j;
         C x[RX];
 #pragma unroll
-        for (int p = 0; p < RX; p++) x[p] = ldg<NTL>(in + p * m + off);
+        for (int p = 0; p < RX; p++) x[p] = ldg<false>(in + p * m + off);
         if (mul) {
             C y[RX];
 #pragma unroll
-            for (int p = 0; p < RX; p++) y[p] = a.mul == a.in ? x[p] : ldg<NTL>(mul + p * m + off);
+            for (int p = 0; p < RX; p++) y[p] = a.mul == a.in ? x[p] : ldg<false>(mul + p * m + off);
 #pragma unroll
             for (int p = 0; p < RX; p++) x[p] = cmul(x[p], y[p]);
         }
@@ -112,9 +117,8 @@ __device__ __forceinline__ void plane_load(const plane_args &a, const C *__restr
 }
 
 // Last column stage, LDS -> global memory (lanes walk the columns in frequency order).
-template <int RX, int SET, int NTM, typename R, typename C>
+template <int RX, int SET, typename R, typename C>
 __device__ __forceinline__ void plane_store(const plane_args &a, long long base, unsigned cols, const C *lds) {
-    constexpr bool NTS = (NTM & 1) != 0;
     const unsigned nb = (unsigned)(a.g1.n / RX);
     const R sc = (R)a.scale, sy = a.conj ? -sc : sc;
     C *__restrict__ out = static_cast<C *>(a.out) + base;
@@ -132,11 +136,11 @@ __device__ __forceinline__ void plane_store(const plane_args &a, long long base,
         const unsigned off = (pl * (unsigned)a.n1 + u) * (unsigned)a.n0 + k0;
         const unsigned st = nb * (unsigned)a.n0;
 #pragma unroll
-        for (int q = 0; q < RX; q++) stg<NTS>(out + q * st + off, cmk<C>(x[q].x * sc, x[q].y * sy));
+        for (int q = 0; q < RX; q++) stg<false>(out + q * st + off, cmk<C>(x[q].x * sc, x[q].y * sy));
     }
 }
 
-template <typename R, int SET, int NTM> __global__ void __launch_bounds__(kMixedThreads) fft_plane(plane_args a) {
+template <typename R, int SET> __global__ void __launch_bounds__(kMixedThreads) fft_plane(plane_args a) {
     using C = typename cvec<R>::type;
     extern __shared__ __align__(16) unsigned char smem_raw[];
     C *lds = reinterpret_cast<C *>(smem_raw);
@@ -146,11 +150,11 @@ template <typename R, int SET, int NTM> __global__ void __launch_bounds__(kMixed
     const C *__restrict__ tw0 = reinterpret_cast<const C *>(static_cast<const char *>(a.tw0) + kMixedHead);
     const C *__restrict__ tw1 = reinterpret_cast<const C *>(static_cast<const char *>(a.tw1) + kMixedHead);
     const mixed_stage *st0 = static_cast<const mixed_stage *>(a.tw0), *st1 = static_cast<const mixed_stage *>(a.tw1);
-#define HMI_PLANE_LOAD(RX) case RX: plane_load<RX, SET, NTM, R>(a, tw0, base, planes * (unsigned)a.n1, lds); break;
+#define HMI_PLANE_LOAD(RX) case RX: plane_load<RX, SET, R>(a, tw0, base, planes * (unsigned)a.n1, lds); break;
 #define HMI_PLANE_ROW(RX) case RX: plane_stage<RX, SET, false>(a, a.g0, tw0 + st.twoff, st.m, st.by_m, lds); break;
 #define HMI_PLANE_COL0(RX) case RX: plane_stage<RX, SET, true>(a, a.g1, tw1, a.g1.m0, a.g1.by_m0, lds); break;
 #define HMI_PLANE_COL(RX) case RX: plane_stage<RX, SET, true>(a, a.g1, tw1 + st.twoff, st.m, st.by_m, lds); break;
-#define HMI_PLANE_STORE(RX) case RX: plane_store<RX, SET, NTM, R>(a, base, planes * (unsigned)a.n0, lds); break;
+#define HMI_PLANE_STORE(RX) case RX: plane_store<RX, SET, R>(a, base, planes * (unsigned)a.n0, lds); break;
     // (a partial group leaves the rows and columns of the missing planes untransformed garbage in LDS)
     HMI_MIXED_SWITCH(a.g0.radix[0], HMI_PLANE_LOAD)
     __syncthreads();
@@ -260,7 +264,6 @@ __device__ __forceinline__ void cols_copy(const plane_args &a, C *dst, long long
 template <typename R, bool XY, int NTH> __global__ void __launch_bounds__(NTH) fft_batch_fused(batch_args b) {
     using C = typename cvec<R>::type;
     constexpr int SET = kSetFull;
-    constexpr int NTM = 0;
     extern __shared__ __align__(16) unsigned char smem_raw[];
     C *lds = reinterpret_cast<C *>(smem_raw);
     for (int i = blockIdx.x; i < b.nitems; i += gridDim.x) {
@@ -351,28 +354,19 @@ template <typename R> struct plane_builds {
     static fn choose(const plane_args &a) {
         // both axes in one set: the odd one only for two plans of it (its radices are light ones too)
         const int set = a.g0.set == kSetFull || a.g1.set == kSetFull ? kSetFull : a.g0.set == a.g1.set ? a.g0.set : kSetLight;
-#ifdef HMI_EMULATE
-        static const fn f[3] = {&fft_plane<R, kSetLight, 0>, &fft_plane<R, kSetFull, 0>, &fft_plane<R, kSetOdd, 0>};
+        static const fn f[3] = {&fft_plane<R, kSetLight>, &fft_plane<R, kSetFull>, &fft_plane<R, kSetOdd>};
         return f[set];
-#else
-        static const fn f[3][2] = {{&fft_plane<R, kSetLight, 0>, &fft_plane<R, kSetLight, kStreamLoadsStores>},
-                                   {&fft_plane<R, kSetFull, 0>, &fft_plane<R, kSetFull, kStreamLoadsStores>},
-                                   {&fft_plane<R, kSetOdd, 0>, &fft_plane<R, kSetOdd, kStreamLoadsStores>}};
-        return f[set][a.stream ? 1 : 0];
-#endif
     }
 #ifndef HMI_EMULATE
     static hipError_t launch(const plane_args &a, int threads, long long nblocks, size_t lds, hipStream_t s) {
         // once per process, thread-safe (static initialisation)
         static const bool configured = [] {
-            for (int stream : {0, (int)kStreamLoadsStores})
-                for (int set : {kSetLight, kSetFull, kSetOdd}) {
-                    plane_args p{};
-                    p.g0.set = p.g1.set = set;
-                    p.stream = stream;
-                    (void)hipFuncSetAttribute(reinterpret_cast<const void *>(choose(p)),
-                                              hipFuncAttributeMaxDynamicSharedMemorySize, kGenericMaxLds);
-                }
+            for (int set : {kSetLight, kSetFull, kSetOdd}) {
+                plane_args p{};
+                p.g0.set = p.g1.set = set;
+                (void)hipFuncSetAttribute(reinterpret_cast<const void *>(choose(p)),
+                                          hipFuncAttributeMaxDynamicSharedMemorySize, kGenericMaxLds);
+            }
             return true;
         }();
         (void)configured;

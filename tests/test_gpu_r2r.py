@@ -122,3 +122,28 @@ def test_cos1_rejects_single_point_axis(hmi):
     b = hmi.box3d([0, 0, 0], [7, 0, 7])
     with pytest.raises(Exception):
         hmi.rtransform(hmi.backend.mi355, b, b, hmi.kind.cos1)
+
+
+def test_streaming_forms_of_the_halved_tile(hmi, cuda, oracle):
+    """Double cosine passes of 256 points over more than the Infinity Cache (160 equal boxes): with
+    non-temporal stores where both sides are contiguous along the axis, loads too elsewhere, and named so
+    in the timing report."""
+    import torch
+    size, batch = (256, 256, 4), 160
+    n = int(np.prod(size))
+    x = np.random.default_rng(7).standard_normal(n)
+    inbox = hmi.box3d([0, 0, 0], [s - 1 for s in size])
+    outbox = hmi.box3d([0, 0, 0], [s - 1 for s in size], (1, 2, 0))
+    plan = hmi.rtransform(hmi.backend.mi355, inbox, outbox, hmi.kind.cos)
+    tx = torch.from_numpy(x).to(cuda).repeat(batch)
+    ty, ws = torch.empty_like(tx), torch.empty(batch * plan.size_workspace(), dtype=tx.dtype, device=cuda)
+    plan.set_timing(True)
+    plan.forward_buffered(tx, ty, ws, hmi.scale.none, batch)
+    names = [k for k in plan.timing() if "radices<8, 8, 4>" in k]
+    plan.set_timing(False)
+    assert sorted(k[-3:] for k in names) == [" 5>", " 7>"], names
+    bi = oracle.Box.make((0, 0, 0), [s - 1 for s in size], (0, 1, 2))
+    bo = oracle.Box.make((0, 0, 0), [s - 1 for s in size], (1, 2, 0))
+    rows = ty.view(batch, n)
+    assert fc.rel_l2(fc.to_host(rows[0]), oracle.r2r_cos(bi, bo, x, -1)) <= fc.TOL["float64"]
+    assert torch.equal(rows, rows[:1].expand_as(rows))

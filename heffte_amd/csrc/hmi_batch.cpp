@@ -157,8 +157,7 @@ void batch_plan::prepare(bool dbl) {
     // Fused phases (fft_batch_fused), for lengths with a runtime-length radix plan without prime factors
     // above 13.  x-y: a padded plane fits the LDS; item = as many consecutive z-planes as fit the
     // smallest block size that holds one.  z: item = as many consecutive (x, y) positions as fit the
-    // smallest block.  (nfused: the transforms of the sizes that fused_count() states.)
-    const int pr = dbl ? 1 : 0;
+    // smallest block.
     std::vector<int> xy_build(xf_.size(), -1);
     std::vector<bool> zcol(xf_.size(), false);
     {
@@ -185,7 +184,6 @@ void batch_plan::prepare(bool dbl) {
         d.nfused = 0;
         for (int i = 0; i < (int)xf_.size(); i++) {
             const batch_xform &x = xf_[i];
-            const int k0 = kids[x.size_id[0]], k1 = kids[x.size_id[1]];
             const long long plane = (long long)xy_row_stride(x.n[0]) * x.n[1];  // LDS elements
             batch_fused &f = fused[i];
             if (mplans[x.size_id[0]].n > 1 && mplans[x.size_id[1]].n > 1 && plane * (long long)elem <= kGenericMaxLds) {
@@ -196,14 +194,10 @@ void batch_plan::prepare(bool dbl) {
                 f.by_cols = make_fast_div((unsigned)(f.planes * x.n[0]));
                 f.by_n0 = make_fast_div((unsigned)x.n[0]);
                 xy_build[i] = b;
+                d.nfused++;
                 xy_elems[i] = f.planes * plane;
                 d.xy_lds[b] = std::max(d.xy_lds[b], (size_t)xy_elems[i] * elem);
                 for (long long t = 0; t * f.planes < x.n[2]; t++) xy[b].push_back({i, (int)t});
-            }
-            // the count the interface reports
-            if (k0 >= 0 && k1 >= 0) {
-                const int cls = std::max(batch_kernel_class(k0), batch_kernel_class(k1));
-                if ((cls <= kXyMaxClass[pr] && plane <= kXyBudget[pr]) || plane <= kXyLargeBudget[pr]) d.nfused++;
             }
             const long long cols = (long long)x.n[0] * x.n[1];
             if (mplans[x.size_id[2]].n > 1 && (long long)elem * x.n[2] <= kFusedLds[0] && cols <= 0x7fffffffLL / 2) {

@@ -52,8 +52,8 @@ class batch_plan {
     void set_autotune(bool on) { autotune_ = on; }
     // off: every transform takes the separate x and y phases (the fused x-y phase is on by default)
     void set_fused(bool on) { fused_ = on; }
-    // transforms of compile-time tile lengths and sizes that the fused x-y phase takes (kXyBudget; the
-    // work lists are built on the first execute of each precision; -1 before that)
+    // transforms the fused x-y phase takes (the work lists are built on the first execute of each
+    // precision; -1 before that)
     int fused_count(bool dbl) const { return dev_[dbl ? 1 : 0].ready ? dev_[dbl ? 1 : 0].nfused : -1; }
     int count() const { return (int)xf_.size(); }
     long long input_elems() const { return in_extent_; }

@@ -84,11 +84,7 @@ hipError_t launch_batched(bool dbl, int cls, const batch_args &b, int nblocks, s
 
 // Fused phases of a batch (fft_batch_fused, hmi_plane.h): the x-y phase for planes that fit the LDS, the
 // column-block z phase.  Work items of three sizes, each with its own launch: kFusedLds[k] bytes of LDS
-// and kFusedThreads[k] threads per block.  The rest: the sizes heffte_mi355_batch_fused_count counts
-// (register classes and padded plane elements by precision).
-constexpr int kXyBudget[2] = {10240, 5120};
-constexpr int kXyLargeBudget[2] = {20480, 0};
-constexpr int kXyMaxClass[2] = {2, 0};
+// and kFusedThreads[k] threads per block.
 constexpr int kFusedSizes = 3;
 constexpr int kFusedLds[kFusedSizes] = {40 * 1024, 80 * 1024, kGenericMaxLds};
 constexpr int kFusedThreads[kFusedSizes] = {256, 512, 512};

@@ -251,16 +251,14 @@ int heffte_mi355_batch_set_graph(heffte_mi355_batch batch, int enable);
  * ignored and rewritten).  enable = 0 takes the untimed defaults.  The
  * first call then runs timing launches on a stream of its own: do it outside stream capture. */
 int heffte_mi355_batch_set_autotune(heffte_mi355_batch batch, int enable);
-/* Fused x-y phase (on by default): a transform whose x and y lengths both have compile-time
- * tiles and whose x-y plane fits the LDS of one block (20480 complex<float> elements;
- * complex<double>: 5120 elements and lengths of at most 12 values per thread) runs its
- * x and y axes in one pass over its planes (one read and one write of the array instead of two),
- * and so does any other transform whose plane fits 160 KiB of LDS and whose x and y lengths have no
- * prime factor above 13; the rest take the separate x and y phases.  With it, a transform whose z
- * length has no prime factor above 13 takes the column-block z phase (the z lines of up to 5120 / n2
- * consecutive (x, y) positions per block of LDS; 2560 for complex<double>).  enable = 0 sends every
+/* Fused x-y phase (on by default): a transform whose x and y lengths are above 1 and have no prime
+ * factor above 13, and whose x-y plane (rows padded to an odd length) fits 160 KiB of LDS, runs its
+ * x and y axes in one pass over its planes (one read and one write of the array instead of two);
+ * the others take the separate x and y phases.  With it, a transform whose z length has no prime
+ * factor above 13 takes the column-block z phase (the z lines of up to 5120 / n2 consecutive
+ * (x, y) positions per block of LDS; 2560 for complex<double>).  enable = 0 sends every
  * transform through the three separate phases.  heffte_mi355_batch_fused_count stores in *count
- * how many transforms are of the first kind in the given precision (-1 before the first
+ * how many transforms the fused x-y phase takes in the given precision (-1 before the first
  * forward/backward call of that precision). */
 int heffte_mi355_batch_set_fused(heffte_mi355_batch batch, int enable);
 int heffte_mi355_batch_fused_count(heffte_mi355_batch batch, int double_precision, int *count);

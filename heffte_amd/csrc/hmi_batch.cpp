@@ -154,85 +154,25 @@ void batch_plan::prepare(bool dbl) {
         plans.push_back(g);
         kids.push_back(kid);
     }
-    // Fused phases (fft_batch_fused), for lengths with a runtime-length radix plan without prime factors
-    // above 13.  x-y: a padded plane fits the LDS; item = as many consecutive z-planes as fit the
-    // smallest block size that holds one.  z: item = as many consecutive (x, y) positions as fit the
-    // smallest block.
-    std::vector<int> xy_build(xf_.size(), -1);
-    std::vector<bool> zcol(xf_.size(), false);
-    {
-        // radix plans and tables (no plan: one point, or a prime factor above 13)
-        std::vector<mixed_plan> mplans;
-        std::vector<unsigned char> mtab;
-        std::vector<int> mtoff;
-        for (size_t l = 0; l < lengths_.size(); l++) {
-            mixed_plan g{};
-            mtoff.push_back((int)mtab.size());
-            const int n = lengths_[l];
-            if (n > 1 && 2 * (size_t)n * elem <= (size_t)kGenericMaxLds)
-                g = make_mixed(n, dbl, false, true, true, 0, 0).plan;
-            if (g.chirp || g.direct) g = mixed_plan{};
-            if (g.n > 1) {
-                const std::vector<unsigned char> t = mixed_table(g, dbl, 1);
-                mtab.insert(mtab.end(), t.begin(), t.end());
-            }
-            mplans.push_back(g);
-        }
-        std::vector<batch_fused> fused(xf_.size());
-        std::vector<batch_item> xy[kFusedSizes], zc;
-        std::vector<long long> xy_elems(xf_.size(), 0), zc_elems(xf_.size(), 0);
-        d.nfused = 0;
-        for (int i = 0; i < (int)xf_.size(); i++) {
-            const batch_xform &x = xf_[i];
-            const long long plane = (long long)xy_row_stride(x.n[0]) * x.n[1];  // LDS elements
-            batch_fused &f = fused[i];
-            if (mplans[x.size_id[0]].n > 1 && mplans[x.size_id[1]].n > 1 && plane * (long long)elem <= kGenericMaxLds) {
-                int b = 0;
-                while (plane * (long long)elem > kFusedLds[b]) b++;
-                f.planes = (int)std::min<long long>(x.n[2], kFusedLds[b] / (plane * (long long)elem));
-                f.by_rows = make_fast_div((unsigned)(f.planes * x.n[1]));
-                f.by_cols = make_fast_div((unsigned)(f.planes * x.n[0]));
-                f.by_n0 = make_fast_div((unsigned)x.n[0]);
-                xy_build[i] = b;
-                d.nfused++;
-                xy_elems[i] = f.planes * plane;
-                d.xy_lds[b] = std::max(d.xy_lds[b], (size_t)xy_elems[i] * elem);
-                for (long long t = 0; t * f.planes < x.n[2]; t++) xy[b].push_back({i, (int)t});
-            }
-            const long long cols = (long long)x.n[0] * x.n[1];
-            if (mplans[x.size_id[2]].n > 1 && (long long)elem * x.n[2] <= kFusedLds[0] && cols <= 0x7fffffffLL / 2) {
-                f.width = (int)std::min<long long>(cols, kFusedLds[0] / ((long long)elem * x.n[2]));
-                f.by_width = make_fast_div((unsigned)f.width);
-                zcol[i] = true;
-                zc_elems[i] = (long long)f.width * x.n[2];
-                d.zc_lds = std::max(d.zc_lds, (size_t)zc_elems[i] * elem);
-                for (long long t = 0; t * f.width < cols; t++) zc.push_back({i, (int)t});
-            }
-        }
-        // largest items first (the blocks take them in list order, so a launch ends on small ones)
-        auto by_size = [](std::vector<batch_item> &v, const std::vector<long long> &e) {
-            std::stable_sort(v.begin(), v.end(),
-                             [&](const batch_item &a, const batch_item &b) { return e[a.xform] > e[b.xform]; });
-            if (v.size() > 0x7fffffffULL) throw std::runtime_error("batch work list too long");
-        };
-        for (int b = 0; b < kFusedSizes; b++) {
-            by_size(xy[b], xy_elems);
-            d.nxy[b] = (int)xy[b].size();
-            tables.add(&d.xy[b], xy[b]);
-        }
-        by_size(zc, zc_elems);
-        d.nzc = (int)zc.size();
-        tables.add(&d.zc, zc);
-        tables.add(&d.fused, fused);
-        tables.add(&d.mplans, mplans);
-        tables.add(&d.mtab, mtab);
-        tables.add(&d.mtoff, mtoff);
+    const fused_lists fl = make_fused_lists(xf_, lengths_, dbl);
+    d.nfused = (int)std::count(fl.in_xy.begin(), fl.in_xy.end(), true);
+    for (int b = 0; b < kFusedSizes; b++) {
+        d.nxy[b] = (int)fl.xy[b].size();
+        d.xy_lds[b] = fl.xy_lds[b];
+        tables.add(&d.xy[b], fl.xy[b]);
     }
+    d.nzc = (int)fl.zc.size();
+    d.zc_lds = fl.zc_lds;
+    tables.add(&d.zc, fl.zc);
+    tables.add(&d.fused, fl.fused);
+    tables.add(&d.mplans, fl.plans);
+    tables.add(&d.mtab, fl.table);
+    tables.add(&d.mtoff, fl.offset);
     // work lists: every tile of every transform, one list per axis and register class; for the
     // x and y axes also the lists without the transforms of the fused phase, for z the list
     // without those of the column-block phase
     for (int ax = 0; ax < 3; ax++) {
-        std::vector<batch_item> items[kBatchClasses], rest[kBatchClasses];  // rest: z phase without zcol
+        std::vector<batch_item> items[kBatchClasses], rest[kBatchClasses];
         for (int i = 0; i < (int)xf_.size(); i++) {
             const batch_xform &x = xf_[i];
             const int col = (ax == 0) ? 1 : 0, b1 = 3 - ax - col;
@@ -241,7 +181,7 @@ void batch_plan::prepare(bool dbl) {
             const long long ntiles = (nlines + lines - 1) / lines;
             const int c = batch_kernel_class(kids[x.size_id[ax]]);
             for (long long t = 0; t < ntiles; t++) items[c].push_back({i, (int)t});
-            if (ax < 2 ? xy_build[i] < 0 : !zcol[i])
+            if (ax < 2 ? !fl.in_xy[i] : !fl.in_zc[i])
                 for (long long t = 0; t < ntiles; t++) rest[c].push_back({i, (int)t});
         }
         for (int c = 0; c < kBatchClasses; c++) {

@@ -330,7 +330,61 @@ int launch_threads(int threads, long long nblocks) {
     return threads;
 }
 
-fast_div make_fast_div(unsigned d) { return make_div(d); }
+fused_lists make_fused_lists(const std::vector<batch_xform> &xf, const std::vector<int> &lengths, bool dbl) {
+    fused_lists f;
+    const long long elem = dbl ? 16 : 8;
+    // radix plans and tables (no plan: one point, or a prime factor above 13)
+    for (int n : lengths) {
+        mixed_plan g{};
+        f.offset.push_back((int)f.table.size());
+        if (n > 1 && 2 * n * elem <= kGenericMaxLds) g = make_mixed(n, dbl, false, true, true, 0, 0).plan;
+        if (g.chirp || g.direct) g = mixed_plan{};
+        if (g.n > 1) {
+            const std::vector<unsigned char> t = mixed_table(g, dbl, 1);
+            f.table.insert(f.table.end(), t.begin(), t.end());
+        }
+        f.plans.push_back(g);
+    }
+    const size_t count = xf.size();
+    f.fused.resize(count);
+    f.in_xy.resize(count);
+    f.in_zc.resize(count);
+    std::vector<long long> xy_elems(count, 0), zc_elems(count, 0);
+    for (int i = 0; i < (int)count; i++) {
+        const batch_xform &x = xf[i];
+        const long long plane = (long long)xy_row_stride(x.n[0]) * x.n[1];  // LDS elements
+        batch_fused &e = f.fused[i];
+        if (f.plans[x.size_id[0]].n > 1 && f.plans[x.size_id[1]].n > 1 && plane * elem <= kGenericMaxLds) {
+            int b = 0;
+            while (plane * elem > kFusedLds[b]) b++;
+            e.planes = (int)std::min<long long>(x.n[2], kFusedLds[b] / (plane * elem));
+            e.by_rows = make_div((unsigned)(e.planes * x.n[1]));
+            e.by_cols = make_div((unsigned)(e.planes * x.n[0]));
+            e.by_n0 = make_div((unsigned)x.n[0]);
+            f.in_xy[i] = true;
+            xy_elems[i] = e.planes * plane;
+            f.xy_lds[b] = std::max(f.xy_lds[b], (size_t)(xy_elems[i] * elem));
+            for (long long t = 0; t * e.planes < x.n[2]; t++) f.xy[b].push_back({i, (int)t});
+        }
+        const long long cols = (long long)x.n[0] * x.n[1];
+        if (f.plans[x.size_id[2]].n > 1 && elem * x.n[2] <= kFusedLds[0] && cols <= 0x7fffffffLL / 2) {
+            e.width = (int)std::min<long long>(cols, kFusedLds[0] / (elem * x.n[2]));
+            e.by_width = make_div((unsigned)e.width);
+            f.in_zc[i] = true;
+            zc_elems[i] = (long long)e.width * x.n[2];
+            f.zc_lds = std::max(f.zc_lds, (size_t)(zc_elems[i] * elem));
+            for (long long t = 0; t * e.width < cols; t++) f.zc.push_back({i, (int)t});
+        }
+    }
+    // largest items first (the blocks take them in list order, so a launch ends on small ones)
+    auto by_size = [](std::vector<batch_item> &v, const std::vector<long long> &e) {
+        std::stable_sort(v.begin(), v.end(), [&](const batch_item &a, const batch_item &b) { return e[a.xform] > e[b.xform]; });
+        if (v.size() > 0x7fffffffULL) throw std::runtime_error("batch work list too long");
+    };
+    for (std::vector<batch_item> &v : f.xy) by_size(v, xy_elems);
+    by_size(f.zc, zc_elems);
+    return f;
+}
 
 void mixed_launch_divs(mixed_plan &g, const pass_args &a) {
     g.by_ncol = make_div((unsigned)a.ncol);

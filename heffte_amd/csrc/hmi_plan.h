@@ -230,7 +230,20 @@ long long min_planes(int n0, int n1, bool dbl);
 // Largest count of threads per block, at most `threads`, with fewer than 2^32 in the grid (the kernels
 // walk their work with a stride of the block's threads, a multiple of 64).
 int launch_threads(int threads, long long nblocks);
-fast_div make_fast_div(unsigned d);
+// Fused phases of a batch (fft_batch_fused), for lengths with a runtime-length radix plan without prime
+// factors above 13.  x-y: a padded plane fits the LDS; item = as many consecutive z-planes as fit the
+// smallest block size that holds one.  z: item = as many consecutive (x, y) positions as fit the smallest
+// block.
+struct fused_lists {
+    std::vector<mixed_plan> plans;      // per length
+    std::vector<unsigned char> table;   // their device tables,
+    std::vector<int> offset;            // each from here on
+    std::vector<batch_fused> fused;     // per transform
+    std::vector<bool> in_xy, in_zc;
+    std::vector<batch_item> xy[kFusedSizes], zc;
+    size_t xy_lds[kFusedSizes] = {}, zc_lds = 0;
+};
+fused_lists make_fused_lists(const std::vector<batch_xform> &xf, const std::vector<int> &lengths, bool dbl);
 // the divisors of one launch's line numbering
 void mixed_launch_divs(mixed_plan &g, const pass_args &a);
 

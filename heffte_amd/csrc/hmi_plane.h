@@ -261,7 +261,7 @@ __device__ __forceinline__ void cols_copy(const plane_args &a, C *dst, long long
 // butterfly chains per line in registers (two 256-thread blocks per CU; x-y 1.2 ms, z 0.75 ms).  Measured
 // around it: radices up to 10 only 3.10 ms; first block size 32, 24 or 52 KB 2.84-2.88; 512 threads in it
 // 3.00, 256 in the second 2.92; z blocks of 20 KB 2.94, of 80 KB with 512 threads 2.79.
-template <typename R, bool XY, int NTH> __global__ void __launch_bounds__(NTH) fft_batch_fused(batch_args b) {
+template <typename R, bool XY> __global__ void __launch_bounds__(kMixedThreads) fft_batch_fused(batch_args b) {
     using C = typename cvec<R>::type;
     constexpr int SET = kSetFull;
     extern __shared__ __align__(16) unsigned char smem_raw[];
@@ -379,14 +379,14 @@ template <typename R> struct plane_builds {
 #ifndef HMI_EMULATE
 template <typename R> hipError_t launch_batch_builds(bool xy, const batch_args &b, int threads, int nblocks, size_t lds, hipStream_t s) {
     static const bool configured = [] {
-        for (const void *f : {reinterpret_cast<const void *>(&fft_batch_fused<R, true, kMixedThreads>),
-                              reinterpret_cast<const void *>(&fft_batch_fused<R, false, kMixedThreads>)})
+        for (const void *f : {reinterpret_cast<const void *>(&fft_batch_fused<R, true>),
+                              reinterpret_cast<const void *>(&fft_batch_fused<R, false>)})
             (void)hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, kGenericMaxLds);
         return true;
     }();
     (void)configured;
     if (threads > kMixedThreads || lds > (size_t)kGenericMaxLds) return hipErrorInvalidValue;
-    (xy ? &fft_batch_fused<R, true, kMixedThreads> : &fft_batch_fused<R, false, kMixedThreads>)
+    (xy ? &fft_batch_fused<R, true> : &fft_batch_fused<R, false>)
         <<<dim3((unsigned)nblocks), dim3(threads), lds, s>>>(b);
     return hipGetLastError();
 }

@@ -284,3 +284,35 @@ def test_batch_random_sides(hmi, cuda, oracle, dtype):
     for s, off in zip(sizes, offsets):
         n = int(np.prod(s))
         assert fc.rel_l2(z[off:off + n], x[off:off + n]) <= TOL[dtype], s
+
+
+# lengths without a compile-time tile, planes of every block size, z lengths up to one column a block and
+# (5000 points, complex<double>) beyond the column-block phase
+WIDE_SIZES = [(50, 60, 72), (72, 100, 33), (150, 100, 5), (200, 100, 3), (100, 150, 7), (60, 50, 200), (22, 26, 130),
+              (3, 5, 2600), (2, 7, 5000), (9, 4, 1300), (144, 10, 256), (12, 180, 100), (90, 108, 4), (75, 128, 3)]
+
+
+@pytest.mark.parametrize("dtype", ["complex64", "complex128"])
+def test_fused_phases_of_other_lengths(hmi, cuda, oracle, dtype):
+    """Fused x-y and column-block z phases of lengths without a compile-time tile and of long z lines,
+    against the oracle transform by transform, both directions, at shuffled offsets."""
+    import torch
+    sizes = WIDE_SIZES
+    counts = [int(np.prod(s)) for s in sizes]
+    in_off = np.cumsum([0] + counts)[:-1]
+    out_off, pos = [0] * len(sizes), 5
+    for i in np.random.default_rng(3).permutation(len(sizes)):
+        out_off[i] = pos
+        pos += counts[i] + 1
+    plan = hmi.batch_plan(sizes, list(in_off), out_off)
+    plan.set_autotune(False)
+    x = fc.uniform_complex(plan.size_input(), 17)
+    tdt = torch.complex64 if dtype == "complex64" else torch.complex128
+    tx = torch.from_numpy(x).to(cuda).to(tdt)
+    for sign, call, scaling in [(-1, plan.forward, 0), (+1, plan.backward, 2)]:
+        dst = torch.zeros(plan.size_output(), dtype=tdt, device=cuda)
+        call(tx, dst, scaling)
+        y = fc.to_host(dst)
+        for s, off, r in zip(sizes, out_off, oracle_each(oracle, sizes, in_off, x, sign, scaling)):
+            assert fc.rel_l2(y[off:off + r.size], r) <= TOL[dtype], s
+    assert plan.fused_count(dtype == "complex128") == sum(fused_eligible(s, dtype) for s in sizes)

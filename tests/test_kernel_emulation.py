@@ -4,7 +4,7 @@ The runtime-length pass takes every length without a compile-time tile in every 
 sides, Hermitian load, partial store, fused product, split-axis twiddle, cosine and sine modes); its
 index arithmetic, radix plans and LDS layouts are checked against direct transforms for all orders
 of both sides, with arrays and LDS that end where the pass may last touch them.  The fused two-axis
-pass likewise over many plane shapes.
+pass likewise over many plane shapes, and the fused phases of a batch over the work lists of one.
 """
 import os
 import shutil
@@ -29,7 +29,7 @@ def build(tmp_path_factory, name, sources):
 
 
 @pytest.mark.skipif(CLANG is None, reason="clang++ not found")
-@pytest.mark.parametrize("name", ["emulate_generic", "emulate_plane"])
+@pytest.mark.parametrize("name", ["emulate_generic", "emulate_plane", "emulate_batch"])
 def test_kernel(tmp_path_factory, name):
     exe = build(tmp_path_factory, name, ["hmi_generic_plan.cpp"])
     runs = [subprocess.Popen([exe, str(i), str(SHARES)], stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)

@@ -891,15 +891,6 @@ __global__ void __launch_bounds__(256) permute_kernel(const E *__restrict__ src,
 
 // ----------------------------------------------------------- fast registry
 
-// Real-to-real passes in complex<double> of 256 and more points, 8 elements per thread: their loads and
-// stores move half the bytes of a complex tile, so the pass is bound by latency, and its LDS holds a CU
-// to half the waves that its registers would allow.  Exchanging the parts one after the other in a tile
-// of half the size: 256^3 double DCT-II / III pair 465 -> 438 us, the results bit for bit the same; above the
-// Infinity Cache with the streaming form of the pass (512 x 256 x 512, the contiguous axis 244 us with
-// non-temporal loads and stores, 231 with stores only).  The
-// complex passes stay as they are (512^3 complex<double> 768 -> 787 us per pass, 256^3 109 -> 108).
-constexpr bool halved_tile(int n, int e, int bytes) { return n >= 256 && bytes == 16 && e <= 8; }
-
 #define HMI_FAST(TYPE, N, E, T, PS, ...)                                                                  \
     static hipError_t launch_##TYPE##_##N##_##T(const pass_args &a, long long nblocks, hipStream_t s) {    \
         if constexpr (halved_tile(N, E, 2 * sizeof(TYPE))) {                                               \
@@ -975,8 +966,7 @@ constexpr bool halved_tile(int n, int e, int bytes) { return n >= 256 && bytes =
 HMI_FAST_TABLE(HMI_FAST)
 
 #define HMI_FAST_ENTRY(TYPE, N, E, T, PS, ...) \
-    {sizeof(TYPE) == 8, N, E, T, PS, {__VA_ARGS__}, radices<__VA_ARGS__>::count, \
-     halved_tile(N, E, 2 * sizeof(TYPE)), &launch_##TYPE##_##N##_##T},
+    {sizeof(TYPE) == 8, N, E, T, PS, {__VA_ARGS__}, radices<__VA_ARGS__>::count, &launch_##TYPE##_##N##_##T},
 
 static const fast_kernel_info kFast[] = {HMI_FAST_TABLE(HMI_FAST_ENTRY)};
 

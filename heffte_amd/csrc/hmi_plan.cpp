@@ -220,6 +220,7 @@ exec_choice fft_plan::build(int dir, bool dbl, bool in_real, bool out_real, bool
     std::vector<int> perm = axes;
     std::sort(perm.begin(), perm.end());
     double best_cost = std::numeric_limits<double>::infinity();
+    double chunk_cost[3] = {-1.0, -1.0, -1.0};
     exec_plan best;
 
     auto try_plan = [&](const std::vector<candidate_pass> &seq) {
@@ -320,7 +321,12 @@ exec_choice fft_plan::build(int dir, bool dbl, bool in_real, bool out_real, bool
                     cost += 1.0;
                     if (p.load_colfast && p.store_colfast) cost += 0.15;
                     else if (p.load_colfast || p.store_colfast) cost += 0.05;
-                    if (!cp.identity && (p.load_colfast || p.store_colfast)) cost += narrow_chunk_cost(p, dbl);
+                    if (!cp.identity && (p.load_colfast || p.store_colfast)) {
+                        // (the same for every schedule: the length and the mode of the axis decide)
+                        double &c = chunk_cost[p.axis];
+                        if (c < 0.0) c = narrow_chunk_cost(p, dbl);
+                        cost += c;
+                    }
                     // a copy pass runs one LDS tile per line: not along an axis too long for one
                     if (cp.identity) cost += 0.5 + (2 * dims[cp.axis] * (dbl ? 16 : 8) > kGenericMaxLds ? 100.0 : 0.0);
                     ep.passes.push_back(p);
@@ -361,7 +367,7 @@ exec_choice fft_plan::build(int dir, bool dbl, bool in_real, bool out_real, bool
 
     exec_choice c;
     finish(best, dbl, sizes_only);
-    c.axes = best;
+    c.axes = std::move(best);
 
     // The two fastest axes in one fused pass where a plane fits the LDS: same layout on both sides and
     // plain complex data, so the passes are (fastest two: in -> out), (slowest: out, in place).
@@ -604,7 +610,7 @@ std::string pass_kernel_name(const pass &p, bool dbl, bool mfma, int precision, 
         for (int i = 0; i < p.fast->nstages; i++) s += (i ? ", " : "") + std::to_string(p.fast->radix[i]);
         s += ">, " + std::to_string(p.fast->E) + ", " + std::to_string(p.fast->T) + ", " +
              std::to_string(p.fast->PS) + ", " +
-             std::to_string(a.stream | (p.fast->halved && p.mode >= kModeDCT2 ? kHalvedTile : 0)) + ">";
+             std::to_string(a.stream | (p.mode >= kModeDCT2 && halved_tile(p.n, p.fast->E, dbl ? 16 : 8) ? kHalvedTile : 0)) + ">";
     } else {
         s = std::string("fft_generic<") + R + "> n=" + std::to_string(p.n);
     }

@@ -6,7 +6,8 @@
 // the block's threads with the lines of the tile fastest (lanes on consecutive lines: consecutive
 // LDS elements, one twiddle for all of them, the line of a thread fixed for the whole loop), except
 // the load and store of a side on which the FFT axis is the contiguous one, where lanes walk the
-// axis.  All divisions are multiplications by the plan's constants.
+// axis.  Divisions are multiplications by the plan's constants (but for two in the direct stages, one a work
+// unit of four outputs).
 //
 // Bound: HBM bytes on complex<double> (384 x 400 x 320, per pass: 305, 315 and 325 us, 4.8-5.2 TB/s;
 // a device copy of such arrays runs at 4.7-5.0 TB/s), issue and latency on complex<float> (40 boxes of

@@ -480,7 +480,7 @@ __device__ __forceinline__ void generic_bfly(const C *sp, int istride, C *dp, in
     for (int q = 0; q < R; q++) dp[q * ostride] = x[q];
 }
 
-// One tile (g.lines lines) of an n-point pass with a runtime radix plan; any block size.
+// One tile (g.lines lines) of an n-point complex pass with a runtime radix plan; any block size.
 template <typename R>
 __device__ void generic_tile(const pass_args &a, const generic_plan &g, unsigned tile,
                              typename cvec<R>::type *smem) {
@@ -498,31 +498,8 @@ __device__ void generic_tile(const pass_args &a, const generic_plan &g, unsigned
         C x = cmk<C>(R(0), R(0));
         const unsigned L = tile * T + l;
         if (L < (unsigned)a.nlines) {
-            const long long lbase = line_offset(L, a, false);
-            const long long off = lbase + (long long)j * a.in_sa;
-            const R *rsrc = static_cast<const R *>(a.in);
-            if (a.mode == kModeDCT2 || a.mode == kModeDST2) {
-                const int jj = (j < (N + 1) / 2) ? 2 * j : 2 * (N - 1 - j) + 1;
-                x.x = rsrc[lbase + (long long)jj * a.in_sa];
-                if (a.mode == kModeDST2 && (jj & 1)) x.x = -x.x;
-            } else if (a.mode == kModeDCT3 || a.mode == kModeDST3) {
-                const bool sine = (a.mode == kModeDST3);
-                const R xk = rsrc[lbase + (long long)(sine ? N - 1 - j : j) * a.in_sa];
-                const R xm = j > 0 ? rsrc[lbase + (long long)(sine ? j - 1 : N - j) * a.in_sa] : R(0);
-                const C w = static_cast<const C *>(a.tw)[g.postoff + j];
-                x = cmk<C>(w.x * xk - w.y * xm, w.x * xm + w.y * xk);  // conj of conj(w) (xk - i xm)
-            } else if (a.mode == kModeDCT1 || a.mode == kModeDCT1B) {
-                x.x = rsrc[lbase + (long long)(j <= N / 2 ? j : N - j) * a.in_sa];
-            } else if (a.in_real) {
-                x.x = static_cast<const R *>(a.in)[off];
-            } else if (a.herm_load && j > N / 2) {
-                x = static_cast<const C *>(a.in)[lbase + (long long)(N - j) * a.in_sa];
-                x.y *= -sg;
-            } else {
-                x = static_cast<const C *>(a.in)[off];
-                if (a.mul) x = cmul(x, a.mul == a.in ? x : static_cast<const C *>(a.mul)[off]);
-                x.y *= sg;
-            }
+            x = static_cast<const C *>(a.in)[line_offset(L, a, false) + (long long)j * a.in_sa];
+            x.y *= sg;
         }
         buf0[l * N + j] = x;
     }
@@ -576,26 +553,9 @@ __device__ void generic_tile(const pass_args &a, const generic_plan &g, unsigned
         int l, j;
         if (a.store_colfast) { l = idx % T; j = idx / T; } else { l = idx / N; j = idx % N; }
         const unsigned L = tile * T + l;
-        if (L >= (unsigned)a.nlines || j >= a.store_len) continue;
+        if (L >= (unsigned)a.nlines) continue;
         const C y = src[l * N + j];
-        const long long lobase = line_offset(L, a, true);
-        const long long off = lobase + (long long)j * a.out_sa;
-        if (a.mode == kModeDCT2 || a.mode == kModeDST2) {
-            const C w = static_cast<const C *>(a.tw)[g.postoff + j];
-            const int k = (a.mode == kModeDST2) ? N - 1 - j : j;
-            static_cast<R *>(a.out)[lobase + (long long)k * a.out_sa] = R(2) * (w.x * y.x - w.y * y.y) * sc;
-        } else if (a.mode == kModeDCT3 || a.mode == kModeDST3) {
-            const int jj = (j < (N + 1) / 2) ? 2 * j : 2 * (N - 1 - j) + 1;
-            R r = R(2) * y.x;
-            if (a.mode == kModeDST3 && (jj & 1)) r = -r;
-            static_cast<R *>(a.out)[lobase + (long long)jj * a.out_sa] = r * sc;
-        } else if (a.mode == kModeDCT1B) {
-            static_cast<R *>(a.out)[off] = R(2) * y.x * sc;
-        } else if (a.out_real) static_cast<R *>(a.out)[off] = y.x * sc;
-        else if (a.tw4) {
-            const C z = cmul(y, static_cast<const C *>(a.tw4)[line_index(L, a, a.tw4_dim) * (unsigned)j]);
-            static_cast<C *>(a.out)[off] = cmk<C>(z.x * sc, sg * z.y * sc);
-        } else static_cast<C *>(a.out)[off] = cmk<C>(y.x * sc, sg * y.y * sc);
+        static_cast<C *>(a.out)[line_offset(L, a, true) + (long long)j * a.out_sa] = cmk<C>(y.x * sc, sg * y.y * sc);
     }
 }
 

@@ -75,7 +75,6 @@ struct generic_plan {
     int radix[kMaxStages];
     int twoff[kMaxStages];     // offset (complex units) of stage twiddles w_{Ls R}^{p k}
     int rootoff[kMaxStages];   // offset of w_R^j, j < R (used by radices without a hard-coded butterfly)
-    int postoff;               // offset of the real-data twiddles (modes other than kModeC2C)
 };
 
 // Division of x < 2^31 by a fixed divisor d: q = umulhi(2 x, mul) >> shift, with 2^(shift-1) < d <=

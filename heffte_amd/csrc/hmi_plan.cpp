@@ -537,8 +537,6 @@ std::vector<R> make_table(const int *radix, int nstages, bool with_roots, int ta
 
 std::vector<int> default_radices(int n) { return factorize(n); }
 
-generic_plan make_generic_plan(int n, int lines) { return make_generic_plan(n, lines, factorize(n)); }
-
 generic_plan make_generic_plan(int n, int lines, const std::vector<int> &rad) {
     generic_plan g{};
     g.n = n;
@@ -558,7 +556,6 @@ generic_plan make_generic_plan(int n, int lines, const std::vector<int> &rad) {
         g.rootoff[s] = off;
         if (!has_butterfly(rad[s])) off += rad[s];
     }
-    g.postoff = off;
     g.lines = lines;
     return g;
 }

@@ -247,12 +247,10 @@ fused_lists make_fused_lists(const std::vector<batch_xform> &xf, const std::vect
 // the divisors of one launch's line numbering
 void mixed_launch_divs(mixed_plan &g, const pass_args &a);
 
-// Runtime radix plan of length n for the generic tile (stage/root/post offsets
-// filled in; lines = lines per tile) and its twiddle table in either precision.
-generic_plan make_generic_plan(int n, int lines);
-// The same with an explicit radix order (their product must be n).
+// Runtime radix plan of length n = the product of radices for the batched kernel's tile (lines = lines per
+// tile) and its twiddle table in either precision.
 generic_plan make_generic_plan(int n, int lines, const std::vector<int> &radices);
-// The radix order the planner uses by default: 8s, then a 4 and a 2, then odd primes.
+// Its radix order by default: 8s, then a 4 and a 2, then odd primes.
 std::vector<int> default_radices(int n);
 std::vector<float> generic_table_f32(const generic_plan &g);
 std::vector<double> generic_table_f64(const generic_plan &g);

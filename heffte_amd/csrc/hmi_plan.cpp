@@ -953,7 +953,7 @@ void fft_plan::execute(int dir, bool dbl, bool in_real, bool out_real, int batch
         for (int d = 0; d < 3; d++) e += (L.n[d] - 1) * L.stride[d];
         return e + (long long)(batch - 1) * (L.n[0] * L.n[1] * L.n[2]) + 1;
     };
-    static const bool debug = std::getenv("HMI_DEBUG_PLAN") != nullptr;
+    const bool debug = std::getenv("HMI_DEBUG_PLAN") != nullptr;
     // per-pass timing: one event before the first pass and one after each pass
     std::unique_lock<std::mutex> tlock(timing_mtx_, std::defer_lock);
     hipEvent_t tprev = nullptr;

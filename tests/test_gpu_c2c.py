@@ -297,3 +297,19 @@ def test_split_length_real_input_and_r2c(hmi, cuda, oracle):
     back = torch.empty_like(tx)
     rplan.backward(ty, back, hmi.scale.full)
     assert fc.rel_l2(fc.to_host(back), x) <= 1e-13
+
+
+def test_plan_trace_follows_the_environment(hmi, cuda, capfd, monkeypatch):
+    """HMI_DEBUG_PLAN prints the passes of the calls made while it is set, also after earlier calls."""
+    import torch
+    box = hmi.box3d([0, 0, 0], [15, 15, 15])
+    plan = hmi.fft3d(hmi.backend.mi355, box, box)
+    x = torch.zeros(16 ** 3, dtype=torch.complex64, device=cuda)
+    y = torch.empty_like(x)
+    for on in (False, True, False):
+        if on:
+            monkeypatch.setenv("HMI_DEBUG_PLAN", "1")
+        else:
+            monkeypatch.delenv("HMI_DEBUG_PLAN", raising=False)
+        plan.forward(x, y)
+        assert ("[hmi] pass" in capfd.readouterr().err) == on

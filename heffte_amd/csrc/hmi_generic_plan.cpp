@@ -157,6 +157,30 @@ int chirp_length(int n, bool dbl) {
     return best;
 }
 
+namespace {
+// Lines per tile (log2) of a launch of nlines lines, l2 the full tile's: few lines take smaller tiles on more
+// CUs, down to 64-byte chunks of a side that walks the column axis.
+int tile_lines(const mixed_plan &g, int l2, bool across, bool dbl, long long nlines) {
+    const int least = across ? (dbl ? 2 : 3) : 0;
+    while (l2 > least && (nlines >> l2) < kFewBlocks) l2--;
+    return l2;
+}
+}  // namespace
+
+mixed_tiles::mixed_tiles(int n, bool dbl, bool copy, bool load_across, bool store_across, int tail)
+    : n_(n), tail_(tail), dbl_(dbl), copy_(copy), load_(load_across), store_(store_across) {
+    full_ = make_mixed(n, dbl, copy, load_across, store_across, 0, tail);
+}
+
+const mixed_config &mixed_tiles::of(long long nlines) {
+    const int l2 = tile_lines(full_.plan, full_.plan.log2t, load_ || store_, dbl_, nlines);
+    if (l2 == full_.plan.log2t) return full_;
+    std::lock_guard<std::mutex> lock(mtx_);
+    std::unique_ptr<mixed_config> &c = smaller_[l2];
+    if (!c) c = std::make_unique<mixed_config>(make_mixed(n_, dbl_, copy_, load_, store_, nlines, tail_));
+    return *c;
+}
+
 mixed_config make_mixed(int n, bool dbl, bool copy, bool load_across, bool store_across, long long nlines,
                         int tail) {
     mixed_config c{};
@@ -214,8 +238,7 @@ mixed_config make_mixed(int n, bool dbl, bool copy, bool load_across, bool store
     int l2 = 0;
     while (l2 < 6 && (n * elem << (l2 + 1)) <= kMixedTile) l2++;
     while ((elem << l2) < 128 && bytes(2 << l2) <= (across ? kGenericMaxLds : kGenericMaxLds / 2)) l2++;
-    // few lines in all (nlines > 0): smaller tiles on more CUs, down to 64-byte chunks
-    while (nlines > 0 && l2 > (across ? (dbl ? 2 : 3) : 0) && (nlines >> l2) < kFewBlocks) l2--;
+    if (nlines > 0) l2 = tile_lines(g, l2, across, dbl, nlines);
     g.log2t = l2;
     const int T = 1 << l2;
     g.pitch = walk && T > 1 ? T + 1 : T;

@@ -50,9 +50,10 @@ constexpr long long kMixedTile = 16 * 1024;  // bytes a tile aims at
 // 4 x (120, 120, 64) 38 -> 30 us.
 constexpr int kPlaneMaxSide = 256;
 constexpr long long kPlaneBytes = kGenericMaxLds, kPlaneTile = 32 * 1024;
-// Launches of fewer blocks take smaller tiles on more CUs (r2c 20 x 14 x 12 float: 14.3 -> 13.1 us a
-// call, 60 x 60 x 40 pair 30.7 -> 28.0 us); many lines keep the full tile, which one transform's line
-// count used to cap also in a batch (one-dimensional lines: one line per block).
+// Launches of fewer blocks, of all lines of a batch, take smaller tiles on more CUs (r2c 20 x 14 x 12 float:
+// 14.3 -> 13.1 us a call, 60 x 60 x 40 pair 30.7 -> 28.0 us).  One line per block wastes its lanes: sized by
+// one transform's lines, 206 x (64, 1, 14) double cosine 43.5 us and by the batch's 16.2, 1386 x (3, 7, 1) double
+// c2r 14.2 and 7.7.
 constexpr long long kFewBlocks = 256;
 hipError_t launch_mixed_f32(const pass_args &a, const mixed_plan &g, int threads, long long nblocks, size_t lds_bytes,
                             hipStream_t s);

@@ -477,12 +477,9 @@ void fft_plan::configure(pass &p, bool dbl, bool sizes_only) const {
     }
     if (sizes_only) return;  // no step buffer: nothing else the workspace depends on
     const int tail = (p.mode >= kModeDCT2 && p.mode <= kModeDST3) ? p.n : 0;
-    const long long lines = std::max(p.lin.n[p.col], p.lout.n[p.col]) * std::max(p.lin.n[p.b1], p.lout.n[p.b1]);
-    auto c = std::make_shared<std::array<mixed_config, 2>>();
-    for (int few = 0; few < 2; few++)
-        (*c)[few] = make_mixed(p.n, dbl, p.identity, p.load_colfast, p.store_colfast, few ? lines : 0, tail);
-    if (!(*c)[0].ok) throw std::runtime_error("transform length " + std::to_string(p.n) + " has no single-pass plan");
-    p.lines = 1 << (*c)[0].plan.log2t;
+    auto c = std::make_shared<mixed_tiles>(p.n, dbl, p.identity, p.load_colfast, p.store_colfast, tail);
+    if (!c->full().ok) throw std::runtime_error("transform length " + std::to_string(p.n) + " has no single-pass plan");
+    p.lines = 1 << c->full().plan.log2t;
     p.mixed = c;
 }
 
@@ -641,7 +638,7 @@ std::vector<unsigned char> pass_table(bool dbl, const pass &p) {
     long long tail_mod = 1;
     if (p.mode == kModeR2C || p.mode == kModeC2R) { tail_count = p.n / 2; tail_mod = p.n; }
     if (p.mode >= kModeDCT2 && p.mode <= kModeDST3) { tail_count = p.n; tail_mod = 4LL * p.n; }
-    if (p.mixed) return mixed_table((*p.mixed)[0].plan, dbl, tail_mod);
+    if (p.mixed) return mixed_table(p.mixed->full().plan, dbl, tail_mod);
     return table_bytes(dbl, p.fast->radix, p.fast->nstages, tail_count, tail_mod);
 }
 }  // namespace
@@ -826,8 +823,7 @@ void split_steps(const pass &p, const pass_args &base, bool dbl, int bt, void *t
 
 namespace {
 void launch_mixed_pass(const pass &p, const pass_args &a, bool dbl, hipStream_t s) {
-    const mixed_config *c = &(*p.mixed)[0];
-    if ((a.nlines >> c->plan.log2t) < kFewBlocks) c = &(*p.mixed)[1];
+    const mixed_config *c = &p.mixed->of(a.nlines);
     mixed_plan g = c->plan;
     mixed_launch_divs(g, a);
     const long long nblocks = ((long long)a.nlines + (1 << g.log2t) - 1) >> g.log2t;

@@ -57,6 +57,22 @@ struct mixed_config {
     size_t lds = 0;
 };
 
+// The tiles of one runtime-length pass: the full one and, made when a launch first has so few lines (of a
+// whole batch), the smaller ones.
+class mixed_tiles {
+  public:
+    mixed_tiles(int n, bool dbl, bool copy, bool load_across, bool store_across, int tail);
+    const mixed_config &full() const { return full_; }
+    const mixed_config &of(long long nlines);
+
+  private:
+    int n_, tail_;
+    bool dbl_, copy_, load_, store_;
+    mixed_config full_;
+    std::mutex mtx_;
+    std::array<std::unique_ptr<mixed_config>, 16> smaller_;  // by log2 of the lines per tile
+};
+
 // Tile and block of the fused pass over the two fastest axes.
 struct plane_config {
     bool ok = false;
@@ -79,8 +95,7 @@ struct pass {
     int mode = 0;           // kModeC2C, or kModeR2C / kModeC2R when the half-length kernel runs it
     // launch configuration
     const fast_kernel_info *fast = nullptr;
-    // set: the runtime-length pass runs it, with the second tile where a launch's lines are few
-    std::shared_ptr<const std::array<mixed_config, 2>> mixed;
+    std::shared_ptr<mixed_tiles> mixed;  // set: the runtime-length pass runs it
     int lines = 1;  // lines (columns) per block
     // set: axis and col (the two fastest axes of lin = lout) run as one fused pass
     std::shared_ptr<const plane_config> plane;

@@ -60,7 +60,9 @@ template <typename R> int run_case(int n, int mode, int flags, int oi, int oo, i
     const sides si = layout_of(oi, nin, ncol, nb1), so = layout_of(oo, nout, ncol, nb1);
     const bool load_across = si.sa != 1 && nin > 1, store_across = so.sa != 1 && nout > 1;
     const int tail = (mode >= hmi::kModeDCT2 && mode <= hmi::kModeDST3) ? n : 0;
-    const hmi::mixed_config c = hmi::make_mixed(n, dbl, copy, load_across, store_across, (flags & 1024) ? 0 : (long long)ncol * nb1, tail);
+    // the full tile, or the one a launch of these lines takes
+    hmi::mixed_tiles tiles(n, dbl, copy, load_across, store_across, tail);
+    const hmi::mixed_config &c = (flags & 1024) || !tiles.full().ok ? tiles.full() : tiles.of((long long)ncol * nb1 * batch);
     what = "n=" + std::to_string(n) + (dbl ? " f64" : " f32") + " mode=" + std::to_string(mode) + " flags=" +
            std::to_string(flags) + " orders=" + std::to_string(oi) + std::to_string(oo) + " ncol=" + std::to_string(ncol) +
            " nb1=" + std::to_string(nb1) + " batch=" + std::to_string(batch);
@@ -171,11 +173,31 @@ template <typename R> int run_case(int n, int mode, int flags, int oi, int oo, i
     return 0;
 }
 
+// The tile of a launch goes by all its lines: the full one from kFewBlocks blocks on, otherwise the
+// largest that makes as many, or the smallest there is.
+int check_tiles() {
+    int fails = 0;
+    for (bool dbl : {false, true})
+        for (int n : {1, 7, 14, 60, 127, 240, 1000})
+            for (int sides = 0; sides < 4; sides++) {
+                hmi::mixed_tiles tiles(n, dbl, false, sides & 1, sides & 2, 0);
+                const int full = tiles.full().plan.log2t, least = std::min(full, sides ? (dbl ? 2 : 3) : 0);
+                for (long long lines : {1LL, 100LL, 330LL, 1000LL, 11880LL, 13184LL, 100000LL, 1LL << 30}) {
+                    const hmi::mixed_config &c = tiles.of(lines);
+                    const int l2 = c.plan.log2t;
+                    const bool enough = (lines >> l2) >= hmi::kFewBlocks;
+                    const bool good = l2 == full ? enough || l2 == least : (lines >> (l2 + 1)) < hmi::kFewBlocks && (enough || l2 == least);
+                    if (!c.ok || !good || &tiles.of(lines) != &c) std::printf("FAIL tile n=%d sides %d lines %lld: %d\n", n, sides, lines, l2), fails++;
+                }
+            }
+    return fails;
+}
+
 int main(int argc, char **argv) {
     const int share = argc > 1 ? std::atoi(argv[1]) : 0, shares = argc > 2 ? std::atoi(argv[2]) : 1;
     std::mt19937 rng(5);
     auto pick = [&](int lo, int hi) { return lo + (int)(rng() % (unsigned)(hi - lo + 1)); };
-    int fails = 0, cases = 0, at = 0;
+    int fails = share == 0 ? check_tiles() : 0, cases = 0, at = 0;
     auto one = [&](bool dbl, int n, int mode, int flags, int oi, int oo, int ncol, int nb1, int batch, double limit = 0) {
         if (at++ % shares != share) return;
         std::string what;

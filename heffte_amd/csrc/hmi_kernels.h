@@ -27,13 +27,16 @@ struct fast_kernel_info {
 };
 
 // Real-to-real passes in complex<double> of 256 and more points, 8 elements per thread, exchange the
-// parts one after the other through a tile of half the size (kHalvedTile): their loads and
-// stores move half the bytes of a complex tile, so the pass is bound by latency, and its LDS holds a CU
-// to half the waves that its registers would allow.  256^3 double DCT-II / III pair 465 -> 438 us, the
-// results bit for bit the same; above the Infinity Cache with the streaming form of the pass (512 x 256 x
-// 512, the contiguous axis 244 us with non-temporal loads and stores, 231 with stores only).  The complex
-// passes stay as they are (512^3 complex<double> 768 -> 787 us per pass, 256^3 109 -> 108).
+// parts one after the other through a tile of half the size (kHalvedTile): their loads and stores move
+// half the bytes of a complex tile, so the pass is bound by latency, and its LDS holds a CU to half the
+// waves that its registers would allow.  256^3 double DCT-II / III pair 465 -> 438 us, the results bit for
+// bit the same; above the Infinity Cache with the streaming form of the pass (512 x 256 x 512, the
+// contiguous axis 244 us with non-temporal loads and stores, 231 with stores only).  The complex passes
+// stay as they are (512^3 complex<double> 768 -> 787 us per pass, 256^3 109 -> 108), and so do launches whose
+// blocks all fit the CUs at once, 16 waves in each, where the additional barriers only cost (12 x 256 x 32
+// 16.6 us whole, 19.0 in halves).
 constexpr bool halved_tile(int n, int e, int bytes) { return n >= 256 && bytes == 16 && e <= 8; }
+constexpr bool halved_launch(long long nblocks, int threads) { return nblocks * threads > 256LL * 16 * 64; }
 
 // wide = the pass walks the column axis on load or store (needs 128-byte column
 // chunks); otherwise the variant with the fewest lines per block is returned.

@@ -854,7 +854,7 @@ __global__ void __launch_bounds__(256) permute_kernel(const E *__restrict__ src,
 #define HMI_FAST(TYPE, N, E, T, PS, ...)                                                                  \
     static hipError_t launch_##TYPE##_##N##_##T(const pass_args &a, long long nblocks, hipStream_t s) {    \
         if constexpr (halved_tile(N, E, 2 * sizeof(TYPE))) {                                               \
-            if (a.mode >= kModeDCT2) {                                                                     \
+            if (a.mode >= kModeDCT2 && halved_launch(nblocks, (N / E) * T)) {                              \
                 (a.stream == 0 ? &fft_uniform<TYPE, radices<__VA_ARGS__>, E, T, PS, kHalvedTile>           \
                  : a.stream == kStreamStores                                                               \
                      ? &fft_uniform<TYPE, radices<__VA_ARGS__>, E, T, PS, kHalvedTile | kStreamStores>     \

@@ -604,7 +604,12 @@ std::string pass_kernel_name(const pass &p, bool dbl, bool mfma, int precision, 
         for (int i = 0; i < p.fast->nstages; i++) s += (i ? ", " : "") + std::to_string(p.fast->radix[i]);
         s += ">, " + std::to_string(p.fast->E) + ", " + std::to_string(p.fast->T) + ", " +
              std::to_string(p.fast->PS) + ", " +
-             std::to_string(a.stream | (p.mode >= kModeDCT2 && halved_tile(p.n, p.fast->E, dbl ? 16 : 8) ? kHalvedTile : 0)) + ">";
+             std::to_string(a.stream | (p.mode >= kModeDCT2 && halved_tile(p.n, p.fast->E, dbl ? 16 : 8) &&
+                                                halved_launch(((long long)a.nlines + p.lines - 1) / p.lines,
+                                                              p.n / p.fast->E * p.fast->T)
+                                            ? kHalvedTile
+                                            : 0)) +
+             ">";
     } else {
         s = std::string("fft_generic<") + R + "> n=" + std::to_string(p.n);
     }

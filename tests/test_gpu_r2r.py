@@ -147,3 +147,22 @@ def test_streaming_forms_of_the_halved_tile(hmi, cuda, oracle):
     rows = ty.view(batch, n)
     assert fc.rel_l2(fc.to_host(rows[0]), oracle.r2r_cos(bi, bo, x, -1)) <= fc.TOL["float64"]
     assert torch.equal(rows, rows[:1].expand_as(rows))
+
+
+def test_halved_tile_by_the_size_of_the_launch(hmi, cuda):
+    """Double cosine passes of 256 points exchange in halves only where their blocks outnumber what the CUs hold
+    at once (256 blocks of 512 threads do not), with the same results bit for bit."""
+    import torch
+    box = hmi.box3d([0, 0, 0], [255, 15, 15])
+    plan = hmi.rtransform(hmi.backend.mi355, box, box, hmi.kind.cos)
+    n, batch = box.count(), 64
+    x = torch.randn(n, dtype=torch.float64, device=cuda)
+    tx = x.repeat(batch)
+    y, ty = torch.empty_like(x), torch.empty_like(tx)
+    for inp, out, many, form in [(x, y, 1, ", 0>"), (tx, ty, batch, ", 4>")]:
+        plan.set_timing(True)
+        plan.forward(inp, out, hmi.scale.none, many)
+        names = [k for k in plan.timing() if "radices<8, 8, 4>" in k]
+        plan.set_timing(False)
+        assert names and all(k.endswith(form) for k in names), names
+    assert torch.equal(ty.view(batch, n), y.expand(batch, n))

@@ -336,16 +336,15 @@ void group_planes(plane_config &c, long long nplanes, bool dbl) {
     c.threads = launch_threads(c.threads, c.nblocks);
 }
 
-// A plane of more than 64 KiB has a CU to itself, and a launch of few of them leaves most CUs idle
-// while one pass per axis spreads their lines.  One pass for both axes over one pass for each, us of a
-// whole transform, complex<float> 128 x 128 x 1 12.7 / 8.8, x 64 22.3 / 21.3, x 128 25.2 / 27.5; 200 x 100 x 64
-// 28.2 / 25.1, x 128 32.9 / 34.4; 100 x 100 x 8 12.1 / 11.5, x 32 13.7 / 13.8; complex<double> 100 x 100 x 32
-// 19.5 / 18.8, x 64 23.3 / 25.0; 80 x 80 x 16 14.3 / 13.3, x 32 15.1 / 15.7; 64 x 64 (65 KiB) x 1 7.0 / 7.0, x 4
-// 10.5 / 10.4, x 32 11.5 / 12.9.  Planes of 64 KiB and less win from the first one on (64 x 64 x 1 complex<float>
-// 5.2 / 7.0).
+// A plane of about 64 KiB or more has a CU to itself, and a launch of few of them leaves most CUs idle
+// while one pass per axis spreads their lines.  One pass for both axes / one pass for each, us of a whole
+// transform: complex<float> 128 x 128 x 1 12.7 / 8.8, x 64 22.3 / 21.3, x 128 25.2 / 27.5; 200 x 100 x 64 28.2 /
+// 25.1, x 128 32.9 / 34.4; 100 x 100 x 8 12.1 / 11.5, x 32 13.7 / 13.8; 80 x 80 (51 KiB) x 1 7.1 / 9.6;
+// complex<double> 100 x 100 x 32 19.5 / 18.8, x 64 23.3 / 25.0; 80 x 80 x 16 14.3 / 13.3, x 32 15.1 / 15.7;
+// 64 x 64 (65 KiB) x 4 10.5 / 10.4, x 8 10.6 / 10.9; 128 x 32 x 4 13.5 / 12.2; 32 x 32 x 1 5.7 / 7.1.
 long long min_planes(int n0, int n1, bool dbl) {
-    const long long elem = dbl ? 16 : 8, above = (long long)(n0 | 1) * n1 - 64 * 1024 / elem;
-    return above <= 0 ? 1 : 1 + above / 96;
+    const long long above = (long long)(n0 | 1) * n1 - (dbl ? 3072 : 8192);  // 48 and 64 KiB
+    return above <= 0 ? 1 : 1 + above / (dbl ? 128 : 96);
 }
 
 int launch_threads(int threads, long long nblocks) {

@@ -267,7 +267,8 @@ def test_scratch_limit_does_not_depend_on_fused_passes(hmi, size, dbl):
 @pytest.mark.parametrize("size,passes", [((64, 64, 64), 2), ((64, 64, 1), 1), ((128, 128, 1), 2), ((128, 128, 16), 3),
                                          ((128, 128, 128), 2), ((256, 64, 2), 3), ((200, 100, 4), 3), ((32, 32, 2), 2)])
 def test_flat_boxes_run_one_pass_per_axis(hmi, size, passes):
-    # (host planning only) a plane that fills a CU runs as one block: few of them take one pass per axis
+    # (host planning only, complex<float>) a plane that fills a CU runs as one block: few of them take one
+    # pass per axis
     box = hmi.box3d([0, 0, 0], [s - 1 for s in size])
     plan = hmi.fft3d(hmi.backend.mi355, box, box)
     assert plan.matrix_core_passes(-1)[1] == passes

@@ -429,6 +429,18 @@ __device__ __forceinline__ void mixed_drain(const pass_args &a, const mixed_plan
     }
 }
 
+// One-stage lengths whose few lines load and store elementwise (mixed_plan::spread): their butterflies.
+template <int RX, int SET, typename C> __device__ __forceinline__ void mixed_only(const mixed_plan &g, C *lds) {
+    for (int l = threadIdx.x; l < 1 << g.log2t; l += blockDim.x) {
+        C x[RX];
+#pragma unroll
+        for (int p = 0; p < RX; p++) x[p] = lds[p * g.pitch + l];
+        butterfly<RX, SET == kSetOdd>(x);
+#pragma unroll
+        for (int p = 0; p < RX; p++) lds[p * g.pitch + l] = x[p];
+    }
+}
+
 // Sums of one direct p-point butterfly at sp (elements pitch apart): outputs q and p - q for q = q0 and
 // q0 + 1.  root = w_p^t, t < p.
 template <typename R, typename C>
@@ -552,6 +564,7 @@ __global__ void __launch_bounds__(kMixedThreads) fft_generic(pass_args a, mixed_
         }
     }
 #define HMI_MIXED_FIRST(RX) case RX: mixed_first<RX, SET, FORM, NTM, R>(a, g, tile, lds); break;
+#define HMI_MIXED_ONLY(RX) case RX: mixed_only<RX, SET>(g, lds); break;
 #define HMI_MIXED_MID(RX) case RX: mixed_middle<RX, SET, false, R>(a, g, st, lds); break;
 #define HMI_MIXED_BACK(RX) case RX: mixed_middle<RX, SET, true, R>(a, g, st, lds); break;
 #define HMI_MIXED_CENTER(RX) case RX: mixed_center<RX, SET, R>(a, g, st, lds); break;
@@ -567,8 +580,17 @@ __global__ void __launch_bounds__(kMixedThreads) fft_generic(pass_args a, mixed_
     }
     const mixed_stage *stages = static_cast<const mixed_stage *>(a.tw);
     [[maybe_unused]] C *other = lds + g.n * g.pitch;  // plans with two direct stages or more
-    if (FORM != kFormChirp && (g.nst == 0 || g.radix[0] > 16)) {
+    if (FORM != kFormChirp && (g.nst == 0 || g.radix[0] > 16 || (FORM == kFormAny && g.spread))) {
         if constexpr (FORM != kFormChirp) mixed_fill<FORM, NTM, R>(a, g, tile, lds);
+        if constexpr (FORM == kFormAny && SET != kSetOdd) {
+            if (g.spread) {
+                __syncthreads();
+                switch (g.radix[0]) {
+                    HMI_MIXED_ONLY(10)
+                    default: if constexpr (SET == kSetFull) { switch (g.radix[0]) { HMI_MIXED_HEAVY(HMI_MIXED_ONLY) } }
+                }
+            }
+        }
         if (FORM == kFormDirect && g.nst > 1) {
             __syncthreads();
             const mixed_stage st{g.radix[0], g.m0, 0, g.by_m0, fast_div{}, g.root0};
@@ -627,21 +649,30 @@ template <typename R> struct generic_builds {
         const int at = stream == 0 ? 0 : (stream == kStreamStores ? 1 : 2);
         return set == kSetOdd ? odd[form][at] : f[set][form][at];
     }
-    static fn choose(const pass_args &a, const mixed_plan &g) {
-        const bool plain = a.mode == kModeC2C && !a.in_real && !a.out_real && !a.herm_load && !a.mul && !a.tw4 &&
-                           a.store_len == g.len;
+    static int form(const pass_args &a, const mixed_plan &g) {
+        if (g.chirp || g.direct) return g.chirp ? kFormChirp : kFormDirect;
+        if (a.mode != kModeC2C || a.in_real || a.out_real || a.herm_load || a.mul || a.tw4 || a.store_len != g.len) return kFormAny;
         // elements up to the furthest one of either side (no stride is negative)
         auto span = [&](long long sa, long long sc, long long sb1, long long sb2) {
             return (g.n - 1) * sa + (a.ncol - 1) * sc + (a.nb1 - 1) * sb1 + (a.nbatch - 1) * sb2 + 1;
         };
         const long long most = std::max(span(a.in_sa, a.in_sc, a.in_sb1, a.in_sb2),
                                         span(a.out_sa, a.out_sc, a.out_sb1, a.out_sb2));
-        const bool near = most * (long long)sizeof(typename cvec<R>::type) <= (1LL << 32);
-        return pick(g.set, g.chirp ? kFormChirp : g.direct ? kFormDirect : !plain ? kFormAny : (near ? kFormPlain32 : kFormPlain), a.stream);
+        return most * (long long)sizeof(typename cvec<R>::type) <= (1LL << 32) ? kFormPlain32 : kFormPlain;
+    }
+    static fn choose(const pass_args &a, const mixed_plan &g) { return pick(g.set, form(a, g), a.stream); }
+    // Few lines of one stage of 10 to 16 points in any form: a wave that loads, transforms and stores whole
+    // lines alone on its CU waits for itself.  Elements are spread over four times the threads instead, with
+    // the butterflies in between (us a call, whole lines / spread: sine 14 x 15 x 4 float 14.0 / 11.8, cosine 10 x
+    // (14, 14, 16) double 19.2 / 17.3, sine (12, 1, 14) double 14.3 / 12.0; with more lines it loses, r2c 4 x (32, 13,
+    // 32) double 13.6 / 15.0, 64 x (64, 14, 32) 36.9 / 50.1, 36 x (33, 12, 10) 21.2 / 25.8, and so do shorter ones, r2c
+    // 4 x (64, 5, 64) 13.1 / 14.7).
+    static int spread(const pass_args &a, mixed_plan &g, int threads) {
+        g.spread = g.nst == 1 && g.n >= 10 && a.nlines <= 3072 && form(a, g) == kFormAny;
+        return g.spread ? std::max(threads, (int)std::min<long long>(256, ((long long)g.n << g.log2t) / 256 * 64)) : threads;
     }
 #ifndef HMI_EMULATE
-    static hipError_t launch(const pass_args &a, const mixed_plan &g, int threads, long long nblocks, size_t lds,
-                             hipStream_t s) {
+    static hipError_t launch(const pass_args &a, mixed_plan g, int threads, long long nblocks, size_t lds, hipStream_t s) {
         // once per process, thread-safe (static initialisation)
         static const bool configured = [] {
             for (int set : {kSetLight, kSetFull, kSetOdd})
@@ -652,6 +683,7 @@ template <typename R> struct generic_builds {
             return true;
         }();
         (void)configured;
+        threads = spread(a, g, threads);
         choose(a, g)<<<dim3((unsigned)nblocks), dim3(threads), lds, s>>>(a, g);
         return hipGetLastError();
     }

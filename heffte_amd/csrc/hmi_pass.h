@@ -109,6 +109,7 @@ struct mixed_plan {
     int len;                         // points of a line (n, unless chirp)
     int chirp, direct;               // direct: number of direct stages
     int set;                         // build of the kernels that runs it (kSetLight, ...)
+    int spread;                      // one-stage lengths: elementwise load and store (set by a launch)
     int log2t, pitch, pad;           // lines per tile 2^log2t, LDS strides (elements)
     int radix[kMixedStages];
     int m0;                          // the first stage's twiddles w_n^{j q}: table[j (r_0 - 1) + q - 1]

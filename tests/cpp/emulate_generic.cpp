@@ -100,8 +100,9 @@ template <typename R> int run_case(int n, int mode, int flags, int oi, int oo, i
     hmi::mixed_plan g = c.plan;
     hmi::mixed_launch_divs(g, a);
     const long long nblocks = (a.nlines + (1LL << g.log2t) - 1) >> g.log2t;
+    const int threads = hmi::generic_builds<R>::spread(a, g, c.threads);
     auto kernel = hmi::generic_builds<R>::choose(a, g);
-    emulate::run_blocks(nblocks, c.threads, hmi::smem_raw, sizeof(hmi::smem_raw), c.lds, [&] { kernel(a, g); });
+    emulate::run_blocks(nblocks, threads, hmi::smem_raw, sizeof(hmi::smem_raw), c.lds, [&] { kernel(a, g); });
     // direct transform of each line
     const roots wn(n), w4n(4 * nin), wd(2 * std::max<long long>(1, nin - 1)), ws(split ? n4 : 1);
     long double num = 0, den = 0;
@@ -222,7 +223,7 @@ int main(int argc, char **argv) {
             for (int k = 0; k < 3; k++)
                 one(dbl, n, hmi::kModeC2C, pick(0, 1) * 64, k == 0 ? 0 : pick(0, 5), k == 0 ? 2 : pick(0, 5), pick(1, 21),
                     pick(1, 3), pick(1, 2));
-    const int few[] = {1, 2, 6, 13, 17, 22, 38, 134, 289, 45, 60, 77, 105, 127, 180, 216};
+    const int few[] = {1, 2, 6, 10, 12, 13, 15, 16, 17, 22, 38, 134, 289, 45, 60, 77, 105, 127, 180, 216};
     for (bool dbl : {false, true})
         for (int n : few) {
             for (int flags : {1, 2, 2 | 8, 4 | 64, 4 | 16 | 64, 16 | 64, 32, 32 | 64, 128, 256, 256 | 64, 8}) {

@@ -337,14 +337,17 @@ void group_planes(plane_config &c, long long nplanes, bool dbl) {
 }
 
 // A plane of about 64 KiB or more has a CU to itself, and a launch of few of them leaves most CUs idle
-// while one pass per axis spreads their lines.  One pass for both axes / one pass for each, us of a whole
-// transform: complex<float> 128 x 128 x 1 12.7 / 8.8, x 64 22.3 / 21.3, x 128 25.2 / 27.5; 200 x 100 x 64 28.2 /
-// 25.1, x 128 32.9 / 34.4; 100 x 100 x 8 12.1 / 11.5, x 32 13.7 / 13.8; 80 x 80 (51 KiB) x 1 7.1 / 9.6;
-// complex<double> 100 x 100 x 32 19.5 / 18.8, x 64 23.3 / 25.0; 80 x 80 x 16 14.3 / 13.3, x 32 15.1 / 15.7;
-// 64 x 64 (65 KiB) x 4 10.5 / 10.4, x 8 10.6 / 10.9; 128 x 32 x 4 13.5 / 12.2; 32 x 32 x 1 5.7 / 7.1.
+// while one pass per axis spreads their lines, the sooner the faster those passes are: the tiles of powers of
+// two against the others.  One pass for both axes / one pass for each, us of a whole transform:
+//   complex<float>   128 x 128 x 1 12.7 / 8.8, x 64 22.3 / 21.3, x 128 25.2 / 27.5; 256 x 64 x 8 16.6 / 12.4
+//                    200 x 100 x 1 17.5 / 8.7, x 32 24.4 / 18.8, x 128 32.9 / 34.4; 100 x 100 x 8 12.1 / 11.5, x 32 13.7 /
+//                    13.8; 96 x 196 x 105 26.8 / 30.6; 112 x 112 x 3 13.5 / 18.2; 80 x 80 (51 KiB) x 1 7.1 / 9.6
+//   complex<double>  64 x 64 (65 KiB) x 4 10.5 / 10.4, x 8 10.6 / 10.9; 128 x 32 x 4 13.5 / 12.2; 32 x 32 x 1 5.7 / 7.1
+//                    100 x 100 x 8 16.4 / 12.7, x 32 19.5 / 18.8, x 64 23.3 / 25.0; 80 x 80 x 2 13.3 / 11.6, x 32 15.1 / 15.7
 long long min_planes(int n0, int n1, bool dbl) {
     const long long above = (long long)(n0 | 1) * n1 - (dbl ? 3072 : 8192);  // 48 and 64 KiB
-    return above <= 0 ? 1 : 1 + above / (dbl ? 128 : 96);
+    const bool powers = (n0 & (n0 - 1)) == 0 && (n1 & (n1 - 1)) == 0;
+    return above <= 0 ? 1 : 1 + above / ((dbl ? 128 : 96) * (powers ? 1 : 4));
 }
 
 int launch_threads(int threads, long long nblocks) {

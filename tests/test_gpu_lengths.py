@@ -95,8 +95,8 @@ def passes_of(plan):
 
 @pytest.mark.parametrize("dtype", ["complex64", "complex128"])
 @pytest.mark.parametrize("size,batch", [((2, 3, 1), 700), ((4, 4, 4), 300), ((5, 7, 3), 401), ((8, 8, 8), 129), ((16, 16, 16), 70),
-                                        ((32, 30, 3), 90), ((81, 64, 2), 60), ((20, 256, 3), 20), ((100, 45, 7), 10),
-                                        ((98, 100, 4), 30), ((256, 20, 6), 9)])
+                                        ((32, 30, 3), 90), ((81, 64, 2), 60), ((20, 256, 3), 20), ((100, 45, 2), 30),
+                                        ((98, 100, 4), 30), ((256, 20, 3), 18), ((128, 32, 5), 12)])
 def test_fused_planes_of_a_batch(hmi, cuda, oracle, dtype, size, batch):
     """The planes of a whole batch are grouped into blocks, and planes that fill a CU take the fused pass
     only where the batch holds enough of them: both schedules of one plan, one transform and the batch."""

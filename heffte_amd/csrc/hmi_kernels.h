@@ -43,14 +43,14 @@ constexpr bool halved_launch(long long nblocks, int threads) { return nblocks * 
 const fast_kernel_info *find_fast_kernel(int n, bool dbl, bool wide);
 
 // Runtime-length pass (hmi_generic.h): at most kMixedThreads threads per block; plans whose radices
-// all stay within kLightRadix run a build of their own with fewer registers.
+// all stay within kLightRadix run builds of their own with fewer registers.
 constexpr int kMixedThreads = 512;
 constexpr int kLightRadix = 10;
 constexpr long long kMixedTile = 16 * 1024;  // bytes a tile aims at
 // Fused two-axis pass: longest side (longer axes keep the compile-time and matrix-core passes), LDS
 // bytes of a plane and of a block's planes.  A plane that fills the LDS alone, one block per CU, still
-// beats two passes: complex<double> 16 x 100^3 286 -> 236 us, 90 x 100 x 108 32 -> 28 us, complex<float>
-// 4 x (120, 120, 64) 38 -> 30 us.
+// beats two passes where there are enough of them (min_planes): complex<double> 16 x 100^3 286 -> 236 us,
+// 90 x 100 x 108 32 -> 28 us, complex<float> 4 x (120, 120, 64) 38 -> 30 us.
 constexpr int kPlaneMaxSide = 256;
 constexpr long long kPlaneBytes = kGenericMaxLds, kPlaneTile = 32 * 1024;
 // Launches of fewer blocks, of all lines of a batch, take smaller tiles on more CUs (r2c 20 x 14 x 12 float:

@@ -92,9 +92,9 @@ struct fast_div {
 // i pitch + (i / m_0) pad + l.
 //
 // Prime factors from 17 to 61 (to 107 beside other factors, max_direct) are direct stages, behind the
-// others: an output pair (q, p - q) sums the (p - 1) / 2 input pairs (k, p - k) against the table w_p^t.  The last stage takes them from LDS to
-// global memory; a length with two or three such factors runs the earlier ones from one LDS buffer
-// to a second one.
+// others: an output pair (q, p - q) sums the (p - 1) / 2 input pairs (k, p - k) against the table w_p^t.
+// The last stage takes them from LDS to global memory; a length with two or three such factors runs the
+// earlier ones from one LDS buffer to a second one.
 //
 // Lines of len points whose length has a larger prime factor run as a chirp convolution (Bluestein,
 // 1970): j k = (j^2 + k^2 - (k - j)^2) / 2, so X_k = c_k sum_j (x_j c_j) conj(c_{k-j}) with c_j =

@@ -227,9 +227,10 @@ class fft_plan {
 };
 
 // Radix order of the runtime-length pass (empty: n has a prime factor beyond the direct stages and runs as
-// a chirp convolution), and its tile for one pass (copy: no transform, only the layout change; *_across: that side walks the column axis; nlines:
-// lines of a launch with few of them, 0 for many; tail: real-data twiddles).  Device table: the later stages' entries,
-// the stage twiddles, w_{tail_mod}^k for k < tail, the chirp and its transform.
+// a chirp convolution), and its tile for one pass (copy: no transform, only the layout change; *_across:
+// that side walks the column axis; nlines: lines of the launch, 0 for many; tail: real-data twiddles).  Device
+// table: the later stages' entries, the stage twiddles, w_{tail_mod}^k for k < tail, the chirp and its
+// transform.
 std::vector<int> mixed_radices(int n, bool dbl);
 mixed_config make_mixed(int n, bool dbl, bool copy, bool load_across, bool store_across, long long nlines,
                         int tail);
